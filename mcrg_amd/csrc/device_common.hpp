@@ -68,61 +68,7 @@ struct Accept {
     uint32_t always0, always1;
 };
 
-// Metropolis decision for the 32 sites of one word.  s, nu, nd, nl, nr are the
-// spin bits of the sites and of their up/down/left/right neighbours; `valid`
-// masks the sites that exist.  Returns the bits to flip.
-//
-// e <= 0 flips outright.  The other sites compare a 32-bit uniform U_i with the
-// threshold of their class.  The first Philox call gives every site the 4 top
-// bits of its U_i (slice q = out[q] supplies bit 31-q of all 32 sites), which
-// decide the comparison unless they equal the threshold's 4 top bits
-// (probability 1/16).  The sites still open, ranked by bit index, take their 28
-// low bits from refinement calls, four sites per call.
-__device__ __forceinline__ uint32_t metropolis_word(uint32_t s, uint32_t nu, uint32_t nd,
-                                                    uint32_t nl, uint32_t nr, uint32_t valid,
-                                                    const Accept &acc, uint32_t k0, uint32_t k1,
-                                                    uint32_t word, uint32_t t, uint32_t colour)
-{
-    const uint32_t a1 = s ^ nu, a2 = s ^ nd, a3 = s ^ nl, a4 = s ^ nr;
-    const uint32_t x1 = a1 ^ a2, y1 = a1 & a2, x2 = a3 ^ a4, y2 = a3 & a4;
-    const uint32_t any = a1 | a2 | a3 | a4;
-    const uint32_t c1 = (x1 ^ x2) & ~(y1 | y2);  // one anti-aligned neighbour: e = 2
-    const uint32_t c2 = ~any;                    // none: e = 4
-    uint32_t flip = any & ~c1;                   // two or more: e <= 0
-    flip |= (acc.always0 ? c1 : 0u) | (acc.always1 ? c2 : 0u);
-    const uint32_t m1 = acc.always0 ? 0u : c1;
-    const uint32_t m2 = acc.always1 ? 0u : c2;
-    uint32_t open = (m1 | m2) & valid;
-    uint32_t accept = 0;
-    if (open != 0u) {
-        const uint32_t tag = (kTagSweep << 28) | (colour << 24);
-        // the first refinement call is drawn beside the first-stage call: a
-        // wave nearly always needs it, and the two independent Philox chains
-        // interleave
-        const u32x4 r = philox(word, t, 0u, tag, k0, k1);
-        u32x4 ref = philox(word, t, 1u, tag, k0, k1);
-        const uint32_t rq[4] = {r.v0, r.v1, r.v2, r.v3};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t b0 = 0u - ((acc.thr0 >> (31 - q)) & 1u);
-            const uint32_t b1 = 0u - ((acc.thr1 >> (31 - q)) & 1u);
-            const uint32_t tb = (m1 & b0) | (m2 & b1);
-            accept |= open & ~rq[q] & tb;
-            open &= ~(rq[q] ^ tb);
-        }
-        for (uint32_t rank = 0; open != 0u; ++rank) {
-            const uint32_t i = (uint32_t)__builtin_ctz(open);
-            open &= open - 1u;
-            if (rank != 0u && (rank & 3u) == 0u) ref = philox(word, t, 1u + (rank >> 2), tag, k0, k1);
-            const uint32_t low = pick4(ref, rank & 3u) >> 4;
-            const uint32_t thr = ((m1 >> i) & 1u) ? acc.thr0 : acc.thr1;
-            accept |= (low < (thr & 0x0FFFFFFFu) ? 1u : 0u) << i;
-        }
-    }
-    return (flip | accept) & valid;
-}
-
-// The two Philox calls metropolis_word draws first for a word (the 4 top bits
+// The two Philox calls a word's Metropolis decision draws first (the 4 top bits
 // of every site's uniform, and the first refinement call), which depend only
 // on the word, sweep and colour: a caller can draw them ahead of the spins.
 __device__ __forceinline__ void metropolis_rng(uint32_t word, uint32_t t, uint32_t colour, uint32_t k0, uint32_t k1,
@@ -133,43 +79,108 @@ __device__ __forceinline__ void metropolis_rng(uint32_t word, uint32_t t, uint32
     ref = philox(word, t, 1u, tag, k0, k1);
 }
 
-// metropolis_word with the first two Philox calls drawn by metropolis_rng
-// (the same decisions bit for bit).
-__device__ __forceinline__ uint32_t metropolis_word_drawn(uint32_t s, uint32_t nu, uint32_t nd, uint32_t nl,
-                                                          uint32_t nr, const Accept &acc, uint32_t k0, uint32_t k1,
-                                                          uint32_t word, uint32_t t, uint32_t colour,
-                                                          const u32x4 &r, u32x4 ref)
+// One open site, the lowest of `open`: accepted when its 28 low bits are below
+// its class's threshold's.  The 28 bits are the top ones of w, and
+// (w >> 4) < T is w < 16 T, so the comparison takes w as it is.
+__device__ __forceinline__ void metropolis_refine(uint32_t &open, uint32_t &accept, uint32_t m1, uint32_t w,
+                                                  uint32_t low0, uint32_t low1)
+{
+    const uint32_t lsb = open & (0u - open);
+    open ^= lsb;
+    accept |= w < ((m1 & lsb) != 0u ? low0 : low1) ? lsb : 0u;
+}
+
+// Metropolis decision for the 32 sites of one word.  s, nu, nd, nl, nr are the
+// spin bits of the sites and of their up/down/left/right neighbours; `valid`
+// masks the sites that exist; r and ref are metropolis_rng's.  Returns the bits
+// to flip.
+//
+// e <= 0 flips outright.  The other sites compare a 32-bit uniform U_i with the
+// threshold of their class.  The first Philox call gives every site the 4 top
+// bits of its U_i (slice q = out[q] supplies bit 31-q of all 32 sites), which
+// decide the comparison unless they equal the threshold's 4 top bits
+// (probability 1/16).  The sites still open, ranked by bit index, take their 28
+// low bits from refinement calls, four sites per call.
+//
+// Bound by VALU issue (about 95 instructions a word beside the Philox calls).
+// The first four ranks are worked off without a branch: of the 64 lanes of a
+// wave one nearly always has four open sites, and a step is then nine
+// instructions, with no loop state and no selection of the word by rank (a
+// loop over the ranks took fifteen): L = 16384 unmeasured 67 -> 49 us a sweep,
+// 256 resident L = 512 lattices 10 % less.  Of the fifth to eighth rank only
+// the fifth is common, so the rest stand behind a branch (without it L = 16384
+// 53 us).
+struct MetropolisStage {
+    uint32_t flip, accept, open, m1;
+};
+
+__device__ __forceinline__ MetropolisStage metropolis_first(uint32_t s, uint32_t nu, uint32_t nd, uint32_t nl,
+                                                            uint32_t nr, uint32_t valid, const Accept &acc,
+                                                            const u32x4 &r)
 {
     const uint32_t a1 = s ^ nu, a2 = s ^ nd, a3 = s ^ nl, a4 = s ^ nr;
     const uint32_t x1 = a1 ^ a2, y1 = a1 & a2, x2 = a3 ^ a4, y2 = a3 & a4;
     const uint32_t any = a1 | a2 | a3 | a4;
-    const uint32_t c1 = (x1 ^ x2) & ~(y1 | y2);
-    const uint32_t c2 = ~any;
-    uint32_t flip = any & ~c1;
-    flip |= (acc.always0 ? c1 : 0u) | (acc.always1 ? c2 : 0u);
-    const uint32_t m1 = acc.always0 ? 0u : c1;
+    const uint32_t c1 = (x1 ^ x2) & ~(y1 | y2);  // one anti-aligned neighbour: e = 2
+    const uint32_t c2 = ~any;                    // none: e = 4
+    MetropolisStage st;
+    st.flip = any & ~c1;  // two or more: e <= 0
+    st.flip |= (acc.always0 ? c1 : 0u) | (acc.always1 ? c2 : 0u);
+    st.m1 = acc.always0 ? 0u : c1;
     const uint32_t m2 = acc.always1 ? 0u : c2;
-    uint32_t open = m1 | m2;
-    uint32_t accept = 0;
-    const uint32_t tag = (kTagSweep << 28) | (colour << 24);
+    st.open = (st.m1 | m2) & valid;
+    st.accept = 0;
     const uint32_t rq[4] = {r.v0, r.v1, r.v2, r.v3};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const uint32_t b0 = 0u - ((acc.thr0 >> (31 - q)) & 1u);
         const uint32_t b1 = 0u - ((acc.thr1 >> (31 - q)) & 1u);
-        const uint32_t tb = (m1 & b0) | (m2 & b1);
-        accept |= open & ~rq[q] & tb;
-        open &= ~(rq[q] ^ tb);
+        const uint32_t tb = (st.m1 & b0) | (m2 & b1);
+        st.accept |= st.open & ~rq[q] & tb;
+        st.open &= ~(rq[q] ^ tb);
     }
-    for (uint32_t rank = 0; open != 0u; ++rank) {
-        const uint32_t i = (uint32_t)__builtin_ctz(open);
-        open &= open - 1u;
-        if (rank != 0u && (rank & 3u) == 0u) ref = philox(word, t, 1u + (rank >> 2), tag, k0, k1);
-        const uint32_t low = pick4(ref, rank & 3u) >> 4;
-        const uint32_t thr = ((m1 >> i) & 1u) ? acc.thr0 : acc.thr1;
-        accept |= (low < (thr & 0x0FFFFFFFu) ? 1u : 0u) << i;
+    return st;
+}
+
+__device__ __forceinline__ uint32_t metropolis_second(MetropolisStage st, uint32_t valid, const Accept &acc,
+                                                      uint32_t k0, uint32_t k1, uint32_t word, uint32_t t,
+                                                      uint32_t colour, u32x4 ref)
+{
+    const uint32_t low0 = acc.thr0 << 4, low1 = acc.thr1 << 4;
+    metropolis_refine(st.open, st.accept, st.m1, ref.v0, low0, low1);
+    metropolis_refine(st.open, st.accept, st.m1, ref.v1, low0, low1);
+    metropolis_refine(st.open, st.accept, st.m1, ref.v2, low0, low1);
+    metropolis_refine(st.open, st.accept, st.m1, ref.v3, low0, low1);
+    for (uint32_t call = 2; st.open != 0u; ++call) {
+        ref = philox(word, t, call, (kTagSweep << 28) | (colour << 24), k0, k1);
+        metropolis_refine(st.open, st.accept, st.m1, ref.v0, low0, low1);
+        if (st.open != 0u) {
+            metropolis_refine(st.open, st.accept, st.m1, ref.v1, low0, low1);
+            metropolis_refine(st.open, st.accept, st.m1, ref.v2, low0, low1);
+            metropolis_refine(st.open, st.accept, st.m1, ref.v3, low0, low1);
+        }
     }
-    return flip | accept;
+    return (st.flip | st.accept) & valid;
+}
+
+__device__ __forceinline__ uint32_t metropolis_word_drawn(uint32_t s, uint32_t nu, uint32_t nd, uint32_t nl,
+                                                          uint32_t nr, uint32_t valid, const Accept &acc,
+                                                          uint32_t k0, uint32_t k1, uint32_t word, uint32_t t,
+                                                          uint32_t colour, const u32x4 &r, const u32x4 &ref)
+{
+    const MetropolisStage st = metropolis_first(s, nu, nd, nl, nr, valid, acc, r);
+    return metropolis_second(st, valid, acc, k0, k1, word, t, colour, ref);
+}
+
+// The same with both calls drawn here.
+__device__ __forceinline__ uint32_t metropolis_word(uint32_t s, uint32_t nu, uint32_t nd, uint32_t nl, uint32_t nr,
+                                                    uint32_t valid, const Accept &acc, uint32_t k0, uint32_t k1,
+                                                    uint32_t word, uint32_t t, uint32_t colour)
+{
+    const uint32_t tag = (kTagSweep << 28) | (colour << 24);
+    const MetropolisStage st =
+        metropolis_first(s, nu, nd, nl, nr, valid, acc, philox(word, t, 0u, tag, k0, k1));
+    return metropolis_second(st, valid, acc, k0, k1, word, t, colour, philox(word, t, 1u, tag, k0, k1));
 }
 
 // Spin bits of the 32 bytes at even (p = 0) or odd (p = 1) positions of a 64-byte

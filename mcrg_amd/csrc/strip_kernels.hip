@@ -525,7 +525,7 @@ __device__ void strip_body(const StripArgs &a, uint32_t *lds)
                 const uint32_t nl = p == 0u ? (o << 1) | (os >> 31) : o;
                 if (one)
                     own[row + q] ^= metropolis_word_drawn(own[row + q], oth[row - wpr + q], oth[row + wpr + q], nl, nr,
-                                                          acc, k0, k1, y * wpr + q, t, c, pr, pref);
+                                                          0xFFFFFFFFu, acc, k0, k1, y * wpr + q, t, c, pr, pref);
                 else
                     own[row + q] ^= metropolis_word(own[row + q], oth[row - wpr + q], oth[row + wpr + q], nl, nr,
                                                     0xFFFFFFFFu, acc, k0, k1, y * wpr + q, t, c);
@@ -627,8 +627,8 @@ __device__ __forceinline__ uint32_t strip_flip(const uint32_t *own, const uint32
     const uint32_t o = oth[row + q], os = oth[row + ((q + 2u * p - 1u) & mk)];
     const uint32_t nr = p == 0u ? o : (o >> 1) | (os << 31);
     const uint32_t nl = p == 0u ? (o << 1) | (os >> 31) : o;
-    return metropolis_word_drawn(own[row + q], oth[row - wpr + q], oth[row + wpr + q], nl, nr, acc, k0, k1,
-                                 y * wpr + q, t, c, r, ref);
+    return metropolis_word_drawn(own[row + q], oth[row - wpr + q], oth[row + wpr + q], nl, nr, 0xFFFFFFFFu, acc, k0,
+                                 k1, y * wpr + q, t, c, r, ref);
 }
 
 // The halo-row form of strip_body (sh.halo).  Rows y0-2 .. y0+R+1 are local
@@ -683,7 +683,8 @@ __device__ void strip_body_halo(const StripArgs &a, uint32_t *lds)
     if (threadIdx.x == 0) m.red[kRedAny] = 0u;
     __syncthreads();
     const Accept acc = lat.acc;
-    const uint32_t k0 = lat.k0, k1 = lat.k1, n = a.n_sweeps;
+    const uint32_t k0i = lat.k0, k1i = lat.k1, n = a.n_sweeps;
+    uint32_t kv0 = k0i, kv1 = k1i;
     const bool own = sh.measure && !sh.split;  // this workgroup measures its samples
     const uint32_t jw = threadIdx.x, jr = jw >> sw, q = jw & mk;
     const uint32_t j2 = jw + NT, jr2 = j2 >> sw, q2 = j2 & mk;
@@ -696,7 +697,7 @@ __device__ void strip_body_halo(const StripArgs &a, uint32_t *lds)
     const uint32_t row0 = (2u + jr) << sw, row1 = (1u + jr) << sw, row2 = (1u + jr2) << sw;
     u32x4 p0{0u, 0u, 0u, 0u}, p0r{0u, 0u, 0u, 0u}, p1{0u, 0u, 0u, 0u}, p1r{0u, 0u, 0u, 0u};
     u32x4 p2{0u, 0u, 0u, 0u}, p2r{0u, 0u, 0u, 0u};  // second words: 256-thread launches only
-    if (has0 && n > 0u) metropolis_rng(ya * wpr + q, a.t0, 0u, k0, k1, p0, p0r);
+    if (has0 && n > 0u) metropolis_rng(ya * wpr + q, a.t0, 0u, k0i, k1i, p0, p0r);
     // neighbour words: local rows 0, 1 from the upper strip's last two rows,
     // R+2, R+3 from the lower strip's first two (one word per thread)
     const bool get_h = jw < hw, get_f = own && jw < fw;
@@ -712,6 +713,11 @@ __device__ void strip_body_halo(const StripArgs &a, uint32_t *lds)
     bool ok = true, bad = false;
     uint32_t vote = 0;
     for (uint32_t it = 0; it < n; ++it) {
+        // the key anew in every sweep, so that its 18 round keys are formed
+        // beside the calls (scalar adds) instead of being kept through the loop
+        // (147 -> 113 VGPRs in the 256-thread kernel)
+        asm volatile("" : "+v"(kv0), "+v"(kv1));
+        const uint32_t k0 = __builtin_amdgcn_readfirstlane(kv0), k1 = __builtin_amdgcn_readfirstlane(kv1);
         const uint32_t t = a.t0 + it, seq = it + 1u, par = it & 1u;
         const bool pub = own && it >= 2u;
         // the lower strip's first blocked rows of sample it-2, sent during
