@@ -2,6 +2,7 @@
 // lockstep lattice groups.
 #include "hbm_group.hpp"
 
+#include <algorithm>
 #include <cstring>
 
 namespace mcrg {
@@ -86,6 +87,22 @@ hipError_t SweepRunner::run(const HbmLattice *d, int n_lats, int L, int n_levels
 {
     hipError_t e;
     uint32_t done = 0;
+    if (sampler == MCRG_SAMPLER_SWENDSEN_WANG && L <= kSwWgMaxL) {
+        if (cus_ == 0) {
+            int dev = 0;
+            if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+            if ((e = hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+        }
+        const int part = sw_wg_part(n_lats, L, cus_);
+        for (; done < n; done += std::min(n - done, kWgSweeps)) {
+            const int ev = tm ? tm->begin(kKindSweep, s) : -1;
+            if ((e = launch_sw_wg(d, n_lats, L, n_levels, part, std::min(n - done, kWgSweeps), measure, cus_, s)) !=
+                hipSuccess)
+                return e;
+            if (tm) tm->end(ev, s);
+        }
+        return hipSuccess;
+    }
     if (!tm && n >= kGraphSweeps) {
         hipGraphExec_t &exec = exec_[measure ? 1 : 0];
         if (!exec) {

@@ -34,6 +34,8 @@ hipError_t enqueue_sweeps(const HbmLattice *d, int n_lats, int L, int n_levels, 
 class SweepRunner {
   public:
     static constexpr uint32_t kGraphSweeps = 32;
+    // sweeps per launch of the one-workgroup kernels (tens of milliseconds)
+    static constexpr uint32_t kWgSweeps = 4096;
     SweepRunner() = default;
     SweepRunner(const SweepRunner &) = delete;
     SweepRunner &operator=(const SweepRunner &) = delete;
@@ -43,6 +45,7 @@ class SweepRunner {
 
   private:
     hipGraphExec_t exec_[2] = {nullptr, nullptr};
+    int cus_ = 0;
 };
 
 // Lattices that share L, level count, sweep counts and bin size, advanced

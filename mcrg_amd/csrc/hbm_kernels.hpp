@@ -111,6 +111,13 @@ struct HbmLattice {
 hipError_t launch_int8_init(const HbmLattice *d, int n_lats, int L, hipStream_t s);
 // One Swendsen-Wang sweep: label reset, bond draw + union, root coin + flip.
 hipError_t launch_sw_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off, hipStream_t s);
+// A Swendsen-Wang lattice of side at most kSwWgMaxL is swept and measured by
+// one workgroup in LDS: n sweeps of n_lats lattices (all measured or none) and
+// their counters in one launch, a thread for each `part` sites (sw_wg_part).
+constexpr int kSwWgMaxL = 128;
+int sw_wg_part(int n_lats, int L, int n_cus);
+hipError_t launch_sw_wg(const HbmLattice *d, int n_lats, int L, int n_levels, int part, uint32_t n, bool measure,
+                        int n_cus, hipStream_t s);
 hipError_t launch_int8_half_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
                                   uint32_t colour, hipStream_t s);
 hipError_t launch_int8_measure0(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
