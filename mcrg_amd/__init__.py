@@ -390,11 +390,10 @@ class Batch:
 
     def records(self, j):
         job = self.jobs[j]
-        rs = record_size(job.get("n_levels", 0))
-        nb = n_bins(job.get("n_meas", 0), job.get("sweeps_per_bin", 1))
-        a = np.zeros(nb * rs, dtype=np.int64)
-        check(_lib.mcrg_batch_get_records(self.handle, j, _ptr(a), a.size))
-        return a.reshape(nb, rs)
+        a = np.zeros((n_bins(job.get("n_meas", 0), job.get("sweeps_per_bin", 1)),
+                      22 * job.get("n_levels", 0) + 16), dtype=np.int64)  # record_size(n_levels)
+        check(_lib.mcrg_batch_get_records(self.handle, j, a.ctypes.data, a.size))
+        return a
 
     def spins(self, j):
         L = self.jobs[j]["L"]

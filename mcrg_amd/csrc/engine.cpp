@@ -767,4 +767,29 @@ hipError_t ResidentEngine::read_records(int id, int64_t *host, int64_t n)
     return check_parts(stream_);
 }
 
+size_t ResidentEngine::record_range(int id, int n, std::vector<size_t> &offsets) const
+{
+    offsets.clear();
+    size_t begin = 0, end = 0;
+    for (int k = id; k < id + n; ++k) {
+        const Job &job = jobs_[(size_t)k];
+        const size_t rec = job.off + round_up(2u * cb_words((uint32_t)job.spec.L) * 4u, 256);
+        if (k == id) begin = rec;
+        else if (rec < end) return 0;
+        offsets.push_back(rec - begin);
+        end = rec + (size_t)job.n_bins * record_size((uint32_t)job.spec.n_levels) * 8u;
+    }
+    return end - begin;
+}
+
+hipError_t ResidentEngine::read_range(int id, size_t bytes, char *host)
+{
+    hipError_t e;
+    if ((e = flush_pending()) != hipSuccess) return e;
+    const Job &job = jobs_[(size_t)id];
+    const char *rec = arena_.base() + job.off + round_up(2u * cb_words((uint32_t)job.spec.L) * 4u, 256);
+    if ((e = hipMemcpyAsync(host, rec, bytes, hipMemcpyDeviceToHost, stream_)) != hipSuccess) return e;
+    return check_parts(stream_);
+}
+
 }  // namespace mcrg

@@ -133,6 +133,11 @@ class ResidentEngine {
 
     hipError_t read_spins(int id, int8_t *host);  // row-major +-1 (synchronous)
     hipError_t read_records(int id, int64_t *host, int64_t n);
+    // The lattices id .. id + n - 1 as one range of the arena: where their
+    // records lie from its start, and its size (0 when they do not lie in order).
+    size_t record_range(int id, int n, std::vector<size_t> &offsets) const;
+    // Copies that range (spins between the records and all) to the host.
+    hipError_t read_range(int id, size_t bytes, char *host);
     // Records of several lattices through one pinned staging buffer and one wait.
     hipError_t read_records_many(const std::vector<int> &ids, const std::vector<int64_t *> &hosts,
                                  const std::vector<int64_t> &ns);

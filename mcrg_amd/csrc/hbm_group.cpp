@@ -9,6 +9,9 @@ namespace mcrg {
 
 static size_t align256(size_t v) { return (v + 255u) & ~size_t(255u); }
 
+// Cluster labels in device memory: lattices beyond one workgroup's LDS.
+static bool sw_labels(int L, int sampler) { return sampler == MCRG_SAMPLER_SWENDSEN_WANG && L > kSwWgMaxL; }
+
 HbmBlock hbm_block(int L, int n_levels, int max_bins, int sampler)
 {
     HbmBlock b;
@@ -22,7 +25,7 @@ HbmBlock hbm_block(int L, int n_levels, int max_bins, int sampler)
     b.state = align256(b.sums + kSumWords * 8u);
     b.rec = align256(b.state + 2u * 4u);
     b.labels = align256(b.rec + (size_t)max_bins * record_size((uint32_t)n_levels) * 8u);
-    b.bytes = align256(b.labels + (sampler == MCRG_SAMPLER_SWENDSEN_WANG ? n_spins * 4u : 0u));
+    b.bytes = align256(b.labels + (sw_labels(L, sampler) ? n_spins * 4u : 0u));
     return b;
 }
 
@@ -43,7 +46,7 @@ HbmLattice hbm_descriptor(char *base, const HbmBlock &b, int L, int n_levels, in
     h.n_levels = n_levels;
     h.sweeps_per_bin = sweeps_per_bin;
     h.sampler = sampler;
-    h.labels = sampler == MCRG_SAMPLER_SWENDSEN_WANG ? reinterpret_cast<int32_t *>(base + b.labels) : nullptr;
+    h.labels = sw_labels(L, sampler) ? reinterpret_cast<int32_t *>(base + b.labels) : nullptr;
     h.bond_thr = bond_threshold(coupling);
     return h;
 }
@@ -214,6 +217,25 @@ hipError_t HbmGroup::read_records(int member, int64_t *host, int64_t n, hipStrea
     if ((e = hipMemcpyAsync(host, host_[(size_t)member].records, (size_t)n * 8u, hipMemcpyDeviceToHost, s)) !=
         hipSuccess)
         return e;
+    return hipStreamSynchronize(s);
+}
+
+size_t HbmGroup::record_pitch() const
+{
+    const size_t width = (size_t)n_bins_ * record_size((uint32_t)spec().n_levels) * 8u;
+    return blk_.bytes <= 16u * width ? blk_.bytes : width;
+}
+
+hipError_t HbmGroup::read_records_block(int member, int count, char *host, hipStream_t s)
+{
+    hipError_t e;
+    const size_t width = (size_t)n_bins_ * record_size((uint32_t)spec().n_levels) * 8u, pitch = record_pitch();
+    const int64_t *rec = host_[(size_t)member].records;
+    if (pitch == blk_.bytes)
+        e = hipMemcpyAsync(host, rec, pitch * ((size_t)count - 1u) + width, hipMemcpyDeviceToHost, s);
+    else
+        e = hipMemcpy2DAsync(host, width, rec, blk_.bytes, width, (size_t)count, hipMemcpyDeviceToHost, s);
+    if (e != hipSuccess) return e;
     return hipStreamSynchronize(s);
 }
 

@@ -72,6 +72,11 @@ class HbmGroup {
         n_measured = q_;
     }
     hipError_t read_records(int member, int64_t *host, int64_t n, hipStream_t s);
+    // Records of members member .. member + count - 1, record_pitch() bytes
+    // apart: with what lies between them where that is little (one plain copy),
+    // else the records alone.
+    size_t record_pitch() const;
+    hipError_t read_records_block(int member, int count, char *host, hipStream_t s);
     hipError_t read_spins(int member, int8_t *host, hipStream_t s);
 
   private:
