@@ -9,8 +9,8 @@ namespace mcrg {
 
 static size_t align256(size_t v) { return (v + 255u) & ~size_t(255u); }
 
-// Cluster labels in device memory: lattices beyond one workgroup's LDS.
-static bool sw_labels(int L, int sampler) { return sampler == MCRG_SAMPLER_SWENDSEN_WANG && L > kSwWgMaxL; }
+// Tile scratch in device memory: cluster-sampled lattices beyond one workgroup's LDS.
+static bool sw_tiled(int L, int sampler) { return sampler == MCRG_SAMPLER_SWENDSEN_WANG && L > kSwWgMaxL; }
 
 HbmBlock hbm_block(int L, int n_levels, int max_bins, int sampler)
 {
@@ -24,8 +24,8 @@ HbmBlock hbm_block(int L, int n_levels, int max_bins, int sampler)
     b.sums = align256(b.lvl + n_lvl * 4u);
     b.state = align256(b.sums + kSumWords * 8u);
     b.rec = align256(b.state + 2u * 4u);
-    b.labels = align256(b.rec + (size_t)max_bins * record_size((uint32_t)n_levels) * 8u);
-    b.bytes = align256(b.labels + (sw_labels(L, sampler) ? n_spins * 4u : 0u));
+    b.sw = align256(b.rec + (size_t)max_bins * record_size((uint32_t)n_levels) * 8u);
+    b.bytes = align256(b.sw + (sw_tiled(L, sampler) ? sw_scratch_bytes(L) : 0u));
     return b;
 }
 
@@ -46,7 +46,7 @@ HbmLattice hbm_descriptor(char *base, const HbmBlock &b, int L, int n_levels, in
     h.n_levels = n_levels;
     h.sweeps_per_bin = sweeps_per_bin;
     h.sampler = sampler;
-    h.labels = sw_labels(L, sampler) ? reinterpret_cast<int32_t *>(base + b.labels) : nullptr;
+    h.sw = sw_tiled(L, sampler) ? reinterpret_cast<uint32_t *>(base + b.sw) : nullptr;
     h.bond_thr = bond_threshold(coupling);
     return h;
 }
@@ -58,7 +58,7 @@ hipError_t enqueue_sweeps(const HbmLattice *d, int n_lats, int L, int n_levels, 
     for (uint32_t i = 0; i < n; ++i) {
         if (sampler == MCRG_SAMPLER_SWENDSEN_WANG) {
             const int ev = tm ? tm->begin(kKindSweep, s) : -1;
-            if ((e = launch_sw_sweep(d, n_lats, L, i, s)) != hipSuccess) return e;
+            if ((e = launch_sw_sweep(d, n_lats, L, i, i == 0u, i + 1u == n, s)) != hipSuccess) return e;
             if (tm) tm->end(ev, s);
         } else {
             for (uint32_t c = 0; c < 2u; ++c) {
@@ -69,7 +69,9 @@ hipError_t enqueue_sweeps(const HbmLattice *d, int n_lats, int L, int n_levels, 
         }
         if (measure) {
             int ev = tm ? tm->begin(kKindMeasure0, s) : -1;
-            if ((e = launch_int8_measure0(d, n_lats, L, i, s)) != hipSuccess) return e;
+            e = sampler == MCRG_SAMPLER_SWENDSEN_WANG ? launch_sw_measure0(d, n_lats, L, i, s)
+                                                      : launch_int8_measure0(d, n_lats, L, i, s);
+            if (e != hipSuccess) return e;
             if (tm) tm->end(ev, s);
             ev = tm ? tm->begin(kKindLevels, s) : -1;
             if ((e = launch_levels_accumulate(d, n_lats, L, n_levels, i, i, s)) != hipSuccess) return e;

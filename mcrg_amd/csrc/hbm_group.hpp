@@ -16,7 +16,7 @@ namespace mcrg {
 
 // Byte offsets (256-aligned) of one lattice's buffers inside its device block.
 struct HbmBlock {
-    size_t spins = 0, lvl = 0, sums = 0, state = 0, rec = 0, labels = 0, bytes = 0;
+    size_t spins = 0, lvl = 0, sums = 0, state = 0, rec = 0, sw = 0, bytes = 0;
 };
 HbmBlock hbm_block(int L, int n_levels, int max_bins, int sampler);
 // Descriptor of the lattice whose block starts at `base`.

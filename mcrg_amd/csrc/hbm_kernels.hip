@@ -5,11 +5,6 @@
 //
 //   k_int8_init           Philox +-1 start        (Lattice::initialize_random_spins, src/lattice.cpp:33-41)
 //   k_int8_half_sweep     checkerboard Metropolis (replaces Wolff, src/ising.cpp:87-149)
-//   k_sw_local, k_sw_boundary, k_sw_flip
-//                         Swendsen-Wang cluster sweep: the Wolff construction
-//                         (src/ising.cpp:96-149) for every cluster at once, with
-//                         GPU union-find on atomicMin
-
 //   k_int8_measure0       level-0 NN/NNN/P + M and b=2 majority blocking into a
 //                         bit-packed level-1 lattice (src/lattice.cpp:102-120, src/mcrg.cpp:314-348)
 //   k_rm_level            one large blocked level: operators and the next
@@ -34,151 +29,6 @@ __global__ __launch_bounds__(256) void k_int8_init(const HbmLattice *__restrict_
     const u32x4 r = philox(m >> 7, 0u, 0u, kTagInit << 28, lat.k0, lat.k1);
     const uint32_t bit = (pick4(r, (m >> 5) & 3u) >> (m & 31u)) & 1u;
     lat.spins[m] = (int8_t)(1 - 2 * (int)bit);
-}
-
-// ---------------------------------------------------------------- Swendsen-Wang
-// Cluster labels form a union-find forest in which every site points to a
-// smaller (or equal) site index, so each tree's root is the smallest site of
-// its cluster whatever the order of the unions.  Two passes build it:
-//   k_sw_local     one workgroup per tile of up to 32 x 32 sites: bond draws,
-//                  union-find of the bonds inside the tile in LDS, then every
-//                  site's global label = its tile-local root (tile rows are
-//                  row-major segments, so the local minimum is the global one)
-//   k_sw_boundary  bonds that leave a tile (right edge, bottom edge), united
-//                  in the global labels with atomicMin
-// Loads of global labels may return stale values while other threads unite:
-// a label only decreases and always names a site of the same cluster, so a
-// stale read lengthens a path but never leaves the cluster, and the atomics
-// decide.
-constexpr uint32_t kSwTile = 32;
-
-__device__ __forceinline__ int32_t sw_root(const int32_t *labels, int32_t i)
-{
-    for (;;) {
-        const int32_t p = __hip_atomic_load(labels + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (p == i) return i;
-        i = p;
-    }
-}
-
-__device__ __forceinline__ void sw_unite(int32_t *labels, int32_t a, int32_t b)
-{
-    for (;;) {
-        a = sw_root(labels, a);
-        b = sw_root(labels, b);
-        if (a == b) return;
-        if (a > b) {
-            const int32_t t = a;
-            a = b;
-            b = t;
-        }
-        // link root b below a; if b stopped being a root, continue from its parent
-        const int32_t old = atomicMin(labels + b, a);
-        if (old == b) return;
-        b = old;
-    }
-}
-
-__device__ __forceinline__ int32_t lds_root(const int32_t *lab, int32_t i)
-{
-    for (;;) {
-        const int32_t p = lab[i];
-        if (p == i) return i;
-        i = p;
-    }
-}
-
-__device__ __forceinline__ void lds_unite(int32_t *lab, int32_t a, int32_t b)
-{
-    for (;;) {
-        a = lds_root(lab, a);
-        b = lds_root(lab, b);
-        if (a == b) return;
-        if (a > b) {
-            const int32_t t = a;
-            a = b;
-            b = t;
-        }
-        const int32_t old = atomicMin(lab + b, a);
-        if (old == b) return;
-        b = old;
-    }
-}
-
-// Tile of TW x TH sites, TW = TH = min(L, 32); blockIdx.x = tile (row-major).
-// Thread pairs of horizontally adjacent sites (2p, 2p+1) share one Philox call,
-// which holds both sites' right and down bond draws.
-__global__ __launch_bounds__(256) void k_sw_local(const HbmLattice *__restrict__ lats, uint32_t t_off)
-{
-    __shared__ int32_t lab[kSwTile * kSwTile];
-    const HbmLattice &lat = lats[blockIdx.y];
-    const uint32_t L = (uint32_t)lat.L, mask = L - 1u;
-    const uint32_t TW = L < kSwTile ? L : kSwTile, nt = TW * TW;
-    const uint32_t tiles_x = L / TW;
-    const uint32_t x0 = (blockIdx.x % tiles_x) * TW, y0 = (blockIdx.x / tiles_x) * TW;
-    const bool wrap = TW == L;  // one tile holds the whole lattice: periodic bonds stay inside
-    const uint32_t t = lat.state[0] + t_off;
-    for (uint32_t i = threadIdx.x; i < nt; i += blockDim.x) lab[i] = (int32_t)i;
-    __syncthreads();
-    for (uint32_t p = threadIdx.x; 2u * p < nt; p += blockDim.x) {
-        const uint32_t i0 = 2u * p, ly = i0 / TW, lx0 = i0 % TW;
-        const uint32_t m0 = (y0 + ly) * L + x0 + lx0;
-        const u32x4 r = philox(m0 >> 1, t, 0u, kTagSwBond << 28, lat.k0, lat.k1);
-        const uint32_t u[4] = {r.v0, r.v1, r.v2, r.v3};
-#pragma unroll
-        for (uint32_t k = 0; k < 2u; ++k) {
-            const uint32_t lx = lx0 + k, m = m0 + k;
-            const int8_t sm = lat.spins[m];
-            if (lx + 1u < TW || wrap) {
-                const uint32_t nb = (y0 + ly) * L + ((x0 + lx + 1u) & mask);
-                if (sm == lat.spins[nb] && u[2u * k] < lat.bond_thr)
-                    lds_unite(lab, (int32_t)(ly * TW + lx), (int32_t)(ly * TW + ((lx + 1u) & (TW - 1u))));
-            }
-            if (ly + 1u < TW || wrap) {
-                const uint32_t nb = ((y0 + ly + 1u) & mask) * L + x0 + lx;
-                if (sm == lat.spins[nb] && u[2u * k + 1u] < lat.bond_thr)
-                    lds_unite(lab, (int32_t)(ly * TW + lx), (int32_t)(((ly + 1u) & (TW - 1u)) * TW + lx));
-            }
-        }
-    }
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < nt; i += blockDim.x) {
-        const uint32_t rt = (uint32_t)lds_root(lab, (int32_t)i);
-        lat.labels[(y0 + i / TW) * L + x0 + i % TW] = (int32_t)((y0 + rt / TW) * L + x0 + rt % TW);
-    }
-}
-
-// Bonds leaving a tile: thread b < L^2/32 takes the right bond of a site on a
-// tile's right edge, the rest the down bond of a site on a bottom edge.
-__global__ __launch_bounds__(256) void k_sw_boundary(const HbmLattice *__restrict__ lats, uint32_t t_off)
-{
-    const HbmLattice &lat = lats[blockIdx.y];
-    const uint32_t L = (uint32_t)lat.L, mask = L - 1u;
-    const uint32_t half = L * (L / kSwTile);
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= 2u * half) return;
-    const bool down = b >= half;
-    const uint32_t c = down ? b - half : b;
-    const uint32_t edge = (c / L) * kSwTile + kSwTile - 1u, along = c % L;
-    const uint32_t x = down ? along : edge, y = down ? edge : along;
-    const uint32_t m = y * L + x;
-    const uint32_t nb = down ? ((y + 1u) & mask) * L + x : y * L + ((x + 1u) & mask);
-    const uint32_t t = lat.state[0] + t_off;
-    const u32x4 r = philox(m >> 1, t, 0u, kTagSwBond << 28, lat.k0, lat.k1);
-    const uint32_t u = pick4(r, 2u * (m & 1u) + (down ? 1u : 0u));
-    if (lat.spins[m] == lat.spins[nb] && u < lat.bond_thr) sw_unite(lat.labels, (int32_t)m, (int32_t)nb);
-}
-
-__global__ __launch_bounds__(256) void k_sw_flip(const HbmLattice *__restrict__ lats, uint32_t t_off)
-{
-    const HbmLattice &lat = lats[blockIdx.y];
-    const uint32_t n = (uint32_t)lat.L * (uint32_t)lat.L;
-    const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= n) return;
-    const uint32_t t = lat.state[0] + t_off;
-    const uint32_t root = (uint32_t)sw_root(lat.labels, (int32_t)m);
-    const u32x4 r = philox(root >> 7, t, 0u, kTagSwFlip << 28, lat.k0, lat.k1);
-    if ((pick4(r, (root >> 5) & 3u) >> (root & 31u)) & 1u) lat.spins[m] = (int8_t)(-lat.spins[m]);
 }
 
 // ---------------------------------------------------------------- sweep
@@ -538,19 +388,6 @@ hipError_t launch_int8_init(const HbmLattice *d, int n_lats, int L, hipStream_t 
 {
     const uint32_t n = (uint32_t)L * (uint32_t)L;
     hipLaunchKernelGGL(k_int8_init, dim3(cdiv(n, 256u), (uint32_t)n_lats), dim3(256), 0, s, d);
-    return hipGetLastError();
-}
-
-hipError_t launch_sw_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off, hipStream_t s)
-{
-    const uint32_t n = (uint32_t)L * (uint32_t)L;
-    const uint32_t tw = (uint32_t)L < kSwTile ? (uint32_t)L : kSwTile;
-    hipLaunchKernelGGL(k_sw_local, dim3(n / (tw * tw), (uint32_t)n_lats), dim3(256), 0, s, d, t_off);
-    if ((uint32_t)L > kSwTile) {
-        const uint32_t nb = 2u * (uint32_t)L * ((uint32_t)L / kSwTile);
-        hipLaunchKernelGGL(k_sw_boundary, dim3(cdiv(nb, 256u), (uint32_t)n_lats), dim3(256), 0, s, d, t_off);
-    }
-    hipLaunchKernelGGL(k_sw_flip, dim3(cdiv(n, 256u), (uint32_t)n_lats), dim3(256), 0, s, d, t_off);
     return hipGetLastError();
 }
 

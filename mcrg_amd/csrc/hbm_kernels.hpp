@@ -102,15 +102,21 @@ struct HbmLattice {
     int n_levels;
     int sweeps_per_bin;
     int sampler;                // MCRG_SAMPLER_METROPOLIS or MCRG_SAMPLER_SWENDSEN_WANG
-    int32_t *labels;            // L*L cluster labels (Swendsen-Wang only)
+    uint32_t *sw;               // tile scratch (Swendsen-Wang lattices beyond kSwWgMaxL)
     uint32_t bond_thr;          // floor((1 - exp(-2J)) 2^32): bond probability of an aligned pair
     uint32_t pad;
 };
 
 // Launchers (host).  `d` points to n_lats device descriptors that all share side L.
 hipError_t launch_int8_init(const HbmLattice *d, int n_lats, int L, hipStream_t s);
-// One Swendsen-Wang sweep: label reset, bond draw + union, root coin + flip.
-hipError_t launch_sw_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off, hipStream_t s);
+// One Swendsen-Wang sweep of lattices with L > kSwWgMaxL.  They are held as bits
+// in the tile scratch: the first sweep of a run of sweeps takes the spins from
+// the int8 lattice, the last one stores them there.  launch_sw_measure0 stands
+// in for launch_int8_measure0 within the run.
+hipError_t launch_sw_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off, bool first, bool last,
+                           hipStream_t s);
+hipError_t launch_sw_measure0(const HbmLattice *d, int n_lats, int L, uint32_t t_off, hipStream_t s);
+size_t sw_scratch_bytes(int L);
 // A Swendsen-Wang lattice of side at most kSwWgMaxL is swept and measured by
 // one workgroup in LDS: n sweeps of n_lats lattices (all measured or none) and
 // their counters in one launch, a thread for each `part` sites (sw_wg_part).

@@ -4,6 +4,11 @@
 //   k_sw_wg   a whole lattice of L <= kSwWgMaxL in one workgroup's LDS, for all
 //             the sweeps of a launch, with the measurement of every level and
 //             the records (src/lattice.cpp:102-120, src/mcrg.cpp:72-98, :314-348)
+//   k_sw_tile, k_sw_seam, k_sw_apply
+//             larger lattices, one sweep in three launches: clusters within
+//             64 x 64 tiles, their unions across tiles, the flips
+//   k_sw_measure0
+//             level-0 operators and the blocking into level 1, from bits
 #include <algorithm>
 #include <mutex>
 
@@ -374,6 +379,351 @@ hipError_t launch_sw_wg(const HbmLattice *d, int n_lats, int L, int n_levels, in
     case 32: return launch_sw_wg_pw<32>(d, n_lats, lds_bytes, n, measure, n_work, threads, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+// ------------------------------------------------------------------ tiles
+// A tile is 64 x 64 sites, two words a row.  k_sw_tile finds its clusters in
+// LDS.  A cluster that reaches none of the tile's edge sites is complete: it is
+// flipped there and then.  Each other cluster is a node, named by its largest
+// edge position (top 0..63, bottom 64..127, left 128..191, right 192..255); no
+// node is named 0, since site (0, 0) is also left position 128, so 0 in the
+// site map stands for clusters that are done.  k_sw_seam unites the nodes
+// across the tiles' edges, and k_sw_apply flips what is left by its root's coin.
+// A node is (parent node, smallest site); roots are linked by their sites, so
+// a tree's root holds the smallest site of the cluster.
+constexpr uint32_t kTile = 64, kTileWords = 128, kTileSites = 4096, kTileNodes = 256;
+constexpr uint32_t kTag = 0x80000000u;  // label of a root that is a node
+
+struct SwTiles {
+    uint32_t *bits;    // [L * L / 32] the lattice's row-major bits
+    uint32_t *runs;    // [tile][128] run bonds
+    uint64_t *nodes;   // [tile][256] parent | site << 32
+    uint64_t *seams;   // [tile][2] bonds over the right and the lower edge
+    uint8_t *map;      // [tile][4096] node of the run that starts at a site
+    uint8_t *edge;     // [tile][256] node of each edge position
+};
+
+__host__ __device__ inline size_t sw_tiles_words(uint32_t L)
+{
+    const size_t n = (size_t)L * L, tiles = n / kTileSites;
+    return n / 32u * 2u + tiles * (2u * kTileNodes + 4u + kTileSites / 4u + kTileNodes / 4u);
+}
+
+__device__ __forceinline__ SwTiles sw_tiles(const HbmLattice &lat)
+{
+    const uint32_t L = (uint32_t)lat.L;
+    const size_t n = (size_t)L * L, tiles = n / kTileSites;
+    SwTiles s;
+    s.nodes = reinterpret_cast<uint64_t *>(lat.sw);
+    s.seams = s.nodes + tiles * kTileNodes;
+    s.bits = reinterpret_cast<uint32_t *>(s.seams + tiles * 2u);
+    s.runs = s.bits + n / 32u;
+    s.map = reinterpret_cast<uint8_t *>(s.runs + n / 32u);
+    s.edge = s.map + tiles * kTileSites;
+    return s;
+}
+
+// The root of label x in a tile, where roots may carry a tag.
+__device__ __forceinline__ uint32_t tile_root(uint32_t *lab, uint32_t x)
+{
+    uint32_t p = lds_ld(lab + x);
+    if (p & kTag) return x;
+    for (;;) {
+        const uint32_t g = lds_ld(lab + p);
+        if (g == p || (g & kTag)) return p;
+        lds_st(lab + x, g);
+        x = p;
+        p = g;
+    }
+}
+
+// One workgroup per tile (blockIdx.x) and lattice (blockIdx.y), a thread for
+// each part of PW sites.  `first`: the spins come from the int8 lattice, else
+// from the bits of the sweep before.
+template <uint32_t PW>
+__global__ __launch_bounds__(kTileSites / PW) void k_sw_tile(const HbmLattice *__restrict__ lats, uint32_t t_off,
+                                                             uint32_t first)
+{
+    constexpr uint32_t NT = kTileSites / PW;
+    __shared__ uint32_t lab[33u * kTileWords];
+    // the lists of unions, later the site map
+    constexpr uint32_t kScratch = NT / 64u * kSwList > kTileSites / 4u ? NT / 64u * kSwList : kTileSites / 4u;
+    __shared__ __align__(16) uint32_t scratch[kScratch];
+    __shared__ uint32_t S[kTileWords + 2u], R[kTileWords], D[kTileWords], C[kTileWords], col[2], node_root[kTileNodes];
+    const HbmLattice &lat = lats[blockIdx.y];
+    const uint32_t L = (uint32_t)lat.L, mask = L - 1u, wpr = L >> 5;
+    const SwTiles st = sw_tiles(lat);
+    const uint32_t tiles_x = L / kTile, tx = blockIdx.x & (tiles_x - 1u), ty = blockIdx.x >> ilog2u(tiles_x);
+    const uint32_t x0 = tx * kTile, y0 = ty * kTile, tile = blockIdx.x;
+    const uint32_t t = lat.state[0] + t_off, k0 = lat.k0, k1 = lat.k1, thr = lat.bond_thr;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    // ---- spins: the tile's words, the row below it, the column right of it
+    if (tid < kTileWords + 2u) {
+        const uint32_t y = (y0 + (tid >> 1)) & mask, x = x0 + 32u * (tid & 1u);
+        S[tid] = first ? sw_load32(lat.spins + (size_t)y * L + x) : st.bits[y * wpr + (x >> 5)];
+    }
+    if (NT < kTileWords + 2u && tid < 2u) {
+        const uint32_t y = (y0 + kTile) & mask, x = x0 + 32u * tid;
+        S[kTileWords + tid] = first ? sw_load32(lat.spins + (size_t)y * L + x) : st.bits[y * wpr + (x >> 5)];
+    }
+    if (tid < 64u) {
+        const uint32_t y = y0 + lane, x = (x0 + kTile) & mask;
+        const uint32_t b = first ? ((uint32_t)(uint8_t)lat.spins[(size_t)y * L + x]) >> 7 : st.bits[y * wpr + (x >> 5)];
+        const uint64_t c = __ballot((b & 1u) != 0u);
+        if (lane < 2u) col[lane] = (uint32_t)(c >> (32u * lane));
+        // coin bits of row lane: 128 sites a call, of which the tile has half
+        const uint32_t m = y * L + x0;
+        const u32x4 r = philox(m >> 7, t, 0u, kTagSwFlip << 28, k0, k1);
+        C[2u * lane] = (m & 64u) ? r.v2 : r.v0;
+        C[2u * lane + 1u] = (m & 64u) ? r.v3 : r.v1;
+    }
+    const uint32_t i = tid / (32u / PW), lo = tid % (32u / PW) * PW, row = i >> 1;
+    uint32_t dr, dd;
+    sw_draw<PW>(((y0 + row) * L + x0 + 32u * (i & 1u) + lo) >> 1, t, thr, k0, k1, dr, dd);
+    dr = word_or<PW>(dr << lo);
+    dd = word_or<PW>(dd << lo);
+    __syncthreads();
+    // ---- bonds
+    if (lo == 0u) {
+        const uint32_t s = S[i];
+        const uint32_t next = (i & 1u) ? (col[row >> 5] >> (row & 31u)) : S[i + 1u];
+        R[i] = dr & ~(s ^ ((s >> 1) | (next << 31)));
+        D[i] = dd & ~(s ^ S[i + 2u]);
+    }
+    __syncthreads();
+    const uint32_t ends = 0x80000000u;
+    const uint32_t r = R[i] & ~ends, up = i >= 2u ? D[i - 2u] : 0u, rup = i >= 2u ? R[i - 2u] & ~ends : 0u;
+    const uint32_t pm = part_mask<PW>(lo);
+    sw_hook(lab, i, kTile, ~(r << 1) & pm, r, up, rup);
+    __syncthreads();
+    sw_unions(
+        lab, scratch + tid / 64u * kSwList, i, r, up & ~((up & r & rup) << 1) & run_later(up, r) & pm,
+        (i & 1u) ? 0u : R[i] & ends & pm, [&](uint32_t b) { return 33u * (i - 2u) + run_start(rup, b); },
+        [&](uint32_t) { return 33u * (i + 1u); });
+    __syncthreads();
+    // ---- nodes: the roots of the edge sites, each named by its largest position
+    for (uint32_t pos = tid; pos < kTileNodes; pos += NT) {
+        const uint32_t k = pos & 63u, side = pos >> 6;
+        const uint32_t y = side == 0u ? 0u : side == 1u ? 63u : k, x = side == 2u ? 0u : side == 3u ? 63u : k;
+        const uint32_t w = 2u * y + (x >> 5);
+        const uint32_t root = tile_root(lab, 33u * w + run_start(R[w] & ~ends, x & 31u));
+        __hip_atomic_fetch_max(lab + root, kTag | pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        node_root[pos] = root;
+    }
+    {
+        uint4 *z = reinterpret_cast<uint4 *>(scratch);
+        for (uint32_t k = tid; k < kTileSites / 16u; k += NT) z[k] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    __syncthreads();
+    for (uint32_t pos = tid; pos < kTileNodes; pos += NT) {
+        const uint32_t root = node_root[pos], id = lds_ld(lab + root) & 0xFFu;
+        st.edge[(size_t)tile * kTileNodes + pos] = (uint8_t)id;
+        if (id == pos) {
+            const uint32_t m = sw_site(root), site = (y0 + (m >> 6)) * L + x0 + (m & 63u);
+            st.nodes[(size_t)tile * kTileNodes + pos] =
+                (uint64_t)(tile * kTileNodes + pos) | ((uint64_t)site << 32);
+        }
+    }
+    // ---- every run: its node into the map, or its coin
+    uint32_t f = 0, starts = ~(r << 1) & pm;
+    uint8_t *map = reinterpret_cast<uint8_t *>(scratch);
+    while (starts != 0u) {
+        uint32_t s[4], x[4], p[4], g[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            s[k] = starts ? (uint32_t)__builtin_ctz(starts) : 32u;
+            starts &= starts - 1u;
+            x[k] = p[k] = 33u * i + (s[k] & 31u);
+            g[k] = lds_ld(lab + p[k]);  // g = the label of p, x the label before p
+        }
+        for (bool more = true; more;) {
+            more = false;
+            uint32_t h[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) h[k] = lds_ld(lab + ((g[k] & kTag) ? p[k] : g[k]));
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                if (g[k] == p[k] || (g[k] & kTag)) continue;
+                // p -> g -> h: p's label moves on to h unless g is a root
+                if (!(h[k] & kTag) && h[k] != g[k]) lds_st(lab + p[k], h[k]);
+                p[k] = g[k];
+                g[k] = h[k];
+                more = true;
+            }
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            if (s[k] >= 32u) continue;
+            if (g[k] & kTag) {
+                map[32u * i + s[k]] = (uint8_t)g[k];
+            } else {
+                const uint32_t m = sw_site(p[k]);
+                f |= ((C[m >> 5] >> (m & 31u)) & 1u) << s[k];
+            }
+        }
+    }
+    f = word_or<PW>(f);
+    if (lo == 0u) {
+        st.bits[(y0 + row) * wpr + (x0 >> 5) + (i & 1u)] = S[i] ^ ((r + f) ^ r);
+        st.runs[(size_t)tile * kTileWords + i] = r;
+    }
+    if (tid < 64u) {
+        const uint64_t b = __ballot((R[2u * lane + 1u] & ends) != 0u);
+        if (lane == 0u) {
+            st.seams[2u * tile] = b;
+            st.seams[2u * tile + 1u] = (uint64_t)D[kTileWords - 2u] | ((uint64_t)D[kTileWords - 1u] << 32);
+        }
+    }
+    __syncthreads();
+    {
+        const uint4 *z = reinterpret_cast<const uint4 *>(scratch);
+        uint4 *out = reinterpret_cast<uint4 *>(st.map + (size_t)tile * kTileSites);
+        for (uint32_t k = tid; k < kTileSites / 16u; k += NT) out[k] = z[k];
+    }
+}
+
+__device__ __forceinline__ uint64_t node_ld(const uint64_t *nodes, uint32_t x)
+{
+    return __hip_atomic_load(nodes + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The root of node x and its smallest site, paths halved on the way.
+__device__ __forceinline__ uint32_t node_root_of(uint64_t *nodes, uint32_t x, uint32_t &site)
+{
+    uint64_t e = node_ld(nodes, x);
+    for (;;) {
+        const uint32_t p = (uint32_t)e;
+        if (p == x) {
+            site = (uint32_t)(e >> 32);
+            return x;
+        }
+        const uint64_t g = node_ld(nodes, p);
+        if ((uint32_t)g != p)
+            __hip_atomic_store(reinterpret_cast<uint32_t *>(nodes + x), (uint32_t)g, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        x = p;
+        e = g;
+    }
+}
+
+// One wave per seam: blockIdx.x covers two tiles, waves 0, 1 the first one's
+// right and lower edge, 2, 3 the second's.
+__global__ __launch_bounds__(256) void k_sw_seam(const HbmLattice *__restrict__ lats)
+{
+    const HbmLattice &lat = lats[blockIdx.y];
+    const uint32_t L = (uint32_t)lat.L;
+    const SwTiles st = sw_tiles(lat);
+    const uint32_t tiles_x = L / kTile, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t tile = 2u * blockIdx.x + (wave >> 1);
+    const bool down = (wave & 1u) != 0u;
+    const uint32_t tx = tile & (tiles_x - 1u), ty = tile >> ilog2u(tiles_x);
+    const uint32_t other = down ? (((ty + 1u) & (tiles_x - 1u)) * tiles_x + tx)
+                                : (ty * tiles_x + ((tx + 1u) & (tiles_x - 1u)));
+    const uint64_t bonds = st.seams[2u * tile + (down ? 1u : 0u)];
+    const uint32_t a = st.edge[(size_t)tile * kTileNodes + (down ? 64u : 192u) + lane];
+    const uint32_t b = st.edge[(size_t)other * kTileNodes + (down ? 0u : 128u) + lane];
+    // a bond that joins the same two nodes as the one before it is left out
+    const uint32_t ab = a | (b << 8) | (uint32_t)((bonds >> lane) & 1u) << 16;
+    const uint32_t before = (uint32_t)__shfl_up((int)ab, 1, 64);
+    if ((ab >> 16) == 0u || (lane > 0u && before == ab)) return;
+    uint32_t u = tile * kTileNodes + a, v = other * kTileNodes + b;
+    for (;;) {
+        uint32_t su, sv;
+        u = node_root_of(st.nodes, u, su);
+        v = node_root_of(st.nodes, v, sv);
+        if (u == v) return;
+        const uint32_t lo = su < sv ? u : v;
+        uint32_t hi = su < sv ? v : u, expect = hi;
+        if (__hip_atomic_compare_exchange_strong(reinterpret_cast<uint32_t *>(st.nodes + hi), &expect, lo,
+                                                 __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            return;
+        // hi was linked meanwhile
+        u = lo;
+        v = expect;
+    }
+}
+
+// One workgroup per tile: the nodes' coins, then the flips of their runs; with
+// `last` the spins as int8 as well.
+__global__ __launch_bounds__(256) void k_sw_apply(const HbmLattice *__restrict__ lats, uint32_t t_off, uint32_t last)
+{
+    __shared__ uint8_t flip[kTileNodes];
+    const HbmLattice &lat = lats[blockIdx.y];
+    const uint32_t L = (uint32_t)lat.L, wpr = L >> 5, tid = threadIdx.x, tile = blockIdx.x;
+    const SwTiles st = sw_tiles(lat);
+    const uint4 ids = reinterpret_cast<const uint4 *>(st.map + (size_t)tile * kTileSites)[tid];
+    const uint32_t r = st.runs[(size_t)tile * kTileWords + (tid >> 1)];
+    uint32_t f = 0;
+    if (tid > 0u && st.edge[(size_t)tile * kTileNodes + tid] == tid) {
+        uint32_t site;
+        (void)node_root_of(st.nodes, tile * kTileNodes + tid, site);
+        const u32x4 c = philox(site >> 7, lat.state[0] + t_off, 0u, kTagSwFlip << 28, lat.k0, lat.k1);
+        f = (pick4(c, (site >> 5) & 3u) >> (site & 31u)) & 1u;
+    }
+    flip[tid] = (uint8_t)f;
+    __syncthreads();
+    // 16 sites a thread: the coins of the runs that start there (site map 0 and
+    // its flip are 0 elsewhere)
+    uint32_t w = 0;
+    const uint32_t d[4] = {ids.x, ids.y, ids.z, ids.w};
+#pragma unroll
+    for (uint32_t k = 0; k < 16u; ++k) w |= (uint32_t)flip[(d[k >> 2] >> (8u * (k & 3u))) & 0xFFu] << k;
+    w <<= 16u * (tid & 1u);
+    w |= (uint32_t)__shfl_xor((int)w, 1, 64);
+    if (tid & 1u) return;
+    const uint32_t i = tid >> 1, tiles_x = L / kTile, tx = tile & (tiles_x - 1u), ty = tile >> ilog2u(tiles_x);
+    const uint32_t y = ty * kTile + (i >> 1), x = tx * kTile + 32u * (i & 1u);
+    uint32_t *bits = st.bits + y * wpr + (x >> 5);
+    const uint32_t s = *bits ^ ((r + w) ^ r);
+    *bits = s;
+    if (last) sw_store32(lat.spins + (size_t)y * L + x, s);
+}
+
+// Level 0 from the bits: operators by words, and level 1 by its words.
+__global__ __launch_bounds__(256) void k_sw_measure0(const HbmLattice *__restrict__ lats, uint32_t t_off)
+{
+    __shared__ uint32_t part[4][4];
+    const HbmLattice &lat = lats[blockIdx.y];
+    const uint32_t L = (uint32_t)lat.L, i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t *bits = sw_tiles(lat).bits;
+    uint32_t c[4] = {0u, 0u, 0u, 0u};
+    rm_ops_item(bits, L, i, c[0], c[1], c[2]);
+    c[3] = (uint32_t)popc(bits[i]);
+    if (i < rm_block_items(L))
+        lat.lvl[i] = rm_block_item(bits, L, i, tie_coin_word(i, lat.state[0] + t_off, 0u, lat.k0, lat.k1));
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        c[k] = group_sum(c[k], 64u);
+        if ((threadIdx.x & 63u) == 0u) part[k][threadIdx.x >> 6] = c[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 4u) {
+        const uint32_t k = threadIdx.x;
+        atomicAdd(lat.sums + k, (unsigned long long)(part[k][0] + part[k][1] + part[k][2] + part[k][3]));
+    }
+}
+
+size_t sw_scratch_bytes(int L) { return sw_tiles_words((uint32_t)L) * 4u; }
+
+hipError_t launch_sw_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off, bool first, bool last, hipStream_t s)
+{
+    const uint32_t tiles = (uint32_t)((int64_t)L * L / kTileSites);
+    const dim3 grid(tiles, (uint32_t)n_lats);
+    // few tiles: more threads for each
+    if ((int64_t)tiles * n_lats <= 512)
+        hipLaunchKernelGGL(k_sw_tile<8>, grid, dim3(kTileSites / 8u), 0, s, d, t_off, first ? 1u : 0u);
+    else
+        hipLaunchKernelGGL(k_sw_tile<16>, grid, dim3(kTileSites / 16u), 0, s, d, t_off, first ? 1u : 0u);
+    hipLaunchKernelGGL(k_sw_seam, dim3(tiles / 2u, (uint32_t)n_lats), dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_sw_apply, grid, dim3(256), 0, s, d, t_off, last ? 1u : 0u);
+    return hipGetLastError();
+}
+
+hipError_t launch_sw_measure0(const HbmLattice *d, int n_lats, int L, uint32_t t_off, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_sw_measure0, dim3((uint32_t)((int64_t)L * L / 32 / 256), (uint32_t)n_lats), dim3(256), 0, s, d,
+                       t_off);
+    return hipGetLastError();
 }
 
 }  // namespace mcrg

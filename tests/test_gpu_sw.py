@@ -58,3 +58,29 @@ def test_batches_of_every_workgroup_size(amd, ctx, orc, L, n_jobs):
             s_ref, r_ref = orc.run_chain(L, j["coupling"], j["seed"], 2, 5, 2, 3, sampler=orc.SAMPLER_SW)
             assert np.array_equal(b.spins(i), s_ref), i
             assert np.array_equal(b.records(i), r_ref), i
+
+
+@pytest.mark.parametrize("L,J,runs", [(256, 0.0, (2, 3)), (256, KC, (1, 40)), (256, 3.0, (3, 1)), (256, 0.35, (2, 2)),
+                                      (512, KC, (4, 1)), (512, 0.6, (2,)), (1024, 0.47, (2,))])
+def test_tiled_lattices(amd, ctx, orc, L, J, runs):
+    """Lattices of 64 x 64 tiles: no bonds, one domain, clusters of every size;
+    runs shorter and longer than a captured graph, which hand the spins over
+    as int8."""
+    print("sw tiles", L, J, runs, flush=True)
+    _chain(amd, ctx, orc, L, J, 77 + L, 2, runs, 3, 4)
+
+
+@pytest.mark.parametrize("L,n_jobs", [(256, 33), (512, 9)])
+def test_tiled_batches(amd, ctx, orc, L, n_jobs):
+    """Enough tiles for the launch shape of many lattices."""
+    print("sw tiled batch", L, n_jobs, flush=True)
+    jobs = [dict(L=L, coupling=0.43 + 0.001 * i, seed=31 + i, n_therm=1, n_meas=3, n_levels=4, sweeps_per_bin=2,
+                 sampler=amd.SAMPLER_SWENDSEN_WANG) for i in range(n_jobs)]
+    with amd.Batch(ctx, jobs, sweeps_per_launch=2) as b:
+        b.run_all()
+        b.sync()
+        for i in (0, n_jobs // 2, n_jobs - 1):
+            j = jobs[i]
+            s_ref, r_ref = orc.run_chain(L, j["coupling"], j["seed"], 1, 3, 4, 2, sampler=orc.SAMPLER_SW)
+            assert np.array_equal(b.spins(i), s_ref), i
+            assert np.array_equal(b.records(i), r_ref), i
