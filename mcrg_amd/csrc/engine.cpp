@@ -5,6 +5,7 @@
 #include <cstring>
 
 #include "runtime.hpp"
+#include "small_core.hpp"
 
 namespace mcrg {
 
@@ -239,6 +240,20 @@ int ResidentEngine::group_size(int L, int nl, int NT) const
     return std::max(G, 1);
 }
 
+int ResidentEngine::small_group(int L, int n, bool alone) const
+{
+    // As few lattices a wave as leave a wave for each SIMD, or for each compute
+    // unit beside larger lattices: a team of T lanes draws T / W sweeps' random
+    // numbers and measures T samples at once, but every wave more takes issue
+    // slots from the others (1000 measured sweeps of 1024 x L = 16: 0.96 ms with
+    // one lattice a wave, 1.37 with four; of 4096: 2.12, four 1.45, 16 2.79).
+    const int waves = alone ? 4 * cus_ : cus_;
+    int G = 64 / (int)cb_words((uint32_t)L);
+    while (G > 1 && (n + G / 2 - 1) / (G / 2) <= waves) G /= 2;
+    while (G > 1 && G > opt_.max_group) G /= 2;
+    return G;
+}
+
 uint32_t ResidentEngine::lds_share(int L, int nl, int NT) const
 {
     const int G = group_size(L, nl, NT);
@@ -247,6 +262,7 @@ uint32_t ResidentEngine::lds_share(int L, int nl, int NT) const
 
 uint64_t ResidentEngine::slot_time_ns(int L, int G, uint32_t n_sweeps) const
 {
+    if (L <= kSmallMaxL) return (uint64_t)n_sweeps * kSmallSweepNs;
     const uint64_t sites_per_lane = (uint64_t)G * (uint64_t)L * (uint64_t)L / (uint64_t)threads_for(L);
     return (uint64_t)n_sweeps * (kSweepFixedNs + kSweepPerSiteNs * sites_per_lane);
 }
@@ -254,6 +270,8 @@ uint64_t ResidentEngine::slot_time_ns(int L, int G, uint32_t n_sweeps) const
 uint32_t ResidentEngine::slot_sweeps(int L, int G, uint32_t chunk) const
 {
     if (opt_.quantum_ns == 0) return chunk;
+    if (L <= kSmallMaxL)
+        return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(opt_.quantum_ns / kSmallSweepNs, chunk));
     const uint64_t sites_per_lane = (uint64_t)G * (uint64_t)L * (uint64_t)L / (uint64_t)threads_for(L);
     const uint64_t n = opt_.quantum_ns / (kSweepFixedNs + kSweepPerSiteNs * sites_per_lane);
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(n, chunk));
@@ -393,13 +411,16 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
         uint64_t work;
         uint32_t lds;
         int threads;
+        bool small;
     };
     std::vector<Pending> pend;
+    const bool alone = !groups.empty() && groups.begin()->first.L <= kSmallMaxL;  // the largest comes first
     slot_lats_.clear();
     for (auto &kv : groups) {
         const int L = kv.first.L, nl = kv.first.nl;
-        const int G = group_size(L, nl, threads_for(L));
         const std::vector<int> &ids = kv.second;
+        const bool small = L <= kSmallMaxL;
+        const int G = small ? small_group(L, (int)ids.size(), alone) : group_size(L, nl, threads_for(L));
         for (size_t a = 0; a < ids.size(); a += (size_t)G) {
             const int g = (int)std::min<size_t>((size_t)G, ids.size() - a);
             // positions: a power of two (so that teams tile the workgroup), empty ones are -1
@@ -418,7 +439,10 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
                 const Job &j = jobs_[(size_t)id];
                 work += (uint64_t)L * (uint64_t)L * std::min<uint64_t>(ns, j.therm_left + j.meas_left);
             }
-            pend.push_back({s, work, lds_bytes(L, gp, nl, threads_for(L)), threads_for(L)});
+            if (small)
+                pend.push_back({s, work, 4u * small_lds_words((uint32_t)L, (uint32_t)gp, (uint32_t)nl), 64, true});
+            else
+                pend.push_back({s, work, lds_bytes(L, gp, nl, threads_for(L)), threads_for(L), false});
         }
     }
     // launch classes by (workgroup size, workgroups resident on the device):
@@ -427,6 +451,8 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
     using ClassKey = std::pair<int, int>;  // (threads, resident workgroups)
     std::map<std::pair<int, uint32_t>, int> resident;  // (threads, slot LDS) -> resident workgroups
     auto key_of = [&](const Pending &p) {
+        // the small lattices' classes come first, one per size
+        if (p.small) return ClassKey((1 << 16) + p.s.L, 0);
         auto it = resident.find({p.threads, p.lds});
         if (it == resident.end())
             it = resident.emplace(std::make_pair(p.threads, p.lds), resident_max_active_groups(p.threads, p.lds)).first;
@@ -440,7 +466,7 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
     const int per_size = kMaxClasses / n_sizes;
     int c = -1, last_threads = -1, in_size = 0;
     for (auto &kv : class_of) {
-        if (kv.first.first != last_threads) {
+        if (kv.first.first != last_threads) {  // a small lattices' size is one of its own
             ++c;
             in_size = 1;
             last_threads = kv.first.first;
@@ -470,6 +496,8 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
         lc.count += 1;
         lc.lds = std::max(lc.lds, pend[i].lds);
         lc.threads = pend[i].threads;
+        lc.small = pend[i].small;
+        lc.L = pend[i].s.L;
         slots_.push_back(pend[i].s);
     }
 }
@@ -513,6 +541,7 @@ hipError_t ResidentEngine::upload_slots()
         if ((e = hipMalloc(&d_done_, sizeof(uint32_t) * done_cap_)) != hipSuccess) return e;
     }
     for (LaunchClass &lc : classes_) {
+        if (lc.small) continue;  // one workgroup per slot, no parts
         const int resident = resident_max_active_groups(lc.threads, lc.lds);
         if (resident <= 0) {
             failed_ = "hipOccupancyMaxActiveBlocksPerMultiprocessor";
@@ -564,24 +593,43 @@ hipError_t ResidentEngine::launch_classes(KernelTimer *tm)
 {
     hipError_t e;
     const int ev = tm ? tm->begin(kKindResident, stream_) : -1;
+    // Streams: stream_, then the auxiliary ones.  The small lattices' classes
+    // (first in classes_: their few waves have to be placed before the larger
+    // lattices fill the compute units) follow each other on one auxiliary
+    // stream beside larger ones, or run beside each other.
+    size_t n_small = 0;
+    while (n_small < classes_.size() && classes_[n_small].small) ++n_small;
+    const bool mixed = n_small > 0 && n_small < classes_.size();
+    auto stream_of = [&](size_t c) -> size_t {
+        if (c < n_small) return mixed ? 0 : c;
+        return mixed ? c - n_small + 1 : c;
+    };
     if (classes_.size() > 1) {
         if ((e = hipEventRecord(ev_fork_, stream_)) != hipSuccess) return e;
     }
+    bool used[kMaxClasses + 1] = {};
     for (size_t c = 0; c < classes_.size(); ++c) {
         const LaunchClass &lc = classes_[c];
-        hipStream_t s = c == 0 ? stream_ : aux_[c - 1];
-        if (c > 0 && (e = hipStreamWaitEvent(s, ev_fork_, 0)) != hipSuccess) return e;
+        const size_t k = stream_of(c);
+        hipStream_t s = k == 0 ? stream_ : aux_[k - 1];
+        if (k > 0 && !used[k] && (e = hipStreamWaitEvent(s, ev_fork_, 0)) != hipSuccess) return e;
+        used[k] = true;
         // one queue counter per class, 64 bytes apart
-        if ((e = launch_resident(lc.threads, d_slots_ + lc.first, lc.count, lc.n_sub, d_slot_lats_, d_lats_,
-                                 d_queue_ + 16u * c, d_done_ + lc.first, d_err_, lc.lds, (uint32_t)lc.grid, s)) !=
-            hipSuccess) {
+        if (lc.small)
+            e = launch_small(lc.L, d_slots_ + lc.first, lc.count, d_slot_lats_, d_lats_, lc.lds, s);
+        else
+            e = launch_resident(lc.threads, d_slots_ + lc.first, lc.count, lc.n_sub, d_slot_lats_, d_lats_,
+                                d_queue_ + 16u * (c - n_small), d_done_ + lc.first, d_err_, lc.lds, (uint32_t)lc.grid,
+                                s);
+        if (e != hipSuccess) {
             failed_ = "launch_resident";
             return e;
         }
-        if (c > 0) {
-            if ((e = hipEventRecord(ev_join_[c], s)) != hipSuccess) return e;
-            if ((e = hipStreamWaitEvent(stream_, ev_join_[c], 0)) != hipSuccess) return e;
-        }
+    }
+    for (size_t k = 1; k <= (size_t)kMaxClasses; ++k) {
+        if (!used[k]) continue;
+        if ((e = hipEventRecord(ev_join_[k], aux_[k - 1])) != hipSuccess) return e;
+        if ((e = hipStreamWaitEvent(stream_, ev_join_[k], 0)) != hipSuccess) return e;
     }
     if (tm) tm->end(ev, stream_);
     return hipSuccess;

@@ -46,6 +46,7 @@ class Arena {
 // Measured-sweep time model of one slot on MI355X (from per-L runs of the
 // batched workload: about 8 us per sample plus 75 ns per site a lane sweeps).
 constexpr uint64_t kSweepFixedNs = 8000;
+constexpr uint64_t kSmallSweepNs = 1500;  // a small lattice's measured sweep (one wave)
 constexpr uint64_t kSweepPerSiteNs = 75;
 
 // The autotuner keeps the configuration in use unless a candidate's measured
@@ -206,6 +207,9 @@ class ResidentEngine {
     size_t tune_next_ = 0;
     hipEvent_t tune_a_ = nullptr, tune_b_ = nullptr;
     void rebuild_slots(uint32_t chunk);
+    // Lattices per wave of n small lattices (L <= kSmallMaxL) of one shape;
+    // `alone`: no larger lattice is in the launch.
+    int small_group(int L, int n, bool alone) const;
     uint32_t slot_sweeps(int L, int G, uint32_t chunk) const;
     // Modelled time of n_sweeps measured sweeps of a slot (the cost model above).
     uint64_t slot_time_ns(int L, int G, uint32_t n_sweeps) const;
@@ -215,16 +219,18 @@ class ResidentEngine {
     // launch class; classes launch concurrently on their own streams, each
     // with its own dynamic LDS size, so that a few large lattices do not cut
     // the occupancy of every small one.
-    static constexpr int kMaxClasses = 6;
+    static constexpr int kMaxClasses = 6;  // of larger lattices
     struct LaunchClass {
         uint32_t first = 0, count = 0, lds = 0;
         int threads = 0, grid = 0;
         uint32_t n_sub = 1;  // parts per slot (sub_chunks)
+        bool small = false;  // slots of small lattices of side L, one wave each
+        int L = 0;
     };
     std::vector<LaunchClass> classes_;
-    hipStream_t aux_[kMaxClasses - 1] = {};
+    hipStream_t aux_[kMaxClasses] = {};  // one more, for the small lattices
     hipEvent_t ev_fork_ = nullptr;
-    hipEvent_t ev_join_[kMaxClasses] = {};
+    hipEvent_t ev_join_[kMaxClasses + 1] = {};  // by stream, from 1
     hipError_t upload_slots();
 
     int device_ = 0;

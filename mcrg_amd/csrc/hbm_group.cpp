@@ -108,6 +108,16 @@ hipError_t SweepRunner::run(const HbmLattice *d, int n_lats, int L, int n_levels
         }
         return hipSuccess;
     }
+    if (sampler == MCRG_SAMPLER_METROPOLIS && L >= kSmallChainMinL && L <= kSmallChainMaxL) {
+        for (; done < n; done += std::min(n - done, kSmallSweeps)) {
+            const int ev = tm ? tm->begin(kKindSweep, s) : -1;
+            if ((e = launch_small_chain(d, n_lats, L, n_levels, std::min(n - done, kSmallSweeps), measure, s)) !=
+                hipSuccess)
+                return e;
+            if (tm) tm->end(ev, s);
+        }
+        return hipSuccess;
+    }
     if (!tm && n >= kGraphSweeps) {
         hipGraphExec_t &exec = exec_[measure ? 1 : 0];
         if (!exec) {

@@ -35,7 +35,7 @@ class SweepRunner {
   public:
     static constexpr uint32_t kGraphSweeps = 32;
     // sweeps per launch of the one-workgroup kernels (tens of milliseconds)
-    static constexpr uint32_t kWgSweeps = 4096;
+    static constexpr uint32_t kWgSweeps = 4096, kSmallSweeps = 32768;
     SweepRunner() = default;
     SweepRunner(const SweepRunner &) = delete;
     SweepRunner &operator=(const SweepRunner &) = delete;

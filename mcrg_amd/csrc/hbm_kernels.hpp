@@ -124,6 +124,11 @@ constexpr int kSwWgMaxL = 128;
 int sw_wg_part(int n_lats, int L, int n_cus);
 hipError_t launch_sw_wg(const HbmLattice *d, int n_lats, int L, int n_levels, int part, uint32_t n, bool measure,
                         int n_cus, hipStream_t s);
+// Metropolis chains of 8 <= L <= 32: n sweeps (all measured or none) of n_lats
+// lattices and their counters in one launch, a wave each.
+constexpr int kSmallChainMinL = 8, kSmallChainMaxL = 32;
+hipError_t launch_small_chain(const HbmLattice *d, int n_lats, int L, int n_levels, uint32_t n, bool measure,
+                              hipStream_t s);
 hipError_t launch_int8_half_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
                                   uint32_t colour, hipStream_t s);
 hipError_t launch_int8_measure0(const HbmLattice *d, int n_lats, int L, uint32_t t_off,

@@ -152,6 +152,20 @@ struct Nbr4 {
     uint32_t nu, nd, nl, nr;
 };
 
+// The same for L <= 32 from the other colour's words o = oth[w], op = oth[w-1]
+// and on = oth[w+1] (indices mod W).
+__device__ __forceinline__ Nbr4 cb_neighbours_small(uint32_t o, uint32_t op, uint32_t on, uint32_t L, uint32_t c)
+{
+    Nbr4 n;
+    const SegMasks m = seg_masks(L);
+    n.nu = (o << m.r) | (op >> (32u - m.r));
+    n.nd = (o >> m.r) | (on << (32u - m.r));
+    const uint32_t m0 = c == 0u ? m.even : ~m.even;  // segments whose row has p = 0
+    n.nl = (rotl_seg(o, m) & m0) | (o & ~m0);
+    n.nr = (o & m0) | (rotr_seg(o, m) & ~m0);
+    return n;
+}
+
 __device__ __forceinline__ Nbr4 cb_neighbours(const uint32_t *oth, uint32_t L, uint32_t W, uint32_t w,
                                               uint32_t c)
 {
@@ -171,14 +185,7 @@ __device__ __forceinline__ Nbr4 cb_neighbours(const uint32_t *oth, uint32_t L, u
         n.nr = p == 0u ? o : (o >> 1) | (side << 31);
         n.nl = p == 0u ? (o << 1) | (side >> 31) : o;
     } else {
-        const SegMasks m = seg_masks(L);
-        const uint32_t o = oth[w];
-        const uint32_t op = oth[(w - 1u) & (W - 1u)], on = oth[(w + 1u) & (W - 1u)];
-        n.nu = (o << m.r) | (op >> (32u - m.r));
-        n.nd = (o >> m.r) | (on << (32u - m.r));
-        const uint32_t m0 = c == 0u ? m.even : ~m.even;  // segments whose row has p = 0
-        n.nl = (rotl_seg(o, m) & m0) | (o & ~m0);
-        n.nr = (o & m0) | (rotr_seg(o, m) & ~m0);
+        n = cb_neighbours_small(oth[w], oth[(w - 1u) & (W - 1u)], oth[(w + 1u) & (W - 1u)], L, c);
     }
     return n;
 }

@@ -386,12 +386,10 @@ __device__ void run_slot(const Slot sl, const int32_t *__restrict__ slot_lats,
     const uint32_t L = (uint32_t)sl.L, G = (uint32_t)sl.G, nl = (uint32_t)sl.n_levels;
     const uint32_t n_chunk = sl.n_sweeps;
     const uint32_t T = tm.T;
-    if constexpr (SHAPE != kShapeGeneric) {
-        // what the shape implies (slot_shape): teams of at least a wave and
-        // L >= 64, so the kernel keeps only those code paths
-        __builtin_assume(T >= 64u);
-        __builtin_assume(L >= 64u);
-    }
+    // lattices of L <= kSmallMaxL run in k_small
+    __builtin_assume(L >= 64u);
+    // what the wide shape implies (slot_shape): teams of at least a wave
+    if constexpr (SHAPE != kShapeGeneric) __builtin_assume(T >= 64u);
     const SlotLayout lay = slot_layout(L, G, nl, T);
     const uint32_t W = lay.W, rs = record_size(nl), nw = lay.team_waves;
     const uint32_t cstride = nw * (nl + 1u) * 4u;
