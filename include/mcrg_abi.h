@@ -175,7 +175,7 @@ mcrg_status mcrg_chain_operators(mcrg_chain ch, int64_t out[4]);
 /* ------------------------------------------------------------------ batches */
 /* Many independent chains (uneven L and coupling) advanced together.  Jobs of
  * 8 <= L <= 512 with the Metropolis sampler run on the resident schedule:
- * bit-packed lattices held in LDS by a persistent grid (L <= 32: in the
+ * bit-packed lattices held in LDS by a persistent grid (L <= 128: in the
  * registers of single waves), one launch per chunk of sweeps.  Jobs of L = 2, 4 and L >= 1024, and Swendsen-Wang jobs, run on the
  * HBM schedule (int8 in device memory): jobs of the same L, n_levels, n_therm,
  * n_meas, sweeps_per_bin and sampler share every launch, on
@@ -211,7 +211,7 @@ typedef struct {
                                   0 = 32 KiB per 256 threads                    */
     int32_t min_team;          /* lanes per lattice at least (1..threads, power
                                   of two); 0 = 16.  The team and workgroup sizes
-                                  are those of L >= 64; smaller lattices take
+                                  are those of L >= 256; smaller lattices take
                                   64 / (lattices of the wave) lanes             */
     int32_t max_team;          /* lanes per lattice at most (power of two,
                                   >= min_team); 0 = threads                     */

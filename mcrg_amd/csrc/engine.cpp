@@ -5,7 +5,7 @@
 #include <cstring>
 
 #include "runtime.hpp"
-#include "small_core.hpp"
+#include "wave_core.hpp"
 
 namespace mcrg {
 
@@ -262,7 +262,7 @@ uint32_t ResidentEngine::lds_share(int L, int nl, int NT) const
 
 uint64_t ResidentEngine::slot_time_ns(int L, int G, uint32_t n_sweeps) const
 {
-    if (L <= kSmallMaxL) return (uint64_t)n_sweeps * kSmallSweepNs;
+    if (L <= kWaveMaxL) return (uint64_t)n_sweeps * wave_sweep_ns(L);
     const uint64_t sites_per_lane = (uint64_t)G * (uint64_t)L * (uint64_t)L / (uint64_t)threads_for(L);
     return (uint64_t)n_sweeps * (kSweepFixedNs + kSweepPerSiteNs * sites_per_lane);
 }
@@ -270,8 +270,8 @@ uint64_t ResidentEngine::slot_time_ns(int L, int G, uint32_t n_sweeps) const
 uint32_t ResidentEngine::slot_sweeps(int L, int G, uint32_t chunk) const
 {
     if (opt_.quantum_ns == 0) return chunk;
-    if (L <= kSmallMaxL)
-        return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(opt_.quantum_ns / kSmallSweepNs, chunk));
+    if (L <= kWaveMaxL)
+        return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(opt_.quantum_ns / wave_sweep_ns(L), chunk));
     const uint64_t sites_per_lane = (uint64_t)G * (uint64_t)L * (uint64_t)L / (uint64_t)threads_for(L);
     const uint64_t n = opt_.quantum_ns / (kSweepFixedNs + kSweepPerSiteNs * sites_per_lane);
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(n, chunk));
@@ -419,8 +419,8 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
     for (auto &kv : groups) {
         const int L = kv.first.L, nl = kv.first.nl;
         const std::vector<int> &ids = kv.second;
-        const bool small = L <= kSmallMaxL;
-        const int G = small ? small_group(L, (int)ids.size(), alone) : group_size(L, nl, threads_for(L));
+        const bool small = L <= kWaveMaxL;
+        const int G = L <= kSmallMaxL ? small_group(L, (int)ids.size(), alone) : small ? 1 : group_size(L, nl, threads_for(L));
         for (size_t a = 0; a < ids.size(); a += (size_t)G) {
             const int g = (int)std::min<size_t>((size_t)G, ids.size() - a);
             // positions: a power of two (so that teams tile the workgroup), empty ones are -1
@@ -440,7 +440,10 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
                 work += (uint64_t)L * (uint64_t)L * std::min<uint64_t>(ns, j.therm_left + j.meas_left);
             }
             if (small)
-                pend.push_back({s, work, 4u * small_lds_words((uint32_t)L, (uint32_t)gp, (uint32_t)nl), 64, true});
+                pend.push_back({s, work,
+                                4u * (L <= kSmallMaxL ? small_lds_words((uint32_t)L, (uint32_t)gp, (uint32_t)nl)
+                                                      : wave_lds_words((uint32_t)L, (uint32_t)nl)),
+                                64, true});
             else
                 pend.push_back({s, work, lds_bytes(L, gp, nl, threads_for(L)), threads_for(L), false});
         }
@@ -451,8 +454,8 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
     using ClassKey = std::pair<int, int>;  // (threads, resident workgroups)
     std::map<std::pair<int, uint32_t>, int> resident;  // (threads, slot LDS) -> resident workgroups
     auto key_of = [&](const Pending &p) {
-        // the small lattices' classes come first, one per size
-        if (p.small) return ClassKey((1 << 16) + p.s.L, 0);
+        // the one-wave slots' class comes first
+        if (p.small) return ClassKey(1 << 16, 0);
         auto it = resident.find({p.threads, p.lds});
         if (it == resident.end())
             it = resident.emplace(std::make_pair(p.threads, p.lds), resident_max_active_groups(p.threads, p.lds)).first;
@@ -461,12 +464,13 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
     auto key_less = [](const ClassKey &a, const ClassKey &b) { return a.first != b.first ? a.first > b.first : a.second > b.second; };
     std::map<ClassKey, int, decltype(key_less)> class_of(key_less);
     for (const Pending &p : pend) class_of[key_of(p)] = 0;
-    // at most kMaxClasses / (workgroup sizes in use) classes per workgroup size
+    // beside the one-wave slots', at most (kMaxClasses - 1) / (workgroup sizes in
+    // use) classes per workgroup size
     const int n_sizes = opt_.threads_large > 0 && opt_.threads_large != opt_.threads ? 2 : 1;
-    const int per_size = kMaxClasses / n_sizes;
+    const int per_size = (kMaxClasses - 1) / n_sizes;
     int c = -1, last_threads = -1, in_size = 0;
     for (auto &kv : class_of) {
-        if (kv.first.first != last_threads) {  // a small lattices' size is one of its own
+        if (kv.first.first != last_threads) {
             ++c;
             in_size = 1;
             last_threads = kv.first.first;
@@ -497,7 +501,6 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
         lc.lds = std::max(lc.lds, pend[i].lds);
         lc.threads = pend[i].threads;
         lc.small = pend[i].small;
-        lc.L = pend[i].s.L;
         slots_.push_back(pend[i].s);
     }
 }
@@ -593,43 +596,30 @@ hipError_t ResidentEngine::launch_classes(KernelTimer *tm)
 {
     hipError_t e;
     const int ev = tm ? tm->begin(kKindResident, stream_) : -1;
-    // Streams: stream_, then the auxiliary ones.  The small lattices' classes
-    // (first in classes_: their few waves have to be placed before the larger
-    // lattices fill the compute units) follow each other on one auxiliary
-    // stream beside larger ones, or run beside each other.
-    size_t n_small = 0;
-    while (n_small < classes_.size() && classes_[n_small].small) ++n_small;
-    const bool mixed = n_small > 0 && n_small < classes_.size();
-    auto stream_of = [&](size_t c) -> size_t {
-        if (c < n_small) return mixed ? 0 : c;
-        return mixed ? c - n_small + 1 : c;
-    };
     if (classes_.size() > 1) {
         if ((e = hipEventRecord(ev_fork_, stream_)) != hipSuccess) return e;
     }
-    bool used[kMaxClasses + 1] = {};
+    // The one-wave slots come first: their waves have to be placed before the
+    // larger lattices' persistent workgroups fill the compute units (the other
+    // way round the whole manifest of uneven sizes took 137 instead of 110 ms).
     for (size_t c = 0; c < classes_.size(); ++c) {
         const LaunchClass &lc = classes_[c];
-        const size_t k = stream_of(c);
-        hipStream_t s = k == 0 ? stream_ : aux_[k - 1];
-        if (k > 0 && !used[k] && (e = hipStreamWaitEvent(s, ev_fork_, 0)) != hipSuccess) return e;
-        used[k] = true;
+        hipStream_t s = c == 0 ? stream_ : aux_[c - 1];
+        if (c > 0 && (e = hipStreamWaitEvent(s, ev_fork_, 0)) != hipSuccess) return e;
         // one queue counter per class, 64 bytes apart
         if (lc.small)
-            e = launch_small(lc.L, d_slots_ + lc.first, lc.count, d_slot_lats_, d_lats_, lc.lds, s);
+            e = launch_wave(d_slots_ + lc.first, lc.count, d_slot_lats_, d_lats_, lc.lds, s);
         else
             e = launch_resident(lc.threads, d_slots_ + lc.first, lc.count, lc.n_sub, d_slot_lats_, d_lats_,
-                                d_queue_ + 16u * (c - n_small), d_done_ + lc.first, d_err_, lc.lds, (uint32_t)lc.grid,
-                                s);
+                                d_queue_ + 16u * c, d_done_ + lc.first, d_err_, lc.lds, (uint32_t)lc.grid, s);
         if (e != hipSuccess) {
             failed_ = "launch_resident";
             return e;
         }
-    }
-    for (size_t k = 1; k <= (size_t)kMaxClasses; ++k) {
-        if (!used[k]) continue;
-        if ((e = hipEventRecord(ev_join_[k], aux_[k - 1])) != hipSuccess) return e;
-        if ((e = hipStreamWaitEvent(stream_, ev_join_[k], 0)) != hipSuccess) return e;
+        if (c > 0) {
+            if ((e = hipEventRecord(ev_join_[c], s)) != hipSuccess) return e;
+            if ((e = hipStreamWaitEvent(stream_, ev_join_[c], 0)) != hipSuccess) return e;
+        }
     }
     if (tm) tm->end(ev, stream_);
     return hipSuccess;

@@ -46,7 +46,8 @@ class Arena {
 // Measured-sweep time model of one slot on MI355X (from per-L runs of the
 // batched workload: about 8 us per sample plus 75 ns per site a lane sweeps).
 constexpr uint64_t kSweepFixedNs = 8000;
-constexpr uint64_t kSmallSweepNs = 1500;  // a small lattice's measured sweep (one wave)
+// A measured sweep of a lattice held by one wave, on a filled device.
+inline uint64_t wave_sweep_ns(int L) { return L <= 32 ? 1500 : L == 64 ? 2500 : 6000; }
 constexpr uint64_t kSweepPerSiteNs = 75;
 
 // The autotuner keeps the configuration in use unless a candidate's measured
@@ -219,18 +220,17 @@ class ResidentEngine {
     // launch class; classes launch concurrently on their own streams, each
     // with its own dynamic LDS size, so that a few large lattices do not cut
     // the occupancy of every small one.
-    static constexpr int kMaxClasses = 6;  // of larger lattices
+    static constexpr int kMaxClasses = 6;
     struct LaunchClass {
         uint32_t first = 0, count = 0, lds = 0;
         int threads = 0, grid = 0;
         uint32_t n_sub = 1;  // parts per slot (sub_chunks)
-        bool small = false;  // slots of small lattices of side L, one wave each
-        int L = 0;
+        bool small = false;  // slots of lattices of L <= kWaveMaxL, one wave each
     };
     std::vector<LaunchClass> classes_;
-    hipStream_t aux_[kMaxClasses] = {};  // one more, for the small lattices
+    hipStream_t aux_[kMaxClasses - 1] = {};
     hipEvent_t ev_fork_ = nullptr;
-    hipEvent_t ev_join_[kMaxClasses + 1] = {};  // by stream, from 1
+    hipEvent_t ev_join_[kMaxClasses] = {};
     hipError_t upload_slots();
 
     int device_ = 0;

@@ -122,10 +122,10 @@ hipError_t launch_resident(int threads, const Slot *slots, uint32_t n_slots, uin
                            const int32_t *slot_lats, PackedLattice *lats, uint32_t *queue, uint32_t *done,
                            uint32_t *err, uint32_t lds_bytes, uint32_t grid, hipStream_t s);
 int resident_max_active_groups(int threads, uint32_t lds_bytes);
-// Slots of lattices of one side L <= kSmallMaxL, one wave each (small_core.hpp);
-// G is a power of two, at most 64 / cb_words(L).
-constexpr int kSmallMaxL = 32;
-hipError_t launch_small(int L, const Slot *slots, uint32_t n_slots, const int32_t *slot_lats, PackedLattice *lats,
-                        uint32_t lds_bytes, hipStream_t s);
+// Slots of one wave each: one lattice of L = 64 or 128 (wave_core.hpp), or G
+// smaller ones, G a power of two, at most 64 / cb_words(L) (small_core.hpp).
+constexpr int kSmallMaxL = 32, kWaveMaxL = 128;
+hipError_t launch_wave(const Slot *slots, uint32_t n_slots, const int32_t *slot_lats, PackedLattice *lats,
+                       uint32_t lds_bytes, hipStream_t s);
 
 }  // namespace mcrg

@@ -1,64 +1,10 @@
-// Small lattices (L = 8, 16, 32) held in the registers of one wave
+// int8 chains of L = 8, 16, 32 held in the registers of one wave
 // (small_core.hpp): Metropolis sweeps (replacing src/ising.cpp:87-149) and the
 // measurement of every level (src/lattice.cpp:102-120, src/mcrg.cpp:72-98,
 // :314-348).
-//
-//   k_small        batch and server jobs: one wave per slot of 64 / T lattices
-//   k_small_chain  int8 chains: one wave per lattice
 #include "small_core.hpp"
 
 namespace mcrg {
-
-template <uint32_t L>
-__device__ __forceinline__ void small_slot(const Slot &sl, const int32_t *__restrict__ slot_lats,
-                                           PackedLattice *__restrict__ lats, uint32_t *lds)
-{
-    constexpr uint32_t W = L * L / 64u;
-    const uint32_t T = 64u / (uint32_t)sl.G, lane = threadIdx.x, u = lane & (T - 1u), w = u & (W - 1u);
-    const int32_t li = slot_lats[sl.first + (int32_t)(lane / T)];
-    SmallLattice me{};
-    uint32_t c0 = 0, c1 = 0;
-    me.spb = 1u;
-    if (li >= 0) {
-        const PackedLattice &P = lats[li];
-        me.alive = true;
-        me.k0 = P.k0;
-        me.k1 = P.k1;
-        me.acc = P.acc;
-        me.t = P.t;
-        me.therm = P.therm_left;
-        me.meas = P.meas_left;
-        me.n_measured = P.n_measured;
-        me.spb = (uint32_t)P.sweeps_per_bin;
-        me.records = P.records;
-        c0 = P.spins[w];
-        c1 = P.spins[W + w];
-    }
-    run_small<L>(me, sl.n_sweeps, (uint32_t)sl.n_levels, T, lds, c0, c1);
-    if (li >= 0) {
-        PackedLattice &P = lats[li];
-        if (u < W) {
-            P.spins[w] = c0;
-            P.spins[W + w] = c1;
-        }
-        if (u == 0u) {
-            const uint32_t total = me.therm + me.meas, swept = total < sl.n_sweeps ? total : sl.n_sweeps;
-            const uint32_t measured = swept > me.therm ? swept - me.therm : 0u;
-            P.t = me.t + swept;
-            P.n_measured = me.n_measured + measured;
-            P.therm_left = me.therm - (swept - measured);
-            P.meas_left = me.meas - measured;
-        }
-    }
-}
-
-template <uint32_t L>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_small(
-    const Slot *__restrict__ slots, const int32_t *__restrict__ slot_lats, PackedLattice *__restrict__ lats)
-{
-    extern __shared__ uint32_t lds[];
-    small_slot<L>(slots[blockIdx.x], slot_lats, lats, lds);
-}
 
 // One int8 lattice: its words through LDS, n sweeps, all measured or none, and
 // its counters.
@@ -109,17 +55,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         lat.state[0] = me.t + n;
         lat.state[1] = me.n_measured + me.meas;
     }
-}
-
-hipError_t launch_small(int L, const Slot *slots, uint32_t n_slots, const int32_t *slot_lats, PackedLattice *lats,
-                        uint32_t lds_bytes, hipStream_t s)
-{
-    const dim3 grid(n_slots), block(64);
-    if (L == 8) hipLaunchKernelGGL(k_small<8u>, grid, block, lds_bytes, s, slots, slot_lats, lats);
-    else if (L == 16) hipLaunchKernelGGL(k_small<16u>, grid, block, lds_bytes, s, slots, slot_lats, lats);
-    else if (L == 32) hipLaunchKernelGGL(k_small<32u>, grid, block, lds_bytes, s, slots, slot_lats, lats);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
 }
 
 hipError_t launch_small_chain(const HbmLattice *d, int n_lats, int L, int n_levels, uint32_t n, bool measure,
