@@ -62,10 +62,12 @@ struct StripShape {
     // and the first halo row on each side itself (the same counters give the
     // neighbours' decisions).  Strips of at most 512 colour-1 words.
     uint32_t halo;
-    // measured halo launches with a second workgroup per strip (split): the
-    // strip publishes each sample's rows y0-1 .. y0+R (snap_words (data, seq)
-    // words) and workgroup n_wg + w measures them, so a strip's sweeps no
-    // longer wait for its measurements
+    // measured halo launches with `split` (1 or 2) more workgroups per strip:
+    // the strip publishes each sample's rows y0-1 .. y0+R (snap_words (data,
+    // seq) words) and workgroup n_wg + (k mod split) n_wg + w measures sample k
+    // of strip w, so a strip's sweeps no longer wait for its measurements.  A
+    // measuring workgroup takes about 13,400 cycles a sample at L = 2048, a
+    // strip 7,800 a sweep: two of them, each on every other sample, keep up.
     uint32_t split, n_meas, snap_words, first_slots;
     // device workspace, offsets in 32-bit words (even where 64-bit words
     // start), all of it cleared per launch:
@@ -76,8 +78,8 @@ struct StripShape {
     //   o_xfirst    (data, seq) words: [strip][first rows of levels 1..lam],
     //               with halo [sample mod first_slots][strip][...]
     //   o_ring      (data, seq) words: [slot][strip][per_wg]
-    //   o_snapc     with split, per strip: samples its measuring workgroup
-    //               has copied (kStripFlagStride apart)
+    //   o_snapc     with split, per measuring workgroup: one more than the
+    //               last sample it has copied (kStripFlagStride apart)
     //   o_snap      with split, (data, seq) words: [slot][strip][snap_words]
     uint32_t o_err, o_consumed, o_xhalo, o_xfirst, o_ring, o_snapc, o_snap, ws_words;
     uint32_t cnt_words;                 // 4 counts per level 0..lam
@@ -94,9 +96,10 @@ __host__ __device__ inline uint32_t strip_row_words(uint32_t L, uint32_t l) { re
 
 // n_wg strips of R = L / n_wg >= 2 rows; lam = min(log2 R, nl) levels block
 // inside a strip.  `halo_ok` allows the halo-row mode where the strip fits it,
-// `split_ok` its measuring workgroups.
+// `split_ok` its measuring workgroups, `sides` a strip.
 __host__ __device__ inline StripShape strip_shape(uint32_t L, uint32_t nl, uint32_t n_wg, uint32_t n_tail,
-                                                  bool measure, bool halo_ok = true, bool split_ok = false)
+                                                  bool measure, bool halo_ok = true, bool split_ok = false,
+                                                  uint32_t sides = 1)
 {
     StripShape s;
     s.L = L;
@@ -125,8 +128,8 @@ __host__ __device__ inline StripShape strip_shape(uint32_t L, uint32_t nl, uint3
         s.overlap = measure && words <= s.threads ? 1u : 0u;
     }
     const uint32_t rows = s.R + 2u + 2u * s.halo;  // rows held in LDS
-    s.split = s.halo && measure && split_ok ? 1u : 0u;
-    s.n_meas = s.split ? n_wg : 0u;
+    s.split = s.halo && measure && split_ok ? sides : 0u;
+    s.n_meas = s.split * n_wg;
     s.snap_words = s.split ? 2u * (s.R + 2u) * s.wpr : 0u;
     s.first_slots = s.halo ? (s.split ? kStripFirstSlotsSplit : kStripFirstSlots) : 1u;
     uint32_t lg = 0;
@@ -147,7 +150,7 @@ __host__ __device__ inline StripShape strip_shape(uint32_t L, uint32_t nl, uint3
     s.o_xfirst = s.o_xhalo + 2u * (2u * n_wg * (2u + 2u * s.halo) * s.wpr);
     s.o_ring = s.o_xfirst + 2u * s.first_slots * n_wg * s.first_words;
     s.o_snapc = s.o_ring + (measure ? 2u * kStripRing * n_wg * s.per_wg : 0u);
-    s.o_snap = s.o_snapc + (s.split ? n_wg * kStripFlagStride : 0u);
+    s.o_snap = s.o_snapc + s.n_meas * kStripFlagStride;
     s.ws_words = s.o_snap + 2u * kStripSnapSlots * n_wg * s.snap_words;
     // strip: both colours of rows y0-1 .. y0+R (y0-2 .. y0+R+1 with halo), the
     // in-strip levels and their tie coins, the pending sample's first and last

@@ -706,7 +706,8 @@ __device__ void strip_body_halo(const StripArgs &a, uint32_t *lds)
     // with split: the samples the measuring workgroup has copied, as last seen
     const uint32_t *snapc = a.ws + sh.o_snapc + w * kStripFlagStride;
     uint64_t *snap = reinterpret_cast<uint64_t *>(a.ws + sh.o_snap);
-    uint32_t copied = 0;
+    uint32_t copied2[2] = {0u, 0u};  // by the sample's measuring workgroup
+    const uint32_t side_mask = sh.split == 2u ? 1u : 0u;
     // Device-memory loads are issued before this wave's agent-scope stores
     // and used after them only once other work has passed: a wave's wait
     // for a load also waits for every store it issued before the load's use.
@@ -727,7 +728,10 @@ __device__ void strip_body_halo(const StripArgs &a, uint32_t *lds)
         // with split, slot it mod kStripSnapSlots is free once sample
         // it - kStripSnapSlots has been copied
         const uint32_t need = it >= kStripSnapSlots ? it - kStripSnapSlots + 1u : 0u;
-        const uint32_t copied_now = sh.split && copied < need ? ld_relaxed(snapc) : copied;
+        const uint32_t side = it & side_mask;
+        const uint32_t *snapc_it = snapc + side * nwg * kStripFlagStride;
+        const uint32_t copied = side ? copied2[1] : copied2[0];
+        const uint32_t copied_now = sh.split && copied < need ? ld_relaxed(snapc_it) : copied;
         if (has0) cb0[row0 + q] ^= strip_flip(cb0, cb1, row0, q, wpr, ya, 0u, acc, k0, k1, t, p0, p0r);
         if (pub && get_f) {
             if ((uint32_t)(vf >> 32) != it - 1u) {
@@ -776,11 +780,13 @@ __device__ void strip_body_halo(const StripArgs &a, uint32_t *lds)
         // barrier.
         uint64_t *dst = nullptr;
         if (sh.split) {
-            copied = copied_now;
-            if (copied < need) {
-                copied = flag_wait(snapc, need, err) ? need : 0u;
-                bad = copied < need;
+            uint32_t seen = copied_now;
+            if (seen < need) {
+                seen = flag_wait(snapc_it, need, err) ? need : 0u;
+                bad = seen < need;
             }
+            if (side) copied2[1] = seen;
+            else copied2[0] = seen;
             if (!bad) {
                 dst = snap + ((size_t)(it % kStripSnapSlots) * nwg + w) * sh.snap_words;
                 if (has1) ll_put(dst + jw, cb0[row1 + q], seq);
@@ -862,27 +868,33 @@ __device__ bool ll_gather(uint32_t n, uint32_t seq, uint32_t *err, uint32_t slee
     return bad;
 }
 
-// The measuring workgroup n_wg + w of a split launch: strip w's samples, one
-// per sweep, from the copies the strip publishes (rows y0-1 .. y0+R of both
-// colours, into local rows 1 .. R+2 of the halo layout).  Per sample k: the
-// tie coins while the copy arrives; the copy, then its slot released to the
-// strip; the publication of sample k-1 (the lower measuring workgroup's first
-// blocked rows of it were sent one sample ago); the measurement of k and its
-// first blocked rows to the upper measuring workgroup.
+// A measuring workgroup n_wg + i n_wg + w of a split launch: samples i, i +
+// split, ... of strip w, from the copies the strip publishes (rows y0-1 .. y0+R
+// of both colours, into local rows 1 .. R+2 of the halo layout).  Per sample k:
+// the tie coins while the copy arrives; the copy, then its slot released to the
+// strip; the publication of sample k - split (the lower measuring workgroup's
+// first blocked rows of it were sent when that one measured it); the
+// measurement of k and its first blocked rows to the upper measuring workgroup.
+// The first rows of sample k are read before this workgroup releases the copy
+// of k + split.  Until then strip w waits at sweep k + split + kStripSnapSlots
+// at the latest, and its neighbours at most one further, so the lower one has
+// not published sample k + kStripFirstSlotsSplit, whose first rows take the same
+// slot (2 + 4 + 1 < 8).
 template <int NT>
 __device__ void strip_body_meas(const StripArgs &a, uint32_t *lds)
 {
     const StripShape &sh = a.sh;
     const HbmLattice &lat = *a.lat;
-    const uint32_t R = sh.R, wpr = sh.wpr, nwg = sh.n_wg;
-    const uint32_t w = blockIdx.x - nwg, dn = (w + 1u) & (nwg - 1u);
+    const uint32_t wpr = sh.wpr, nwg = sh.n_wg;
+    const uint32_t mine = blockIdx.x - nwg, step = sh.split, i0 = mine / nwg;
+    const uint32_t w = mine - i0 * nwg, dn = (w + 1u) & (nwg - 1u);
     const StripLds m = strip_lds(sh, lds, w);
     const uint32_t cbs = m.cbs, fw = sh.first_words, fs = sh.first_slots, n = a.n_sweeps;
     const uint32_t half = sh.snap_words >> 1;
     uint32_t *err = a.ws + sh.o_err;
     uint64_t *xfirst = reinterpret_cast<uint64_t *>(a.ws + sh.o_xfirst);
     const uint64_t *snap = reinterpret_cast<const uint64_t *>(a.ws + sh.o_snap);
-    uint32_t *snapc = a.ws + sh.o_snapc + w * kStripFlagStride;
+    uint32_t *snapc = a.ws + sh.o_snapc + mine * kStripFlagStride;
     for (uint32_t i = threadIdx.x; i < kStripRing; i += NT) m.red[i] = 0u;  // consumed counts seen
     for (uint32_t i = threadIdx.x; i < kStripCntWords; i += NT) m.pend[i] = 0u;
     if (threadIdx.x == 0) m.red[kRedAny] = 0u;
@@ -891,10 +903,11 @@ __device__ void strip_body_meas(const StripArgs &a, uint32_t *lds)
     const bool get_f = jw < fw;
     bool ok = true;
     uint32_t vote = 0;
-    for (uint32_t k = 0; k < n && ok; ++k) {
-        // loads first: sample k-1's first rows from below, sample k's copy
-        const uint64_t *src_f = xfirst + ((size_t)((k + fs - 1u) % fs) * nwg + dn) * fw + jw;
-        uint64_t vf = k >= 1u && get_f ? ll_peek(src_f) : 0ull;
+    uint32_t last = 0xFFFFFFFFu;
+    for (uint32_t k = i0; k < n && ok; k += step) {
+        // loads first: sample k - step's first rows from below, sample k's copy
+        const uint64_t *src_f = xfirst + ((size_t)((k + fs - step) % fs) * nwg + dn) * fw + jw;
+        uint64_t vf = k >= step && get_f ? ll_peek(src_f) : 0ull;
         const uint64_t *slot = snap + ((size_t)(k % kStripSnapSlots) * nwg + w) * sh.snap_words;
         if (sh.lam > 0u) strip_coins<NT>(a, m, a.t0 + k, k0, k1);
         bool bad = ll_gather<NT>(
@@ -903,10 +916,11 @@ __device__ void strip_body_meas(const StripArgs &a, uint32_t *lds)
                 const uint32_t c = i >= half ? 1u : 0u;
                 m.cb0[c * cbs + wpr + (i - c * half)] = v;
             });
-        if (k >= 1u && get_f) {
-            if ((uint32_t)(vf >> 32) != k) {
-                vf = ll_wait(src_f, k, err, a.strip_sleep);
-                if ((uint32_t)(vf >> 32) != k) bad = true;
+        if (k >= step && get_f) {
+            const uint32_t seq = k - step + 1u;
+            if ((uint32_t)(vf >> 32) != seq) {
+                vf = ll_wait(src_f, seq, err, a.strip_sleep);
+                if ((uint32_t)(vf >> 32) != seq) bad = true;
             }
             m.dfirst[jw] = (uint32_t)vf;
         }
@@ -917,17 +931,18 @@ __device__ void strip_body_meas(const StripArgs &a, uint32_t *lds)
         // every thread's copy of the slot is in LDS: the strip may reuse it
         if (threadIdx.x == 0)
             __hip_atomic_store(snapc, k + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (k >= 1u && !(ok = strip_publish<NT>(a, m, k - 1u))) break;
+        if (k >= step && !(ok = strip_publish<NT>(a, m, k - step))) break;
+        last = k;
         strip_measure<NT>(a, m, m.cb0 + wpr);
         for (uint32_t i = threadIdx.x; i < fw; i += NT)
             ll_put(xfirst + ((size_t)(k % fs) * nwg + w) * fw + i, m.frow[i], k + 1u);
     }
-    if (!ok || n == 0u) return;
+    if (!ok || last == 0xFFFFFFFFu) return;
     // the last sample: its first rows from below, then its publication
     bool bad = false;
     if (get_f)
-        m.dfirst[jw] = ll_get(xfirst + ((size_t)((n - 1u) % fs) * nwg + dn) * fw + jw, n, err, bad, a.strip_sleep);
-    if (!strip_any(bad, m.red + kRedAny, ++vote)) (void)strip_publish<NT>(a, m, n - 1u);
+        m.dfirst[jw] = ll_get(xfirst + ((size_t)(last % fs) * nwg + dn) * fw + jw, last + 1u, err, bad, a.strip_sleep);
+    if (!strip_any(bad, m.red + kRedAny, ++vote)) (void)strip_publish<NT>(a, m, last);
 }
 
 // A tail workgroup: samples q = tail, tail + n_tail, ...  For each, once every
@@ -1019,7 +1034,12 @@ __global__ __launch_bounds__(NT) void k_strip(StripArgs a)
     extern __shared__ uint32_t lds[];
     if (blockIdx.x >= a.sh.n_wg + a.sh.n_meas) tail_body<NT>(a, lds);
     else if (blockIdx.x >= a.sh.n_wg) strip_body_meas<NT>(a, lds);
-    else if (a.sh.halo) strip_body_halo<NT>(a, lds);
+    else if (a.sh.halo) {
+        // the sweeps are the longest chain: their waves issue before those of
+        // the measuring workgroups on the same SIMD (1 %)
+        __builtin_amdgcn_s_setprio(3);
+        strip_body_halo<NT>(a, lds);
+    }
     else strip_body<NT>(a, lds);
 }
 

@@ -73,12 +73,14 @@ bool StripRunner::plan(const HbmLattice &h, bool measure, StripShape &sh, int &t
     }
     if (n_wg > L / 2u) n_wg = L / 2u;
     if (n_wg < 2u) return false;
-    // tail workgroups: 4 (fewer when they do not fit beside the strips);
-    // MCRG_STRIP_TAILS = 1, 2 or 4 asks for that many
-    uint32_t want = 4u;
+    // tail workgroups: 8, one per ring slot (fewer when they do not fit beside
+    // the strips); a measured L = 512 sweep, whose tails work off every level
+    // from side 256 on with 64 threads, takes 6.2 us with 4 and 3.5 with 8;
+    // MCRG_STRIP_TAILS = 1, 2, 4 or 8 asks for that many
+    uint32_t want = 8u;
     if (const char *v = std::getenv("MCRG_STRIP_TAILS")) {
         const int n = std::atoi(v);
-        if (n == 1 || n == 2 || n == 4) want = (uint32_t)n;
+        if (n == 1 || n == 2 || n == 4 || n == 8) want = (uint32_t)n;
     }
     // MCRG_STRIP_HALO=0 keeps two exchanges per sweep where halo rows would
     // fit; MCRG_STRIP_SPLIT=0 keeps a halo strip's measurements in its own
@@ -87,11 +89,12 @@ bool StripRunner::plan(const HbmLattice &h, bool measure, StripShape &sh, int &t
     const bool halo_ok = !(hv && std::atoi(hv) == 0);
     const char *sv = std::getenv("MCRG_STRIP_SPLIT");
     const bool split_ok = !(sv && std::atoi(sv) == 0);
-    for (uint32_t n_tail : {4u, 2u, 1u}) {
+    for (uint32_t n_tail : {8u, 4u, 2u, 1u}) {
         if (n_tail > want) continue;
         // measuring workgroups when they fit (resident and within max_words)
-        for (int sp = split_ok ? 1 : 0; sp >= 0; --sp) {
-            sh = strip_shape(L, (uint32_t)h.n_levels, n_wg, n_tail, measure, halo_ok, sp != 0);
+        for (int sp = split_ok ? 2 : 0; sp >= 0; --sp) {
+            sh = strip_shape(L, (uint32_t)h.n_levels, n_wg, n_tail, measure, halo_ok, sp != 0,
+                             (uint32_t)std::max(sp, 1));
             if (sp && !sh.split) continue;
             threads = strip_threads(sh);
             // every thread gets at most one neighbour word of each kind per exchange
