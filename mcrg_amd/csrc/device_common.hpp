@@ -142,24 +142,38 @@ __device__ __forceinline__ MetropolisStage metropolis_first(uint32_t s, uint32_t
     return st;
 }
 
-__device__ __forceinline__ uint32_t metropolis_second(MetropolisStage st, uint32_t valid, const Accept &acc,
-                                                      uint32_t k0, uint32_t k1, uint32_t word, uint32_t t,
-                                                      uint32_t colour, u32x4 ref)
+// The first four ranks of the open sites.
+__device__ __forceinline__ void metropolis_ranks(MetropolisStage &st, const Accept &acc, const u32x4 &ref)
 {
     const uint32_t low0 = acc.thr0 << 4, low1 = acc.thr1 << 4;
     metropolis_refine(st.open, st.accept, st.m1, ref.v0, low0, low1);
     metropolis_refine(st.open, st.accept, st.m1, ref.v1, low0, low1);
     metropolis_refine(st.open, st.accept, st.m1, ref.v2, low0, low1);
     metropolis_refine(st.open, st.accept, st.m1, ref.v3, low0, low1);
-    for (uint32_t call = 2; st.open != 0u; ++call) {
-        ref = philox(word, t, call, (kTagSweep << 28) | (colour << 24), k0, k1);
-        metropolis_refine(st.open, st.accept, st.m1, ref.v0, low0, low1);
-        if (st.open != 0u) {
-            metropolis_refine(st.open, st.accept, st.m1, ref.v1, low0, low1);
-            metropolis_refine(st.open, st.accept, st.m1, ref.v2, low0, low1);
-            metropolis_refine(st.open, st.accept, st.m1, ref.v3, low0, low1);
+}
+
+// The ranks from the fifth on.
+__device__ __forceinline__ void metropolis_rest(uint32_t &open, uint32_t &accept, uint32_t m1, const Accept &acc,
+                                                uint32_t k0, uint32_t k1, uint32_t word, uint32_t t, uint32_t colour)
+{
+    const uint32_t low0 = acc.thr0 << 4, low1 = acc.thr1 << 4;
+    for (uint32_t call = 2; open != 0u; ++call) {
+        const u32x4 ref = philox(word, t, call, (kTagSweep << 28) | (colour << 24), k0, k1);
+        metropolis_refine(open, accept, m1, ref.v0, low0, low1);
+        if (open != 0u) {
+            metropolis_refine(open, accept, m1, ref.v1, low0, low1);
+            metropolis_refine(open, accept, m1, ref.v2, low0, low1);
+            metropolis_refine(open, accept, m1, ref.v3, low0, low1);
         }
     }
+}
+
+__device__ __forceinline__ uint32_t metropolis_second(MetropolisStage st, uint32_t valid, const Accept &acc,
+                                                      uint32_t k0, uint32_t k1, uint32_t word, uint32_t t,
+                                                      uint32_t colour, const u32x4 &ref)
+{
+    metropolis_ranks(st, acc, ref);
+    metropolis_rest(st.open, st.accept, st.m1, acc, k0, k1, word, t, colour);
     return (st.flip | st.accept) & valid;
 }
 
@@ -181,6 +195,57 @@ __device__ __forceinline__ uint32_t metropolis_word(uint32_t s, uint32_t nu, uin
     const MetropolisStage st =
         metropolis_first(s, nu, nd, nl, nr, valid, acc, philox(word, t, 0u, tag, k0, k1));
     return metropolis_second(st, valid, acc, k0, k1, word, t, colour, philox(word, t, 1u, tag, k0, k1));
+}
+
+// The decisions of K words of one colour a lane, f[k] the bits to flip: at(k)
+// gives word k's index, its spins and its neighbours' (MetropolisSites).  A
+// fifth open site is rare in a lane but common in a wave, so a word at a time
+// nearly every wave draws a third Philox call for one or two lanes.  Here the
+// words' rests wait for each other: a call then serves each lane's first word
+// that needs one.  At K = 4, J = 0.44: strips of L = 16384 62.6 -> 59.4 us a
+// sweep, L = 8192 17.3 -> 16.5; 4096 uneven lattices of 8..128, one wave each,
+// 81 -> 73 ms for their 11000 sweeps.
+struct MetropolisSites {
+    uint32_t word, s, nu, nd, nl, nr;
+};
+// APART keeps the compiler from working on several words at once (registers).
+template <uint32_t K, bool APART, typename At>
+__device__ __forceinline__ void metropolis_words(uint32_t (&f)[K], const Accept &acc, uint32_t k0, uint32_t k1,
+                                                 uint32_t t, uint32_t colour, At at)
+{
+    const uint32_t tag = (kTagSweep << 28) | (colour << 24);
+    uint32_t open[K], m1[K], word[K];
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k) {
+        const MetropolisSites x = at(k);
+        word[k] = x.word;
+        MetropolisStage st = metropolis_first(x.s, x.nu, x.nd, x.nl, x.nr, 0xFFFFFFFFu, acc,
+                                              philox(x.word, t, 0u, tag, k0, k1));
+        metropolis_ranks(st, acc, philox(x.word, t, 1u, tag, k0, k1));
+        f[k] = st.flip | st.accept;
+        open[k] = st.open;
+        m1[k] = st.m1;
+        if (APART) __builtin_amdgcn_sched_barrier(0);
+    }
+    for (;;) {
+        uint32_t o = 0, m = 0, w = 0;
+        for (uint32_t k = 0; k < K; ++k) {
+            const bool has = o == 0u;
+            o = has ? open[k] : o;
+            m = has ? m1[k] : m;
+            w = has ? word[k] : w;
+        }
+        if (o == 0u) break;
+        uint32_t accept = 0;
+        metropolis_rest(o, accept, m, acc, k0, k1, w, t, colour);
+        bool mine = true;  // the first word with open sites
+        for (uint32_t k = 0; k < K; ++k) {
+            const bool take = mine && open[k] != 0u;
+            f[k] |= take ? accept : 0u;
+            open[k] = take ? 0u : open[k];
+            mine = mine && !take;
+        }
+    }
 }
 
 // Spin bits of the 32 bytes at even (p = 0) or odd (p = 1) positions of a 64-byte

@@ -515,7 +515,23 @@ __device__ void strip_body(const StripArgs &a, uint32_t *lds)
         for (uint32_t c = 0; c < 2u && ok; ++c) {
             uint32_t *own = cb0 + c * cbs;
             const uint32_t *oth = cb0 + (c ^ 1u) * cbs;
-            for (uint32_t j = threadIdx.x; j < R * wpr; j += NT) {
+            // Four words a thread at once where there are as many.  Workgroups of
+            // 256 threads hardly ever have them and were 3% slower with this
+            // loop in their code (L = 2048: 3.17 -> 3.28 us a sweep).
+            uint32_t jw4 = threadIdx.x;
+            for (; NT >= 512 && jw4 + 3u * NT < R * wpr; jw4 += 4u * NT) {
+                uint32_t f[4];
+                metropolis_words<4u, true>(f, acc, k0, k1, t, c, [&](uint32_t k) {
+                    const uint32_t jk = jw4 + k * NT, r = 1u + (jk >> sw), q = jk & mk, y = y0 + r - 1u, row = r << sw;
+                    const uint32_t p = (y + c) & 1u;
+                    const uint32_t o = oth[row + q], os = oth[row + ((q + 2u * p - 1u) & mk)];
+                    return MetropolisSites{y * wpr + q, own[row + q], oth[row - wpr + q], oth[row + wpr + q],
+                                           p == 0u ? (o << 1) | (os >> 31) : o, p == 0u ? o : (o >> 1) | (os << 31)};
+                });
+#pragma unroll
+                for (uint32_t k = 0; k < 4u; ++k) own[wpr + jw4 + k * NT] ^= f[k];
+            }
+            for (uint32_t j = jw4; j < R * wpr; j += NT) {
                 const uint32_t r = 1u + (j >> sw), q = j & mk, y = y0 + r - 1u, row = r << sw;
                 // o and the word beside it that holds the wrap-around site
                 // (q - 1 on p = 0 rows, q + 1 on p = 1 rows): one load each

@@ -63,17 +63,15 @@ __device__ __forceinline__ void wave_half(uint32_t (&own)[WaveGeom<L>::WPL], con
                                   acc, k0, k1, l, t, c);
     } else {
         const uint32_t up[2] = {wave_prev(oth[2]), wave_prev(oth[3])}, dn[2] = {wave_next(oth[0]), wave_next(oth[1])};
+        uint32_t f[4];
+        metropolis_words<4u, false>(f, acc, k0, k1, t, c, [&](uint32_t k) {
+            const uint32_t a = k >> 1, q = k & 1u, o = oth[k], side = oth[k ^ 1u];
+            const bool p = ((a + c) & 1u) != 0u;
+            return MetropolisSites{4u * l + k, own[k], a ? oth[q] : up[q], a ? dn[q] : oth[2u + q],
+                                   row_left(o, side, p), row_right(o, side, p)};
+        });
 #pragma unroll
-        for (uint32_t a = 0; a < 2u; ++a) {
-#pragma unroll
-            for (uint32_t q = 0; q < 2u; ++q) {
-                const uint32_t o = oth[2u * a + q], side = oth[2u * a + (q ^ 1u)];
-                const bool p = ((a + c) & 1u) != 0u;
-                const uint32_t k = 2u * a + q;
-                own[k] ^= metropolis_word(own[k], a ? oth[q] : up[q], a ? dn[q] : oth[2u + q], row_left(o, side, p),
-                                          row_right(o, side, p), 0xFFFFFFFFu, acc, k0, k1, 4u * l + k, t, c);
-            }
-        }
+        for (uint32_t k = 0; k < 4u; ++k) own[k] ^= f[k];
     }
 }
 
@@ -109,6 +107,44 @@ __device__ __forceinline__ uint32_t majority(uint32_t b1, uint32_t b2, uint32_t 
     return maj3 | (tie & coin);
 }
 
+// A level of 32 rows of 32 sites, row l / 2 in each even lane: its counts to
+// cnt[0..1] and, when the sample is blocked further, the 16 rows of level
+// lv + 1 to w16 (8 words).  coin(call, level) draws four tie-coin words.
+template <typename Coin>
+__device__ __forceinline__ void rows32(uint32_t row, uint32_t lv, uint32_t nl, Coin coin, uint32_t *cnt, uint32_t *w16)
+{
+    const uint32_t l = threadIdx.x & 63u;
+    const uint32_t d = wave_next(wave_next(row)), r = (row >> 1) | (row << 31), g = (d >> 1) | (d << 31);
+    const uint32_t on = (l & 1u) ? 0u : 0xFFFFFFFFu;
+    put_counts(cnt, (uint32_t)(popc((row ^ r) & on) + popc((row ^ d) & on)),
+               (uint32_t)(popc((row ^ g) & on) + popc((r ^ d) & on)), (uint32_t)popc((xor3(row, r, d) ^ g) & on), 0u);
+    if (nl == lv) return;
+    // row l / 4 at every fourth lane, coin word l / 8
+    const u32x4 x = coin(l >> 5, lv);
+    const uint32_t b16 = block16(row, d, (pick4(x, (l >> 3) & 3u) >> (16u * ((l >> 2) & 1u))) & 0xFFFFu);
+    if ((l & 3u) == 0u) reinterpret_cast<uint16_t *>(w16)[l >> 2] = (uint16_t)b16;
+}
+
+// A level of 64 rows of 64 sites, row l (lo, hi) in each lane: its counts to
+// cnt[0..1], then as rows32 with the counts of level lv + 1 to cnt[2..3].
+template <typename Coin>
+__device__ __forceinline__ void rows64(uint32_t lo, uint32_t hi, uint32_t lv, uint32_t nl, Coin coin, uint32_t *cnt,
+                                       uint32_t *w16)
+{
+    const uint32_t l = threadIdx.x & 63u;
+    const uint32_t dlo = wave_next(lo), dhi = wave_next(hi);
+    const uint32_t rlo = (lo >> 1) | (hi << 31), rhi = (hi >> 1) | (lo << 31);
+    const uint32_t glo = (dlo >> 1) | (dhi << 31), ghi = (dhi >> 1) | (dlo << 31);
+    put_counts(cnt, (uint32_t)(popc(lo ^ rlo) + popc(hi ^ rhi) + popc(lo ^ dlo) + popc(hi ^ dhi)),
+               (uint32_t)(popc(lo ^ glo) + popc(hi ^ ghi) + popc(rlo ^ dlo) + popc(rhi ^ dhi)),
+               (uint32_t)(popc(xor3(lo, rlo, dlo) ^ glo) + popc(xor3(hi, rhi, dhi) ^ ghi)), 0u);
+    if (nl == lv) return;
+    // rows l / 2 at the even lanes: coin word l / 2
+    const u32x4 x = coin(l >> 3, lv);
+    const uint32_t cw = pick4(x, (l >> 1) & 3u);
+    rows32(block16(lo, dlo, cw & 0xFFFFu) | (block16(hi, dhi, cw >> 16) << 16), lv + 1u, nl, coin, cnt + 2, w16);
+}
+
 // The sample's first step: counts of the front levels and the side-16 level
 // into out (WaveGeom<L>::stride words).
 template <uint32_t L>
@@ -116,7 +152,7 @@ __device__ __forceinline__ void wave_sample(const uint32_t (&c0)[WaveGeom<L>::WP
                                             uint32_t nl, uint32_t t, uint32_t k0, uint32_t k1, uint32_t *out)
 {
     const uint32_t l = threadIdx.x & 63u;
-    uint32_t dnn = 0, dnnn = 0, dp = 0, down = 0, row = 0;  // row: 32 x 32 level, row l / 2 at even lanes
+    uint32_t dnn = 0, dnnn = 0, dp = 0, down = 0;
     auto coin = [&](uint32_t call, uint32_t level) {
         return philox(call, t, 0u, (kTagTie << 28) | (level << 16), k0, k1);
     };
@@ -129,7 +165,7 @@ __device__ __forceinline__ void wave_sample(const uint32_t (&c0)[WaveGeom<L>::WP
         if (nl == 0u) return;
         // coin word by = l / 2 of level 0
         const u32x4 x = coin(l >> 3, 0u);
-        row = majority(a, b, an, bn, pick4(x, (l >> 1) & 3u));
+        rows32(majority(a, b, an, bn, pick4(x, (l >> 1) & 3u)), 1u, nl, coin, out + 2, out + 2u * WaveGeom<L>::front);
     } else {
         uint32_t n0[2], n1[2];
 #pragma unroll
@@ -152,33 +188,12 @@ __device__ __forceinline__ void wave_sample(const uint32_t (&c0)[WaveGeom<L>::WP
         }
         put_counts(out, dnn, dnnn, dp, down);
         if (nl == 0u) return;
-        // ---- level 1: 64 rows of 64 sites, row l; coin words 2l, 2l + 1
-        u32x4 x = coin(l >> 1, 0u);
-        const uint32_t lo = majority(c0[0], c1[0], c0[2], c1[2], (l & 1u) ? x.v2 : x.v0);
-        const uint32_t hi = majority(c0[1], c1[1], c0[3], c1[3], (l & 1u) ? x.v3 : x.v1);
-        const uint32_t dlo = wave_next(lo), dhi = wave_next(hi);
-        const uint32_t rlo = (lo >> 1) | (hi << 31), rhi = (hi >> 1) | (lo << 31);
-        const uint32_t glo = (dlo >> 1) | (dhi << 31), ghi = (dhi >> 1) | (dlo << 31);
-        put_counts(out + 2, (uint32_t)(popc(lo ^ rlo) + popc(hi ^ rhi) + popc(lo ^ dlo) + popc(hi ^ dhi)),
-                   (uint32_t)(popc(lo ^ glo) + popc(hi ^ ghi) + popc(rlo ^ dlo) + popc(rhi ^ dhi)),
-                   (uint32_t)(popc(xor3(lo, rlo, dlo) ^ glo) + popc(xor3(hi, rhi, dhi) ^ ghi)), 0u);
-        if (nl == 1u) return;
-        // ---- level 2 at the even lanes: coin word l / 2
-        x = coin(l >> 3, 1u);
-        const uint32_t cw = pick4(x, (l >> 1) & 3u);
-        row = block16(lo, dlo, cw & 0xFFFFu) | (block16(hi, dhi, cw >> 16) << 16);
+        // level 1: 64 rows of 64 sites, row l; coin words 2l, 2l + 1
+        const u32x4 x = coin(l >> 1, 0u);
+        rows64(majority(c0[0], c1[0], c0[2], c1[2], (l & 1u) ? x.v2 : x.v0),
+               majority(c0[1], c1[1], c0[3], c1[3], (l & 1u) ? x.v3 : x.v1), 1u, nl, coin, out + 2,
+               out + 2u * WaveGeom<L>::front);
     }
-    // ---- 32 rows of 32 sites at the even lanes
-    constexpr uint32_t lv = WaveGeom<L>::front - 1u;
-    const uint32_t d = wave_next(wave_next(row)), r = (row >> 1) | (row << 31), g = (d >> 1) | (d << 31);
-    const uint32_t on = (l & 1u) ? 0u : 0xFFFFFFFFu;
-    put_counts(out + 2u * lv, (uint32_t)(popc((row ^ r) & on) + popc((row ^ d) & on)),
-               (uint32_t)(popc((row ^ g) & on) + popc((r ^ d) & on)), (uint32_t)popc((xor3(row, r, d) ^ g) & on), 0u);
-    if (nl == lv) return;
-    // ---- 16 rows of 16 sites at every fourth lane: row l / 4, coin word l / 8
-    const u32x4 x = coin(l >> 5, lv);
-    const uint32_t b16 = block16(row, d, (pick4(x, (l >> 3) & 3u) >> (16u * ((l >> 2) & 1u))) & 0xFFFFu);
-    if ((l & 3u) == 0u) reinterpret_cast<uint16_t *>(out + 2u * WaveGeom<L>::front)[l >> 2] = (uint16_t)b16;
 }
 
 // Adds the samples with `take` to the partial record; the terms are at most
