@@ -197,8 +197,8 @@ __device__ __forceinline__ uint32_t metropolis_word(uint32_t s, uint32_t nu, uin
     return metropolis_second(st, valid, acc, k0, k1, word, t, colour, philox(word, t, 1u, tag, k0, k1));
 }
 
-// The decisions of K words of one colour a lane, f[k] the bits to flip: at(k)
-// gives word k's index, its spins and its neighbours' (MetropolisSites).  A
+// The decisions of K words of one colour a lane, f[k] the bits to flip of
+// word word0 + k * STEP; at(k) gives its spins and its neighbours' (MetropolisSites).  A
 // fifth open site is rare in a lane but common in a wave, so a word at a time
 // nearly every wave draws a third Philox call for one or two lanes.  Here the
 // words' rests wait for each other: a call then serves each lane's first word
@@ -206,22 +206,22 @@ __device__ __forceinline__ uint32_t metropolis_word(uint32_t s, uint32_t nu, uin
 // sweep, L = 8192 17.3 -> 16.5; 4096 uneven lattices of 8..128, one wave each,
 // 81 -> 73 ms for their 11000 sweeps.
 struct MetropolisSites {
-    uint32_t word, s, nu, nd, nl, nr;
+    uint32_t s, nu, nd, nl, nr;
 };
 // APART keeps the compiler from working on several words at once (registers).
-template <uint32_t K, bool APART, typename At>
+template <uint32_t K, uint32_t STEP, bool APART, typename At>
 __device__ __forceinline__ void metropolis_words(uint32_t (&f)[K], const Accept &acc, uint32_t k0, uint32_t k1,
-                                                 uint32_t t, uint32_t colour, At at)
+                                                 uint32_t t, uint32_t colour, uint32_t word0, At at)
 {
     const uint32_t tag = (kTagSweep << 28) | (colour << 24);
-    uint32_t open[K], m1[K], word[K];
+    uint32_t open[K], m1[K];
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k) {
         const MetropolisSites x = at(k);
-        word[k] = x.word;
+        const uint32_t word = word0 + k * STEP;
         MetropolisStage st = metropolis_first(x.s, x.nu, x.nd, x.nl, x.nr, 0xFFFFFFFFu, acc,
-                                              philox(x.word, t, 0u, tag, k0, k1));
-        metropolis_ranks(st, acc, philox(x.word, t, 1u, tag, k0, k1));
+                                              philox(word, t, 0u, tag, k0, k1));
+        metropolis_ranks(st, acc, philox(word, t, 1u, tag, k0, k1));
         f[k] = st.flip | st.accept;
         open[k] = st.open;
         m1[k] = st.m1;
@@ -233,7 +233,7 @@ __device__ __forceinline__ void metropolis_words(uint32_t (&f)[K], const Accept 
             const bool has = o == 0u;
             o = has ? open[k] : o;
             m = has ? m1[k] : m;
-            w = has ? word[k] : w;
+            w = has ? word0 + k * STEP : w;
         }
         if (o == 0u) break;
         uint32_t accept = 0;

@@ -5,7 +5,7 @@
 #include <cstring>
 
 #include "runtime.hpp"
-#include "wave_core.hpp"
+#include "resident_body.hpp"
 
 namespace mcrg {
 
@@ -201,7 +201,7 @@ size_t ResidentEngine::job_bytes(const JobSpec &j)
 uint32_t ResidentEngine::lds_bytes(int L, int G, int nl, int NT) const
 {
     const uint32_t T = (uint32_t)NT / (uint32_t)G;
-    return slot_layout((uint32_t)L, (uint32_t)G, (uint32_t)nl, T).total * 4u;
+    return slot_words((uint32_t)L, (uint32_t)G, (uint32_t)nl, T) * 4u;
 }
 
 void ResidentEngine::enable_autotune()
@@ -420,10 +420,10 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
         const int L = kv.first.L, nl = kv.first.nl;
         const std::vector<int> &ids = kv.second;
         const bool small = L <= kWaveMaxL;
-        const int G = L <= kSmallMaxL ? small_group(L, (int)ids.size(), alone) : small ? 1 : group_size(L, nl, threads_for(L));
+        const int G = L <= kSmallMaxL ? small_group(L, (int)ids.size(), alone) : 1;
         for (size_t a = 0; a < ids.size(); a += (size_t)G) {
             const int g = (int)std::min<size_t>((size_t)G, ids.size() - a);
-            // positions: a power of two (so that teams tile the workgroup), empty ones are -1
+            // positions: a power of two (so that teams tile the wave), empty ones are -1
             int gp = 1;
             while (gp < g) gp *= 2;
             const uint32_t ns = slot_sweeps(L, gp, chunk);
@@ -445,7 +445,7 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
                                                       : wave_lds_words((uint32_t)L, (uint32_t)nl)),
                                 64, true});
             else
-                pend.push_back({s, work, lds_bytes(L, gp, nl, threads_for(L)), threads_for(L), false});
+                pend.push_back({s, work, 4u * big_layout((uint32_t)L, (uint32_t)nl).total, threads_for(L), false});
         }
     }
     // launch classes by (workgroup size, workgroups resident on the device):

@@ -1,7 +1,8 @@
-// LDS-resident schedule: bit-packed (CB) lattices held in LDS by a workgroup
-// for a whole chunk of sweeps.  A "slot" is G lattices of one side L and one
-// level count that a workgroup advances together; a persistent grid pulls
-// slots from a queue.  Shared by the host engine and the kernels.
+// Resident schedule: bit-packed (CB) lattices held in a wave's registers (L <=
+// 128) or a workgroup's LDS (L = 256, 512) for a whole chunk of sweeps.  A
+// "slot" is G lattices of one side L and one level count that a wave advances
+// together, or one lattice of a workgroup; a persistent grid of workgroups
+// pulls those from a queue.  Shared by the host engine and the kernels.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -46,64 +47,17 @@ __host__ __device__ inline uint32_t level_words(uint32_t L, uint32_t l)
     return w ? w : 1u;
 }
 
-// LDS layout of one slot, offsets in 32-bit words.  T = threads per lattice.
-struct SlotLayout {
-    uint32_t W;           // CB words per colour
-    uint32_t lvl_words;   // RM words of levels 1..nl, per lattice (also the coin words)
-    uint32_t team_waves;  // waves per lattice team (count partials per level)
-    uint32_t n_sv;        // operator values per lattice: 3 (nl+1) + M, |M|, 1
-    uint32_t coin_calls;  // Philox calls for all tie-coin words (4 words per call)
-    uint32_t meta, spins, lvl, coin, cnt, sv, pairs, rec, total;
-};
-
-__host__ __device__ inline SlotLayout slot_layout(uint32_t L, uint32_t G, uint32_t nl, uint32_t T)
+// LDS words that admission counts for G lattices of one slot, T = threads per
+// lattice: spins, blocked levels and their tie coins, counts, operator values
+// and records.  What a launch takes is big_layout() (up to 1.6 k words more: 64
+// samples wait there), small_lds_words() or wave_lds_words().
+__host__ __device__ inline uint32_t slot_words(uint32_t L, uint32_t G, uint32_t nl, uint32_t T)
 {
-    SlotLayout s;
-    s.W = cb_words(L);
-    s.lvl_words = 0;
-    s.coin_calls = 0;
-    for (uint32_t l = 1; l <= nl; ++l) {
-        s.lvl_words += level_words(L, l);
-        s.coin_calls += (level_words(L, l) + 3u) / 4u;
-    }
-    s.team_waves = T > 64u ? T / 64u : 1u;
-    s.meta = 0;
-    s.spins = s.meta + G * kMetaWords;
-    s.lvl = s.spins + G * 2u * s.W;
-    s.coin = s.lvl + G * s.lvl_words;
-    s.cnt = s.coin + G * s.lvl_words;
-    s.n_sv = 3u * (nl + 1u) + 3u;
-    s.sv = s.cnt + G * s.team_waves * (nl + 1u) * 4u;  // int32 operator values (teams within one wave)
-    s.pairs = s.sv + G * s.n_sv;                         // one (x, y) operand pair per record entry
-    s.rec = (s.pairs + record_size(nl) + 1u) & ~1u;  // int64 aligned
-    s.total = s.rec + G * record_size(nl) * 2u;
-    return s;
-}
-
-// First blocked level whose rows fit one per lane of a team of T lanes (at
-// most one wave), or 0 when no level from 1 to nl does: the levels from it on
-// are measured in registers (the "pyramid").
-__host__ __device__ inline uint32_t pyramid_level(uint32_t L, uint32_t T, uint32_t nl)
-{
-    const uint32_t lanes = T < 64u ? T : 64u;
-    for (uint32_t l = 1; l <= nl; ++l)
-        if ((L >> l) <= lanes) return l;
-    return 0u;
-}
-
-// Slot bodies the resident kernel is compiled with: the wide body for teams of
-// at least a wave on L >= 64, whose register pyramid starts at rows of 64
-// (L >= 128) or 32 sites (L = 64), unrolled for those two shapes and without
-// the small-lattice code paths; the generic body for everything else.
-enum SlotShape : uint32_t { kShapeGeneric = 0, kShapeRows64 = 1, kShapeRows32 = 2 };
-
-__host__ __device__ inline uint32_t slot_shape(uint32_t L, uint32_t G, uint32_t nl, uint32_t NT)
-{
-    const uint32_t T = NT / G;
-    const uint32_t pl = pyramid_level(L, T, nl);
-    if (pl == 0u || T < 64u) return kShapeGeneric;
-    const uint32_t Lp = L >> pl;
-    return Lp == 64u ? kShapeRows64 : Lp == 32u && L >= 64u ? kShapeRows32 : kShapeGeneric;
+    uint32_t lvl = 0;
+    for (uint32_t l = 1; l <= nl; ++l) lvl += level_words(L, l);
+    const uint32_t counts = (T > 64u ? T / 64u : 1u) * (nl + 1u) * 4u, values = 3u * (nl + 1u) + 3u;
+    const uint32_t before = G * (kMetaWords + 2u * cb_words(L) + 2u * lvl + counts + values) + record_size(nl);
+    return ((before + 1u) & ~1u) + G * record_size(nl) * 2u;
 }
 
 // Admits n lattices: lats[idx[k]] = stage[k], its records zeroed, its spins

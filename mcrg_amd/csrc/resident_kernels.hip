@@ -1,19 +1,19 @@
-// LDS-resident schedule kernels (see resident_core.hpp for the phase structure).
+// LDS-resident schedule kernels (see resident_body.hpp for the phase structure).
 //
 //   k_packed_init   admission of bit-packed (CB) lattices: descriptor from a
 //                   staging array into the table, records zeroed, Philox +-1
 //                   start (Lattice::initialize_random_spins, src/lattice.cpp:33-41)
 //   k_resident      persistent grid; each workgroup pulls work items (one part
-//                   of one slot: G lattices of one L) from an atomic queue and
-//                   runs the part's sweeps and measurements with the lattices
-//                   held in LDS; a slot's parts run in order, possibly in
+//                   of one slot: one lattice of L = 256 or 512) from an atomic
+//                   queue and runs the part's sweeps and measurements with the
+//                   lattice held in LDS; a slot's parts run in order, possibly in
 //                   different workgroups (src/ising.cpp:87-149 replaced by
 //                   Metropolis; src/lattice.cpp:102-120, src/mcrg.cpp:72-98 and
 //                   :314-348 fused)
 //   k_reset_queue   zeroes a launch's work counter and per-slot progress words
 #include <mutex>
 
-#include "resident_core.hpp"
+#include "resident_body.hpp"
 
 namespace mcrg {
 
@@ -103,23 +103,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_
             ok = uni<true>(s_ok) != 0u;
         }
         if (ok && sl.n_sweeps > 0u) {
-            Team tm;
-            tm.T = (uint32_t)NT / (uint32_t)sl.G;
-            tm.g0 = threadIdx.x / tm.T;
-            tm.gs = (uint32_t)sl.G;
-            tm.u0 = threadIdx.x % tm.T;
-            tm.us = tm.T;
-            tm.lane = threadIdx.x;
-            tm.block = tm.T > 64u;
-            // Slots of either wide shape run the wide body (slot_shape), the
-            // others the generic body.  Workgroups of 64 and 128 threads keep
-            // the generic body only: with both, their register allocation
-            // spills.
-            if (NT >= 256 && slot_shape((uint32_t)sl.L, (uint32_t)sl.G, (uint32_t)sl.n_levels, (uint32_t)NT) !=
-                                 kShapeGeneric)
-                run_slot<kShapeRows64>(sl, slot_lats, lats, lds, tm);
+            if (sl.L == 512)
+                run_slot<NT, 512u>(sl, slot_lats, lats, lds);
             else
-                run_slot<kShapeGeneric>(sl, slot_lats, lats, lds, tm);
+                run_slot<NT, 256u>(sl, slot_lats, lats, lds);
         }
         if (n_sub > 1u) {
             // this part's write-back (spins, records, counters) goes to the

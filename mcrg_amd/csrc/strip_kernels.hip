@@ -521,11 +521,11 @@ __device__ void strip_body(const StripArgs &a, uint32_t *lds)
             uint32_t jw4 = threadIdx.x;
             for (; NT >= 512 && jw4 + 3u * NT < R * wpr; jw4 += 4u * NT) {
                 uint32_t f[4];
-                metropolis_words<4u, true>(f, acc, k0, k1, t, c, [&](uint32_t k) {
+                metropolis_words<4u, (uint32_t)NT, true>(f, acc, k0, k1, t, c, y0 * wpr + jw4, [&](uint32_t k) {
                     const uint32_t jk = jw4 + k * NT, r = 1u + (jk >> sw), q = jk & mk, y = y0 + r - 1u, row = r << sw;
                     const uint32_t p = (y + c) & 1u;
                     const uint32_t o = oth[row + q], os = oth[row + ((q + 2u * p - 1u) & mk)];
-                    return MetropolisSites{y * wpr + q, own[row + q], oth[row - wpr + q], oth[row + wpr + q],
+                    return MetropolisSites{own[row + q], oth[row - wpr + q], oth[row + wpr + q],
                                            p == 0u ? (o << 1) | (os >> 31) : o, p == 0u ? o : (o >> 1) | (os << 31)};
                 });
 #pragma unroll

@@ -64,10 +64,10 @@ __device__ __forceinline__ void wave_half(uint32_t (&own)[WaveGeom<L>::WPL], con
     } else {
         const uint32_t up[2] = {wave_prev(oth[2]), wave_prev(oth[3])}, dn[2] = {wave_next(oth[0]), wave_next(oth[1])};
         uint32_t f[4];
-        metropolis_words<4u, false>(f, acc, k0, k1, t, c, [&](uint32_t k) {
+        metropolis_words<4u, 1u, false>(f, acc, k0, k1, t, c, 4u * l, [&](uint32_t k) {
             const uint32_t a = k >> 1, q = k & 1u, o = oth[k], side = oth[k ^ 1u];
             const bool p = ((a + c) & 1u) != 0u;
-            return MetropolisSites{4u * l + k, own[k], a ? oth[q] : up[q], a ? dn[q] : oth[2u + q],
+            return MetropolisSites{own[k], a ? oth[q] : up[q], a ? dn[q] : oth[2u + q],
                                    row_left(o, side, p), row_right(o, side, p)};
         });
 #pragma unroll
@@ -113,7 +113,7 @@ __device__ __forceinline__ uint32_t majority(uint32_t b1, uint32_t b2, uint32_t 
 template <typename Coin>
 __device__ __forceinline__ void rows32(uint32_t row, uint32_t lv, uint32_t nl, Coin coin, uint32_t *cnt, uint32_t *w16)
 {
-    const uint32_t l = threadIdx.x & 63u;
+    const uint32_t l = __lane_id();
     const uint32_t d = wave_next(wave_next(row)), r = (row >> 1) | (row << 31), g = (d >> 1) | (d << 31);
     const uint32_t on = (l & 1u) ? 0u : 0xFFFFFFFFu;
     put_counts(cnt, (uint32_t)(popc((row ^ r) & on) + popc((row ^ d) & on)),
@@ -131,7 +131,7 @@ template <typename Coin>
 __device__ __forceinline__ void rows64(uint32_t lo, uint32_t hi, uint32_t lv, uint32_t nl, Coin coin, uint32_t *cnt,
                                        uint32_t *w16)
 {
-    const uint32_t l = threadIdx.x & 63u;
+    const uint32_t l = __lane_id();
     const uint32_t dlo = wave_next(lo), dhi = wave_next(hi);
     const uint32_t rlo = (lo >> 1) | (hi << 31), rhi = (hi >> 1) | (lo << 31);
     const uint32_t glo = (dlo >> 1) | (dhi << 31), ghi = (dhi >> 1) | (dlo << 31);
