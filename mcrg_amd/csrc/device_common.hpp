@@ -152,12 +152,13 @@ __device__ __forceinline__ void metropolis_ranks(MetropolisStage &st, const Acce
     metropolis_refine(st.open, st.accept, st.m1, ref.v3, low0, low1);
 }
 
-// The ranks from the fifth on.
+// The ranks of call `from` and on: 2 for the fifth.
 __device__ __forceinline__ void metropolis_rest(uint32_t &open, uint32_t &accept, uint32_t m1, const Accept &acc,
-                                                uint32_t k0, uint32_t k1, uint32_t word, uint32_t t, uint32_t colour)
+                                                uint32_t k0, uint32_t k1, uint32_t word, uint32_t t, uint32_t colour,
+                                                uint32_t from = 2u)
 {
     const uint32_t low0 = acc.thr0 << 4, low1 = acc.thr1 << 4;
-    for (uint32_t call = 2; open != 0u; ++call) {
+    for (uint32_t call = from; open != 0u; ++call) {
         const u32x4 ref = philox(word, t, call, (kTagSweep << 28) | (colour << 24), k0, k1);
         metropolis_refine(open, accept, m1, ref.v0, low0, low1);
         if (open != 0u) {
@@ -195,6 +196,78 @@ __device__ __forceinline__ uint32_t metropolis_word(uint32_t s, uint32_t nu, uin
     const MetropolisStage st =
         metropolis_first(s, nu, nd, nl, nr, valid, acc, philox(word, t, 0u, tag, k0, k1));
     return metropolis_second(st, valid, acc, k0, k1, word, t, colour, philox(word, t, 1u, tag, k0, k1));
+}
+
+// A word's random numbers in the form that its decision takes, drawn and
+// prepared ahead of the spins, for callers that wait for them: the first stage's
+// outcome of a site of either class (a accepted, o open), and for each rank of
+// the first CALLS refinement calls whether a site of either class is accepted
+// (all ones or 0).  The decision is then some 55 instructions instead of 95.
+template <uint32_t CALLS>
+struct MetropolisAhead {
+    uint32_t a1, o1, a2, o2, p1[4u * CALLS], p2[4u * CALLS];
+};
+
+template <uint32_t CALLS>
+__device__ __forceinline__ MetropolisAhead<CALLS> metropolis_ahead(const Accept &acc, uint32_t k0, uint32_t k1,
+                                                                   uint32_t word, uint32_t t, uint32_t colour)
+{
+    const uint32_t tag = (kTagSweep << 28) | (colour << 24), low0 = acc.thr0 << 4, low1 = acc.thr1 << 4;
+    MetropolisAhead<CALLS> h;
+    const u32x4 r = philox(word, t, 0u, tag, k0, k1);
+    const uint32_t rq[4] = {r.v0, r.v1, r.v2, r.v3};
+    h.a1 = h.a2 = 0u;
+    h.o1 = h.o2 = 0xFFFFFFFFu;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t b0 = 0u - ((acc.thr0 >> (31 - q)) & 1u), b1 = 0u - ((acc.thr1 >> (31 - q)) & 1u);
+        h.a1 |= h.o1 & ~rq[q] & b0;
+        h.o1 &= ~(rq[q] ^ b0);
+        h.a2 |= h.o2 & ~rq[q] & b1;
+        h.o2 &= ~(rq[q] ^ b1);
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < CALLS; ++c) {
+        const u32x4 x = philox(word, t, 1u + c, tag, k0, k1);
+        const uint32_t w[4] = {x.v0, x.v1, x.v2, x.v3};
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            h.p1[4u * c + k] = w[k] < low0 ? 0xFFFFFFFFu : 0u;
+            h.p2[4u * c + k] = w[k] < low1 ? 0xFFFFFFFFu : 0u;
+            // drawn here and not, by the compiler, where it is first needed
+            asm volatile("" : "+v"(h.p1[4u * c + k]), "+v"(h.p2[4u * c + k]));
+        }
+    }
+    asm volatile("" : "+v"(h.a1), "+v"(h.o1), "+v"(h.a2), "+v"(h.o2));
+    return h;
+}
+
+// The bits to flip, as metropolis_word.
+template <uint32_t CALLS>
+__device__ __forceinline__ uint32_t metropolis_decide(const MetropolisAhead<CALLS> &h, uint32_t s, uint32_t nu,
+                                                      uint32_t nd, uint32_t nl, uint32_t nr, const Accept &acc,
+                                                      uint32_t k0, uint32_t k1, uint32_t word, uint32_t t,
+                                                      uint32_t colour)
+{
+    const uint32_t a1 = s ^ nu, a2 = s ^ nd, a3 = s ^ nl, a4 = s ^ nr;
+    const uint32_t x1 = a1 ^ a2, y1 = a1 & a2, x2 = a3 ^ a4, y2 = a3 & a4;
+    const uint32_t any = a1 | a2 | a3 | a4;
+    const uint32_t c1 = (x1 ^ x2) & ~(y1 | y2), c2 = ~any;  // one anti-aligned neighbour, none
+    const uint32_t m1 = acc.always0 ? 0u : c1, m2 = acc.always1 ? 0u : c2;
+    uint32_t flip = (any & ~c1) | (c1 & ~m1) | (c2 & ~m2) | (m1 & h.a1) | (m2 & h.a2);
+    uint32_t open = (m1 & h.o1) | (m2 & h.o2);
+#pragma unroll
+    for (uint32_t c = 0; c < CALLS; ++c) {
+        if (c > 0u && open == 0u) break;
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            const uint32_t lsb = open & (0u - open);
+            open ^= lsb;
+            flip |= lsb & ((m1 & h.p1[4u * c + k]) | (~m1 & h.p2[4u * c + k]));
+        }
+    }
+    metropolis_rest(open, flip, m1, acc, k0, k1, word, t, colour, 1u + CALLS);
+    return flip;
 }
 
 // The decisions of K words of one colour a lane, f[k] the bits to flip of

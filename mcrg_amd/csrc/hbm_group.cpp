@@ -108,12 +108,13 @@ hipError_t SweepRunner::run(const HbmLattice *d, int n_lats, int L, int n_levels
         }
         return hipSuccess;
     }
-    if (sampler == MCRG_SAMPLER_METROPOLIS && L >= kSmallChainMinL && L <= kSmallChainMaxL) {
+    if (chain_on_chip(L, sampler == MCRG_SAMPLER_METROPOLIS)) {
         for (; done < n; done += std::min(n - done, kSmallSweeps)) {
             const int ev = tm ? tm->begin(kKindSweep, s) : -1;
-            if ((e = launch_small_chain(d, n_lats, L, n_levels, std::min(n - done, kSmallSweeps), measure, s)) !=
-                hipSuccess)
-                return e;
+            const uint32_t part = std::min(n - done, kSmallSweeps);
+            e = L <= kSmallChainMaxL ? launch_small_chain(d, n_lats, L, n_levels, part, measure, s)
+                                     : launch_colour_chain(d, n_lats, L, n_levels, part, measure, s);
+            if (e != hipSuccess) return e;
             if (tm) tm->end(ev, s);
         }
         return hipSuccess;

@@ -129,6 +129,15 @@ hipError_t launch_sw_wg(const HbmLattice *d, int n_lats, int L, int n_levels, in
 constexpr int kSmallChainMinL = 8, kSmallChainMaxL = 32;
 hipError_t launch_small_chain(const HbmLattice *d, int n_lats, int L, int n_levels, uint32_t n, bool measure,
                               hipStream_t s);
+// The same for 64 <= L <= kColourMaxL, a workgroup each.
+constexpr int kColourMaxL = 128;
+hipError_t launch_colour_chain(const HbmLattice *d, int n_lats, int L, int n_levels, uint32_t n, bool measure,
+                               hipStream_t s);
+// Whether SweepRunner holds an int8 Metropolis lattice on chip for a launch.
+inline bool chain_on_chip(int L, bool metropolis)
+{
+    return metropolis && L >= kSmallChainMinL && L <= kColourMaxL;
+}
 hipError_t launch_int8_half_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
                                   uint32_t colour, hipStream_t s);
 hipError_t launch_int8_measure0(const HbmLattice *d, int n_lats, int L, uint32_t t_off,

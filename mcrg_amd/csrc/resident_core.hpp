@@ -8,6 +8,16 @@
 
 namespace mcrg {
 
+// LDS words that several waves read and write between barriers.
+__device__ __forceinline__ uint32_t lds_ld(const uint32_t *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_st(uint32_t *p, uint32_t v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // Sum over the aligned group of `width` lanes (1..64, a power of two) that
 // contains this lane; for width 64 the total is valid in lanes 0..31.
 __device__ __forceinline__ uint32_t group_sum(uint32_t v, uint32_t width)

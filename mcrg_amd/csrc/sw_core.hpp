@@ -88,15 +88,6 @@ __device__ __forceinline__ uint32_t run_later(uint32_t g, uint32_t r)
     return (g & r) << 1;
 }
 
-__device__ __forceinline__ uint32_t lds_ld(const uint32_t *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void lds_st(uint32_t *p, uint32_t v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 // Joins the trees of a and b, walking up both at once and halving the paths
 // (every second label on the way moves to its parent's parent, so that the
 // chains that simultaneous links leave behind shrink under the walks); of two

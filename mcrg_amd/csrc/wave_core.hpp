@@ -234,6 +234,49 @@ __device__ __forceinline__ void wave_accumulate(int64_t *rec, const int32_t (&S)
     add(tail + 3u, 1);
 }
 
+// A block of samples, one a lane with `pending`: the rest of the sample of
+// sweep ts, whose entry is `in`, to the record of its bin.  rec holds the record
+// of rec_bin (0xFFFFFFFF: none), flush adds it to the results and clears it.
+template <uint32_t L, typename Flush>
+__device__ __forceinline__ void wave_finish(const uint32_t *in, uint32_t nl, uint32_t k0, uint32_t k1, uint32_t ts,
+                                            uint32_t bin, bool pending, int64_t *rec, uint32_t &rec_bin, Flush flush)
+{
+    using Geom = WaveGeom<L>;
+    int32_t S[Geom::NLMAX + 1u][3], M = 0;
+#pragma unroll
+    for (uint32_t l = 0; l < Geom::front; ++l) {
+        const uint32_t x = in[2u * l], y = in[2u * l + 1u];
+        const int32_t sites = (int32_t)((L >> l) * (L >> l));
+        S[l][0] = 2 * sites - 2 * (int32_t)(x & 0xFFFFu);
+        S[l][1] = 2 * sites - 2 * (int32_t)(x >> 16);
+        S[l][2] = sites - 2 * (int32_t)(y & 0xFFFFu);
+        if (l == 0u) M = sites - 2 * (int32_t)(y >> 16);
+    }
+    if (nl >= Geom::front) {
+        SmallLevel<16u> x;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) x.w[k] = in[2u * Geom::front + k];
+        small_levels<16u, Geom::front, Geom::NLMAX>(x, nl, S, [&](uint32_t call, uint32_t level, uint32_t *out) {
+            const u32x4 c = philox(call, ts, 0u, (kTagTie << 28) | (level << 16), k0, k1);
+            out[0] = c.v0;
+            out[1] = c.v1;
+            out[2] = c.v2;
+            out[3] = c.v3;
+        });
+    }
+    for (uint64_t pend; (pend = __ballot(pending)) != 0ull;) {
+        // the earliest bin of the pending samples
+        const uint32_t nb = (uint32_t)__builtin_amdgcn_readlane((int)bin, (int)__builtin_ctzll(pend));
+        if (nb != rec_bin) {
+            if (rec_bin != 0xFFFFFFFFu) flush();
+            rec_bin = nb;
+        }
+        const bool take = pending && bin == nb;
+        wave_accumulate<Geom::NLMAX>(rec, S, M, take, nl);
+        pending = pending && !take;
+    }
+}
+
 // Advances the wave's lattice by up to n sweeps; `me` is the same in every lane.
 template <uint32_t L>
 __device__ __forceinline__ void run_wave(const SmallLattice &me, uint32_t n, uint32_t nl, uint32_t *lds,
@@ -272,46 +315,9 @@ __device__ __forceinline__ void run_wave(const SmallLattice &me, uint32_t n, uin
         if (slot + 1u < 64u && it + 1u < last) continue;
         // ---- a block of samples: lane u finishes sweep block + u
         small_sync();
-        bool pending = u <= slot;
-        const uint32_t q0 = me.n_measured + (block - therm), spb = me.spb;
-        const uint32_t bin = (q0 + u) / spb;
-        int32_t S[Geom::NLMAX + 1u][3], M = 0;
-        {
-            const uint32_t *in = lds + u * Geom::stride;
-#pragma unroll
-            for (uint32_t l = 0; l < Geom::front; ++l) {
-                const uint32_t x = in[2u * l], y = in[2u * l + 1u];
-                const int32_t sites = (int32_t)((L >> l) * (L >> l));
-                S[l][0] = 2 * sites - 2 * (int32_t)(x & 0xFFFFu);
-                S[l][1] = 2 * sites - 2 * (int32_t)(x >> 16);
-                S[l][2] = sites - 2 * (int32_t)(y & 0xFFFFu);
-                if (l == 0u) M = sites - 2 * (int32_t)(y >> 16);
-            }
-            if (nl >= Geom::front) {
-                SmallLevel<16u> x;
-#pragma unroll
-                for (uint32_t k = 0; k < 8u; ++k) x.w[k] = in[2u * Geom::front + k];
-                const uint32_t ts = t0 + block + u;
-                small_levels<16u, Geom::front, Geom::NLMAX>(x, nl, S, [&](uint32_t call, uint32_t level, uint32_t *out) {
-                    const u32x4 c = philox(call, ts, 0u, (kTagTie << 28) | (level << 16), k0, k1);
-                    out[0] = c.v0;
-                    out[1] = c.v1;
-                    out[2] = c.v2;
-                    out[3] = c.v3;
-                });
-            }
-        }
-        for (uint64_t pend; (pend = __ballot(pending)) != 0ull;) {
-            // the earliest bin of the pending samples
-            const uint32_t nb = (uint32_t)__builtin_amdgcn_readlane((int)bin, (int)__builtin_ctzll(pend));
-            if (nb != rec_bin) {
-                if (rec_bin != 0xFFFFFFFFu) flush();
-                rec_bin = nb;
-            }
-            const bool take = pending && bin == nb;
-            wave_accumulate<Geom::NLMAX>(rec, S, M, take, nl);
-            pending = pending && !take;
-        }
+        const uint32_t q0 = me.n_measured + (block - therm);
+        wave_finish<L>(lds + u * Geom::stride, nl, k0, k1, t0 + block + u, (q0 + u) / me.spb, u <= slot, rec, rec_bin,
+                       flush);
         block = it + 1u;
         small_sync();
     }
