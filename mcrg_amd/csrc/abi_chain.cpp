@@ -98,6 +98,8 @@ struct mcrg_chain_s {
     uint32_t n_measured = 0;       // host mirror of state[1]
     SweepRunner runner;            // replayed graphs of long sweep runs
     StripRunner strip;             // cooperative strip launches (large Metropolis chains)
+    std::shared_ptr<ResultLines> lines;  // the context's, of which this chain has `line`, or -1
+    int line = -1;
 };
 
 // Fails when a strip launch since the last check gave up on a wait.
@@ -164,6 +166,10 @@ mcrg_status mcrg_ctx_create(int32_t device, mcrg_ctx *out)
     // the allocation-free sweep's workspace on this device (see strip.hpp); a
     // failure is reported by that entry point, not here
     (void)static_scratch_setup(device);
+    try {
+        c->lines = std::make_shared<ResultLines>();
+    } catch (const std::bad_alloc &) {  // results are copied instead
+    }
     *out = c;
     return MCRG_OK;
 }
@@ -263,6 +269,8 @@ mcrg_status mcrg_chain_create(mcrg_ctx ctx, const mcrg_chain_desc *desc, mcrg_ch
         return fail(e, "hipMemcpyAsync");
     if ((e = launch_int8_init(ch->d_desc, 1, d.L, ch->stream)) != hipSuccess) return fail(e, "k_int8_init");
     if ((e = hipStreamSynchronize(ch->stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
+    ch->lines = ctx->lines;
+    if (ch->lines) ch->line = ch->lines->take();
     *out = ch;
     return MCRG_OK;
 }
@@ -274,6 +282,7 @@ mcrg_status mcrg_chain_destroy(mcrg_chain ch)
     (void)hipStreamSynchronize(ch->stream);
     (void)hipStreamDestroy(ch->stream);
     (void)hipFree(ch->d_block);
+    if (ch->lines) ch->lines->give(ch->line);
     delete ch;
     return MCRG_OK;
 }
@@ -292,6 +301,18 @@ mcrg_status mcrg_chain_set_coupling(mcrg_chain ch, double coupling)
     return MCRG_OK;
 }
 
+// The longest run of sweeps that a launch per step takes to its end sooner than
+// a cooperative launch of strips, which is 57 us before its first sweep (L =
+// 1024: 21 us against 60 for one sweep, 48 / 68 for four, 83 / 78 for eight;
+// measured 39 / 74 for one, 91 / 81 for three; L = 2048: 56 / 70 for four, 78 / 76
+// for six; measured 78 / 81 for two; L = 4096: 67 / 76 for two, 92 / 83 for
+// three; measured 76 / 82 for one).
+static int32_t launched_singly(int L, bool measure)
+{
+    if (L <= 2048) return measure ? 2 : 5;
+    return L == 4096 ? (measure ? 1 : 2) : 0;
+}
+
 mcrg_status mcrg_chain_sweep(mcrg_chain ch, int32_t n_sweeps, int32_t measure)
 {
     MCRG_REQUIRE(ch != nullptr, "chain is null");
@@ -308,7 +329,8 @@ mcrg_status mcrg_chain_sweep(mcrg_chain ch, int32_t n_sweeps, int32_t measure)
     MCRG_REQUIRE((uint64_t)ch->t + (uint64_t)n_sweeps <= 0xFFFFFFFFull, "sweep counter overflow");
     MCRG_HIP(hipSetDevice(ch->ctx->device));
     KernelTimer *tm = ch->ctx->timer.enabled ? &ch->ctx->timer : nullptr;
-    if (!chain_on_chip(d.L, d.sampler == MCRG_SAMPLER_METROPOLIS) && ch->strip.usable(ch->host, measure != 0))
+    if (!chain_on_chip(d.L, d.sampler == MCRG_SAMPLER_METROPOLIS) &&
+        n_sweeps > launched_singly(d.L, measure != 0) && ch->strip.usable(ch->host, measure != 0))
         MCRG_HIP(ch->strip.run(ch->d_desc, ch->host, ch->t, ch->n_measured, (uint32_t)n_sweeps, measure != 0,
                                ch->stream, tm));
     else
@@ -422,12 +444,17 @@ mcrg_status mcrg_chain_operators(mcrg_chain ch, int64_t out[4])
     MCRG_REQUIRE(ch != nullptr && out != nullptr, "null argument");
     MCRG_HIP(hipSetDevice(ch->ctx->device));
     hipStream_t s = ch->stream;
-    MCRG_HIP(hipMemsetAsync(ch->host.sums, 0, 4 * sizeof(unsigned long long), s));
-    MCRG_HIP(launch_int8_measure0(ch->d_desc, 1, ch->desc.L, 0u, s));
     unsigned long long cnt[4];
-    MCRG_HIP(hipMemcpyAsync(cnt, ch->host.sums, sizeof(cnt), hipMemcpyDeviceToHost, s));
-    MCRG_HIP(hipMemsetAsync(ch->host.sums, 0, 4 * sizeof(unsigned long long), s));
-    MCRG_HIP(hipStreamSynchronize(s));
+    if (ch->line >= 0) {
+        unsigned long long *line = ch->lines->base + ch->line * ResultLines::kWords;
+        MCRG_HIP(launch_int8_operators(ch->d_desc, ch->desc.L, line, s));
+        MCRG_HIP(hipStreamSynchronize(s));
+        std::memcpy(cnt, line, sizeof(cnt));
+    } else {
+        MCRG_HIP(launch_int8_operators(ch->d_desc, ch->desc.L, ch->host.sums + kSumOut, s));
+        MCRG_HIP(hipMemcpyAsync(cnt, ch->host.sums + kSumOut, sizeof(cnt), hipMemcpyDeviceToHost, s));
+        MCRG_HIP(hipStreamSynchronize(s));
+    }
     const int64_t n0 = (int64_t)ch->desc.L * ch->desc.L;
     out[0] = 2 * n0 - 2 * (int64_t)cnt[0];
     out[1] = 2 * n0 - 2 * (int64_t)cnt[1];

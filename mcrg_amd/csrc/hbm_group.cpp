@@ -22,7 +22,7 @@ HbmBlock hbm_block(int L, int n_levels, int max_bins, int sampler)
     b.spins = 0;
     b.lvl = align256(b.spins + n_spins);
     b.sums = align256(b.lvl + n_lvl * 4u);
-    b.state = align256(b.sums + kSumWords * 8u);
+    b.state = align256(b.sums + kSumAlloc * 8u);
     b.rec = align256(b.state + 2u * 4u);
     b.sw = align256(b.rec + (size_t)max_bins * record_size((uint32_t)n_levels) * 8u);
     b.bytes = align256(b.sw + (sw_tiled(L, sampler) ? sw_scratch_bytes(L) : 0u));

@@ -261,6 +261,105 @@ __global__ __launch_bounds__(256) void k_int8_measure0(const HbmLattice *__restr
     block_add<4>(lat.sums, c);
 }
 
+// Rows a thread of k_int8_operators works off: at most 256 workgroups of 1024
+// threads, since each takes a ticket of the same word (12 ns).
+static uint32_t operators_rows(uint32_t L)
+{
+    uint32_t rows = 1u;
+    while ((uint64_t)(L / rows) * (L / 16u) > 262144u) rows *= 2u;
+    return rows;
+}
+
+// The level-0 counts of the lattice as it is, without a blocking: a thread per 16
+// columns and `rows` rows (L >= 16) or per site.  Workgroups leave their counts in
+// the level scratch, and the one that finishes last adds them up.
+// Bound by the launch and the host's wait for it below L = 4096, and by memory
+// above (L = 16384 reads 268 MB).
+__global__ __launch_bounds__(1024) void k_int8_operators(const HbmLattice *__restrict__ lats, uint32_t rows,
+                                                         unsigned long long *__restrict__ out)
+{
+    __shared__ uint32_t sum[4], last;
+    if (threadIdx.x < 4u) sum[threadIdx.x] = 0u;
+    __syncthreads();
+    const HbmLattice &lat = lats[0];
+    const uint32_t L = (uint32_t)lat.L, i = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
+    const int8_t *spins = lat.spins;
+    uint32_t c[4] = {0u, 0u, 0u, 0u};  // dNN, dNNN, dP, ndown
+    if (L >= 16u) {
+        const uint32_t cpr = L >> 4, q = i & (cpr - 1u), y0 = (i >> __builtin_ctz(cpr)) * rows;
+        const bool on = y0 < L;
+        // the chunk to the right sits in a lane of this wave, but for lane 63 of wider rows
+        const uint32_t right = cpr >= 64u ? (lane + 1u) & 63u : (lane & ~(cpr - 1u)) | ((q + 1u) & (cpr - 1u));
+        const bool outside = cpr > 64u && lane == 63u;
+        const int8_t *col = spins + 16u * q, *col_next = spins + ((16u * q + 16u) & (L - 1u));
+        auto load = [&](uint32_t y, uint32_t &w, uint32_t &shifted) {
+            const size_t at = (size_t)(y & (L - 1u)) * L;
+            uint4 v = make_uint4(0u, 0u, 0u, 0u);
+            if (on) v = *reinterpret_cast<const uint4 *>(col + at);
+            uint32_t b = 0;
+            if (on && outside) b = sbit(col_next[at]);
+            w = sign4(v.x) | (sign4(v.y) << 4) | (sign4(v.z) << 8) | (sign4(v.w) << 12);
+            const uint32_t n = (uint32_t)__shfl((int)w, (int)right, 64);
+            shifted = (w >> 1) | ((outside ? b : n & 1u) << 15);
+        };
+        uint32_t s, rt;
+        load(y0, s, rt);
+        for (uint32_t r = 0; r < rows; ++r) {
+            uint32_t d, g;
+            load(y0 + r + 1u, d, g);
+            c[0] += popc(s ^ rt) + popc(s ^ d);
+            c[1] += popc(s ^ g) + popc(rt ^ d);
+            c[2] += popc(xor3(s, rt, d) ^ g);
+            c[3] += popc(s);
+            s = d;
+            rt = g;
+        }
+    } else if (i < L * L) {
+        const uint32_t x = i & (L - 1u), y = i / L, xp = (x + 1u) & (L - 1u), yp = (y + 1u) & (L - 1u);
+        const uint32_t a = sbit(spins[y * L + x]), b = sbit(spins[y * L + xp]);
+        const uint32_t e = sbit(spins[yp * L + x]), d = sbit(spins[yp * L + xp]);
+        c[0] = (a ^ b) + (a ^ e);
+        c[1] = (a ^ d) + (b ^ e);
+        c[2] = a ^ b ^ e ^ d;
+        c[3] = a;
+    }
+    auto add = [&]() {
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            c[k] = wave_sum(c[k]);
+            if (lane == 0u) atomicAdd(sum + k, c[k]);
+        }
+        __syncthreads();
+    };
+    add();
+    if (gridDim.x > 1u) {
+        if (threadIdx.x < 4u)
+            __hip_atomic_store(lat.lvl + 4u * blockIdx.x + threadIdx.x, sum[threadIdx.x], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (threadIdx.x == 0u) {
+            __threadfence();
+            last = atomicAdd(lat.sums + kSumTicket, 1ull) + 1ull == (unsigned long long)gridDim.x ? 1u : 0u;
+            __threadfence();
+        }
+        __syncthreads();
+        if (last == 0u) return;
+        // at most 256 workgroups: one a thread (sums at most 2^29)
+        if (threadIdx.x < 4u) sum[threadIdx.x] = 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k)
+            c[k] = threadIdx.x < gridDim.x ? __hip_atomic_load(lat.lvl + 4u * threadIdx.x + k, __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_AGENT)
+                                           : 0u;
+        __syncthreads();
+        add();
+        if (threadIdx.x == 0u) lat.sums[kSumTicket] = 0ull;
+    }
+    if (threadIdx.x < 4u)
+        __hip_atomic_store(out + threadIdx.x, (unsigned long long)sum[threadIdx.x], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---------------------------------------------------------------- levels >= 1
 // A grid-measured level l (side Ll >= kGridLevelMinL): one thread per word of
 // the level for its operators, and one per word of level l + 1 for the
@@ -400,6 +499,15 @@ hipError_t launch_int8_half_sweep(const HbmLattice *d, int n_lats, int L, uint32
     const uint32_t n_items = L >= 64 ? n_words / half_sweep_rows((uint32_t)L) : n_words;
     hipLaunchKernelGGL(k_int8_half_sweep, dim3(cdiv(n_items, 256u), (uint32_t)n_lats), dim3(256), 0,
                        s, d, t_off, colour);
+    return hipGetLastError();
+}
+
+hipError_t launch_int8_operators(const HbmLattice *d, int L, unsigned long long *out, hipStream_t s)
+{
+    const uint32_t rows = operators_rows((uint32_t)L), n = (uint32_t)L;
+    const uint32_t n_items = n >= 16u ? n / rows * (n / 16u) : n * n;
+    const uint32_t threads = n_items >= 1024u ? 1024u : 256u;  // 256: one workgroup
+    hipLaunchKernelGGL(k_int8_operators, dim3(cdiv(n_items, threads)), dim3(threads), 0, s, d, rows, out);
     return hipGetLastError();
 }
 

@@ -19,6 +19,8 @@ constexpr uint32_t kWgLevelMaxL = kGridLevelMinL / 2;
 // Counters per lattice: level-0 dNN, dNNN, dP, ndown, then dNN, dNNN, dP of
 // every grid-measured level l >= 1 at 4 + 3 (l - 1).
 constexpr uint32_t kSumWords = 4u + 3u * kMaxLevels;
+// behind them: k_int8_operators' count of finished workgroups and its results
+constexpr uint32_t kSumTicket = kSumWords, kSumOut = kSumWords + 1u, kSumAlloc = kSumWords + 5u;
 
 // Rows per thread strip of the int8 half-sweep (L >= 64).  Up to L = 8192 the
 // lattice (<= 64 MiB) stays in the 256 MB last-level cache, so each row's three
@@ -93,7 +95,7 @@ __device__ __forceinline__ int64_t record_term(uint32_t j, uint32_t nl, const in
 struct HbmLattice {
     int8_t *spins;              // L*L int8, row-major (x fastest)
     uint32_t *lvl;              // bit-packed levels 1.. at level_offset(L, l)
-    unsigned long long *sums;   // kSumWords disagreement counters
+    unsigned long long *sums;   // kSumWords disagreement counters, 0 between kernels; kSumAlloc words
     int64_t *records;           // max_bins * record_size(n_levels)
     uint32_t *state;            // [0] sweep counter t, [1] measured-sample counter
     uint32_t k0, k1;            // Philox key = seed
@@ -140,6 +142,9 @@ inline bool chain_on_chip(int L, bool metropolis)
 }
 hipError_t launch_int8_half_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
                                   uint32_t colour, hipStream_t s);
+// Level-0 disagreement counts of one lattice (as k_int8_measure0's) into out[0..3]:
+// device memory or mapped host memory.
+hipError_t launch_int8_operators(const HbmLattice *d, int L, unsigned long long *out, hipStream_t s);
 hipError_t launch_int8_measure0(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
                                 hipStream_t s);
 // Levels 1..nl (grid launches for the large ones, then one workgroup per

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -69,9 +70,47 @@ struct KernelTimer {
     hipError_t collect();
 };
 
+// Pinned lines (64 bytes) that kernels write a chain's results to, one a chain:
+// 64 chains of a context at a time; others go without.  Kept by the context and
+// its chains.
+struct ResultLines {
+    static constexpr int kLines = 64, kWords = 8;
+    unsigned long long *base = nullptr;
+    ResultLines()
+    {
+        if (hipHostMalloc(reinterpret_cast<void **>(&base), kLines * kWords * 8u, hipHostMallocDefault) != hipSuccess) {
+            base = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+    ~ResultLines()
+    {
+        if (base) (void)hipHostFree(base);
+    }
+    ResultLines(const ResultLines &) = delete;
+    ResultLines &operator=(const ResultLines &) = delete;
+    std::mutex mu;
+    uint64_t used = 0;
+    // A free line's index, or -1.
+    int take()
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (!base || ~used == 0ull) return -1;
+        const int k = __builtin_ctzll(~used);
+        used |= 1ull << k;
+        return k;
+    }
+    void give(int k)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (k >= 0) used &= ~(1ull << k);
+    }
+};
+
 }  // namespace mcrg
 
 struct mcrg_ctx_s {
     int device = 0;
     mcrg::KernelTimer timer;
+    std::shared_ptr<mcrg::ResultLines> lines;
 };
