@@ -445,7 +445,8 @@ void ResidentEngine::rebuild_slots(uint32_t chunk)
                                                       : wave_lds_words((uint32_t)L, (uint32_t)nl)),
                                 64, true});
             else
-                pend.push_back({s, work, 4u * big_layout((uint32_t)L, (uint32_t)nl).total, threads_for(L), false});
+                pend.push_back({s, work, 4u * big_layout((uint32_t)L, (uint32_t)nl, (uint32_t)threads_for(L)).total,
+                                threads_for(L), false});
         }
     }
     // launch classes by (workgroup size, workgroups resident on the device):

@@ -4,21 +4,22 @@
 // Checkerboard words of both colours in LDS, four words a thread at a time
 // (metropolis_words).  Per measured sweep, a barrier after each:
 //   colour 0; colour 1 with the tie coins of the large blockings;
-//   level 0: operator counts and the blocking into level 1; then level by level
-//   down to side 64, spread over the workgroup, counts into the sample's entry
-//   of a ring.
-// Wave 0 alone then counts the levels of side 64 and 32 in registers (rows64)
-// and leaves the 16 x 16 level in the ring, while the others sweep on; once 64
-// samples are there, its lane u finishes sample u: the levels from side 16 down
-// and the record's terms.  So wave 0 is behind by two short steps a sample
-// instead of by every small level and the record.
+//   level 0 and the blockings down to side 64: each wave its band of rows, with
+//   the counts into the sample's entry of a ring;
+// and the operators of the levels between, spread over the workgroup.
+// Once each wave has a sample, it counts that one's levels of side 64 and 32 in
+// registers (rows64) and leaves the 16 x 16 level in the ring; once 64 samples
+// are there, wave 0's lane u finishes sample u: the levels from side 16 down and
+// the record's terms.  So no wave works on a small level while others wait.
 //
-// Bound by VALU issue (Philox) with 1024 threads, and by a lattice's latency
-// where one lattice has a compute unit to itself.  us a sweep, unmeasured and
-// measured, against one word at a time and every level in each sample's turn:
-// one L = 512, 1024 threads 14.1 -> 11.7 and 20.9 -> 17.3; 512 of them, 512
-// threads 32.5 -> 28.3 and 41.3 -> 34.5; 1024 of L = 256, 256 threads 18.0 ->
-// 14.6 and 22.8 -> 19.2.
+// Bound by VALU issue (Philox) where lattices fill the device, and by the
+// phases' latency where one has a compute unit to itself (a measured sweep's
+// level 0 2.0 us of 16.5, level 1 2.0, the others 1.2).  us a sweep, unmeasured
+// and measured, against one word at a time and every level in each sample's
+// turn: one L = 512, 1024 threads 14.1 -> 11.5 and 20.9 -> 16.5; 512 of them, 512
+// threads 32.5 -> 27.5 and 41.3 -> 30.7; 1024 of L = 256, 256 threads 18.0 ->
+// 14.6 and 22.8 -> 19.0.  With level 0 a word at a time and wave 0 alone on sides
+// 64 and 32 the first measured sweep took 17.3 and the second 35.
 #pragma once
 
 #include "wave_core.hpp"
@@ -29,12 +30,13 @@ struct BigLayout {
     uint32_t W, ls;       // words per colour; levels 0 .. ls - 1 are spread (side > 64)
     uint32_t lvl_words;   // words of levels 1 .. min(ls, nl), and of their tie coins
     uint32_t coin_calls;  // Philox calls for those
+    uint32_t row64;       // level ls of a sample a wave
     uint32_t stride;      // ring entry: 4 counts a spread level, 2 packed words for
                           // sides 64 and 32 each, 8 words of side 16; odd
     uint32_t spins, lvl, coin, ring, rec, total;
 };
 
-__host__ __device__ inline BigLayout big_layout(uint32_t L, uint32_t nl)
+__host__ __device__ inline BigLayout big_layout(uint32_t L, uint32_t nl, uint32_t threads)
 {
     BigLayout b;
     b.W = cb_words(L);
@@ -49,7 +51,8 @@ __host__ __device__ inline BigLayout big_layout(uint32_t L, uint32_t nl)
     b.spins = 0;
     b.lvl = 2u * b.W;
     b.coin = b.lvl + b.lvl_words;
-    b.ring = b.coin + b.lvl_words;
+    b.row64 = b.coin + b.lvl_words;
+    b.ring = b.row64 + (nl >= b.ls ? threads / 64u * 128u : 0u);
     b.rec = (b.ring + 64u * b.stride + 1u) & ~1u;
     b.total = b.rec + 2u * record_size(nl);
     return b;
@@ -114,11 +117,14 @@ __device__ __forceinline__ void run_slot(const Slot sl, const int32_t *__restric
     PackedLattice &P = lats[li];
     // what is the same in every lane is kept scalar
     const uint32_t nl = uni<true>((uint32_t)sl.n_levels);
-    const BigLayout lay = big_layout(L, nl);
-    const uint32_t W = lay.W, rs = record_size(nl), ls = lay.ls;
+    const BigLayout lay = big_layout(L, nl, (uint32_t)NT);
+    constexpr uint32_t W = L * L / 64u, ls = L == 512u ? 3u : 2u;
+    const uint32_t rs = record_size(nl);
     uint32_t tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     uint32_t *c0 = lds + lay.spins, *c1 = c0 + W, *lvl = lds + lay.lvl, *coins = lds + lay.coin, *ring = lds + lay.ring;
+    uint32_t *row64 = lds + lay.row64;
+    constexpr uint32_t NW = (uint32_t)NT / 64u;
     int64_t *rec = reinterpret_cast<int64_t *>(lds + lay.rec);
     Accept acc;
     acc.thr0 = uni<true>(P.acc.thr0);
@@ -187,53 +193,69 @@ __device__ __forceinline__ void run_slot(const Slot sl, const int32_t *__restric
             __syncthreads();
         }
         if (!measuring) continue;
-        // ---- the spread levels: counts into the ring entry, the next blocking
+        // ---- level 0, and every blocking down to side 64: a wave's band of rows
+        //      is blocked from its own rows alone
         const uint32_t slot = (it - therm) & 63u, block = it - slot;  // block: the ring's first sweep
-        uint32_t *entry = ring + slot * lay.stride;
-        uint32_t off = 0;
-#pragma unroll 1
-        for (uint32_t l = 0; l < ls && l <= nl; ++l) {
-            const uint32_t *src = lvl + off, *cw = coins + off + (l ? level_words(L, l) : 0u);
-            uint32_t *dst = lvl + off + (l ? level_words(L, l) : 0u);
-            uint32_t d0 = 0, d1 = 0, d2 = 0, d3 = 0;
-            if (l == 0u) {
-                for (uint32_t w = me; w < W; w += NT) {
-                    cb_ops_item(c0, c1, L, W, w, 0u, d0, d1, d2, d3);
-                    cb_ops_item(c1, c0, L, W, w, 1u, d0, d1, d2, d3);
-                }
-                if (nl > 0u)
-                    for (uint32_t j = me; j < cb_block_items(L); j += NT) dst[j] = cb_block_item(c0, c1, L, W, j, cw[j]);
-            } else {
-                const uint32_t Ll = L >> l;
-                for (uint32_t i = me; i < rm_ops_items(Ll); i += NT) rm_ops_item(src, Ll, i, d0, d1, d2);
-                if (l < nl)
-                    for (uint32_t j = me; j < rm_block_items(Ll); j += NT) dst[j] = rm_block_item(src, Ll, j, cw[j]);
-                off += level_words(L, l);
-            }
+        uint32_t *entry = ring + slot * lay.stride, *last64 = row64 + (slot % NW) * 128u;
+        const uint32_t band = me >> 6;
+        auto count = [&](uint32_t l, uint32_t d0, uint32_t d1, uint32_t d2, uint32_t d3) {
             d0 = group_sum(d0, 64u);
             d1 = group_sum(d1, 64u);
             d2 = group_sum(d2, 64u);
-            d3 = l == 0u ? group_sum(d3, 64u) : 0u;
+            if (l == 0u) d3 = group_sum(d3, 64u);
             if (lane == 0u) {
                 atomicAdd(entry + 4u * l, d0);
                 atomicAdd(entry + 4u * l + 1u, d1);
                 atomicAdd(entry + 4u * l + 2u, d2);
                 if (l == 0u) atomicAdd(entry + 3, d3);
             }
-            __syncthreads();
-        }
-        if (me >= 64u) continue;
-        // ---- wave 0: sides 64 and 32, the side-16 level into the ring.  No
-        //      barrier follows: the others touch neither the ring nor the
-        //      levels before wave 0 has met them twice in the next sweep.
-        auto coin = [&](uint32_t call, uint32_t level) {
-            return philox(call, t, 0u, (kTagTie << 28) | (level << 16), k0, k1);
         };
-        if (nl >= ls) {
-            const uint32_t *row = lvl + off + 2u * lane;
-            rows64(row[0], row[1], ls, nl, coin, entry + 4u * ls, entry + 4u * ls + 4u);
+        {
+            constexpr uint32_t wpr = L / 64u, n = W / 2u / NW;
+            uint32_t d0 = 0, d1 = 0, d2 = 0, d3 = 0;
+            for (uint32_t k = lane; k < n; k += 64u) {
+                const uint32_t i = band * n + k, q = i % wpr, y = i / wpr * 2u;
+                cb_rows<2u>(c0, c1, L, q, y, nl > 0u, coins + i, lvl + i, d0, d1, d2, d3);
+            }
+            uint32_t off = 0;
+            for (uint32_t l = 1; l < ls && l < nl; ++l) {
+                small_sync();
+                const uint32_t *src = lvl + off;
+                off += level_words(L, l);
+                uint32_t *dst = l + 1u < ls ? lvl + off : last64;
+                const uint32_t m = level_words(L, l + 1u) / NW;
+                for (uint32_t k = lane; k < m; k += 64u)
+                    dst[band * m + k] = rm_block_item(src, L >> l, band * m + k, coins[off + band * m + k]);
+            }
+            count(0u, d0, d1, d2, d3);
         }
-        if (slot + 1u < 64u && it + 1u < last) continue;
+        __syncthreads();
+        // ---- the operators of the levels down to side 128
+        {
+            uint32_t off = 0;
+            for (uint32_t l = 1; l < ls && l <= nl; ++l) {
+                uint32_t d0 = 0, d1 = 0, d2 = 0;
+                for (uint32_t i = me; i < rm_ops_items(L >> l); i += NT) rm_ops_item(lvl + off, L >> l, i, d0, d1, d2);
+                count(l, d0, d1, d2, 0u);
+                off += level_words(L, l);
+            }
+        }
+        // ---- a sample a wave: sides 64 and 32, the side-16 level into the ring.
+        //      The next sample's levels are written two barriers from here.
+        const bool full = slot + 1u == 64u || it + 1u == last;
+        if (nl >= ls && (full || slot % NW + 1u == NW)) {
+            const uint32_t mine = slot - slot % NW + (me >> 6);
+            if (mine <= slot) {
+                const uint32_t ts = t0 + block + mine, *row = row64 + (me >> 6) * 128u + 2u * lane;
+                auto coin = [&](uint32_t call, uint32_t level) {
+                    return philox(call, ts, 0u, (kTagTie << 28) | (level << 16), k0, k1);
+                };
+                uint32_t *e = ring + mine * lay.stride + 4u * ls;
+                rows64(row[0], row[1], ls, nl, coin, e, e + 4u);
+            }
+        }
+        if (full) __syncthreads();
+        if (me >= 64u || !full) continue;
         // ---- 64 samples: lane u finishes sweep block + u
         small_sync();
         bool pending = lane <= slot;
