@@ -168,7 +168,8 @@ mcrg_status mcrg_ctx_create(int32_t device, mcrg_ctx *out)
     (void)static_scratch_setup(device);
     try {
         c->lines = std::make_shared<ResultLines>();
-    } catch (const std::bad_alloc &) {  // results are copied instead
+        c->arenas = std::make_shared<ArenaPool>();
+    } catch (const std::bad_alloc &) {  // results are copied, arenas freed
     }
     *out = c;
     return MCRG_OK;
@@ -244,7 +245,7 @@ mcrg_status mcrg_chain_create(mcrg_ctx ctx, const mcrg_chain_desc *desc, mcrg_ch
     const HbmBlock blk = hbm_block(d.L, d.n_levels, d.max_bins, d.sampler);
     const size_t o_desc = blk.bytes;
     const size_t total = align256(o_desc + sizeof(HbmLattice));
-    hipError_t e = hipMalloc(&ch->d_block, total);
+    hipError_t e = device_malloc(&ch->d_block, total, ctx->arenas.get());
     if (e != hipSuccess) {
         delete ch;
         set_error(std::string("hipMalloc: ") + hipGetErrorString(e));

@@ -315,7 +315,7 @@ mcrg_status mcrg_server_create(mcrg_ctx ctx, const mcrg_server_opts *opts, mcrg_
     s->lds_budget = lds_budget;
     s->adaptive_large = adaptive;
     hipError_t e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = s->engine.init(ctx->device, (size_t)budget, max_jobs, eo, s->stream);
+    if (e == hipSuccess) e = s->engine.init(ctx->device, (size_t)budget, max_jobs, eo, s->stream, ctx->arenas, true);
     if (e != hipSuccess) {
         set_error(std::string("server allocation: ") + hipGetErrorString(e));
         delete s;

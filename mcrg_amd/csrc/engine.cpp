@@ -12,16 +12,20 @@ namespace mcrg {
 static size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // ------------------------------------------------------------------ Arena
-hipError_t Arena::init(size_t bytes)
+hipError_t Arena::init(size_t bytes, std::shared_ptr<ArenaPool> pool, bool keep)
 {
     cap_ = round_up(bytes, 256);
     used_ = 0;
     free_.clear();
-    void *p = nullptr;
-    hipError_t e = hipMalloc(&p, cap_);
-    if (e != hipSuccess) {
-        cap_ = 0;
-        return e;
+    pool_ = std::move(pool);
+    keep_ = keep && pool_ != nullptr;
+    void *p = keep_ ? pool_->take(cap_) : nullptr;
+    if (!p) {
+        hipError_t e = device_malloc(&p, cap_, pool_.get());
+        if (e != hipSuccess) {
+            cap_ = 0;
+            return e;
+        }
     }
     base_ = static_cast<char *>(p);
     free_[0] = cap_;
@@ -30,7 +34,7 @@ hipError_t Arena::init(size_t bytes)
 
 void Arena::release()
 {
-    if (base_) (void)hipFree(base_);
+    if (base_ && !(keep_ && pool_->give(base_, cap_))) (void)hipFree(base_);
     base_ = nullptr;
     cap_ = used_ = 0;
     free_.clear();
@@ -123,7 +127,6 @@ ResidentEngine::~ResidentEngine()
     if (tune_b_) (void)hipEventDestroy(tune_b_);
     for (hipEvent_t e : ev_join_)
         if (e) (void)hipEventDestroy(e);
-    arena_.release();
     if (d_lats_) (void)hipFree(d_lats_);
     if (d_slots_) (void)hipFree(d_slots_);
     if (d_slot_lats_) (void)hipFree(d_slot_lats_);
@@ -140,17 +143,18 @@ ResidentEngine::~ResidentEngine()
         (void)hipStreamSynchronize(rb_);
         (void)hipStreamDestroy(rb_);
     }
+    arena_.release();  // nothing reads or writes it any more
 }
 
-hipError_t ResidentEngine::init(int device, size_t arena_bytes, int capacity, const EngineOptions &opt,
-                                hipStream_t s)
+hipError_t ResidentEngine::init(int device, size_t arena_bytes, int capacity, const EngineOptions &opt, hipStream_t s,
+                                std::shared_ptr<ArenaPool> pool, bool keep)
 {
     device_ = device;
     stream_ = s;
     opt_ = opt;
     capacity_ = capacity;
     hipError_t e;
-    if ((e = arena_.init(arena_bytes)) != hipSuccess) return e;
+    if ((e = arena_.init(arena_bytes, std::move(pool), keep)) != hipSuccess) return e;
     if ((e = hipMalloc(&d_lats_, sizeof(PackedLattice) * (size_t)capacity)) != hipSuccess) return e;
     if ((e = hipMalloc(&d_queue_, 64u * kMaxClasses)) != hipSuccess) return e;
     if ((e = hipMalloc(&d_err_, sizeof(uint32_t))) != hipSuccess) return e;

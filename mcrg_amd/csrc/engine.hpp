@@ -8,10 +8,12 @@
 #include <cmath>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
 #include "resident.hpp"
+#include "runtime.hpp"
 
 namespace mcrg {
 
@@ -28,7 +30,9 @@ struct JobSpec {
 // First-fit allocator over one device allocation (offsets in bytes).
 class Arena {
   public:
-    hipError_t init(size_t bytes);
+    // `keep`: the memory comes from the pool when it has some of this size, and
+    // goes back there.
+    hipError_t init(size_t bytes, std::shared_ptr<ArenaPool> pool, bool keep);
     void release();
     // Returns false when no free range is large enough.
     bool alloc(size_t bytes, size_t &off);
@@ -40,15 +44,19 @@ class Arena {
   private:
     char *base_ = nullptr;
     size_t cap_ = 0, used_ = 0;
+    std::shared_ptr<ArenaPool> pool_;
+    bool keep_ = false;
     std::map<size_t, size_t> free_;  // offset -> size
 };
 
-// Measured-sweep time model of one slot on MI355X (from per-L runs of the
-// batched workload: about 8 us per sample plus 75 ns per site a lane sweeps).
-constexpr uint64_t kSweepFixedNs = 8000;
-// A measured sweep of a lattice held by one wave, on a filled device.
-inline uint64_t wave_sweep_ns(int L) { return L <= 32 ? 1500 : L == 64 ? 2500 : 6000; }
-constexpr uint64_t kSweepPerSiteNs = 75;
+// Measured-sweep time model of one slot on MI355X: L = 512 with 1024 threads (256
+// sites a lane) 16.5 us, with 512 threads and two a compute unit 30.7; L = 256
+// with 1024 threads 7, with 256 threads and four a unit 19.
+constexpr uint64_t kSweepFixedNs = 4000;
+constexpr uint64_t kSweepPerSiteNs = 50;
+// A measured sweep of a lattice held by one wave, beside workgroups of larger
+// ones (L = 128: 8 us; 5.7 without them).
+inline uint64_t wave_sweep_ns(int L) { return L <= 32 ? 1500 : L == 64 ? 2500 : 8000; }
 
 // The autotuner keeps the configuration in use unless a candidate's measured
 // rate exceeds it by this factor.
@@ -110,7 +118,9 @@ class PinnedPair {
 class ResidentEngine {
   public:
     ~ResidentEngine();
-    hipError_t init(int device, size_t arena_bytes, int capacity, const EngineOptions &opt, hipStream_t s);
+    // `keep`: the arena comes from the pool and goes back there (Arena::init).
+    hipError_t init(int device, size_t arena_bytes, int capacity, const EngineOptions &opt, hipStream_t s,
+                    std::shared_ptr<ArenaPool> pool, bool keep);
 
     // Validates a job for this engine; empty string when it is admissible.
     static std::string check(const JobSpec &j);
