@@ -440,16 +440,29 @@ __device__ __forceinline__ uint32_t tile_root(uint32_t *lab, uint32_t x)
 // One workgroup per tile (blockIdx.x) and lattice (blockIdx.y), a thread for
 // each part of PW sites.  `first`: the spins come from the int8 lattice, else
 // from the bits of the sweep before.
+// Bound by the latency of the walks in the union-find (14k cycles of 45k for the
+// unions, 12k for the runs' roots, alike with four and with six waves a SIMD)
+// and by VALU issue (about 70%).  64 lattices of L = 1024: three launches 377 ->
+// 347 us a sweep with seven workgroups a compute unit instead of six, one
+// comparison a step of a walk instead of three, and every run's label set to
+// its root at the end of its walk.
 template <uint32_t PW>
 __global__ __launch_bounds__(kTileSites / PW) void k_sw_tile(const HbmLattice *__restrict__ lats, uint32_t t_off,
                                                              uint32_t first)
 {
     constexpr uint32_t NT = kTileSites / PW;
-    __shared__ uint32_t lab[33u * kTileWords];
+    // 23040 bytes in all, a multiple of the allocation unit (1280) of which seven
+    // workgroups find room in a compute unit: the row below and the column to the
+    // right are read before there are labels, and the edge positions' roots take
+    // the words of the down bonds, which are in registers by then
+    __shared__ uint32_t words[kTileWords + 33u * kTileWords];
+    uint32_t *S = words, *lab = words + kTileWords, *col = lab + 2;
     // the lists of unions, later the site map
     constexpr uint32_t kScratch = NT / 64u * kSwList > kTileSites / 4u ? NT / 64u * kSwList : kTileSites / 4u;
     __shared__ __align__(16) uint32_t scratch[kScratch];
-    __shared__ uint32_t S[kTileWords + 2u], R[kTileWords], D[kTileWords], C[kTileWords], col[2], node_root[kTileNodes];
+    __shared__ uint32_t R[kTileWords], D[kTileWords], C[kTileWords];
+    uint16_t *node_root = reinterpret_cast<uint16_t *>(D);
+    static_assert(2u * kTileNodes <= sizeof(D), "node_root");
     const HbmLattice &lat = lats[blockIdx.y];
     const uint32_t L = (uint32_t)lat.L, mask = L - 1u, wpr = L >> 5;
     const SwTiles st = sw_tiles(lat);
@@ -493,6 +506,7 @@ __global__ __launch_bounds__(kTileSites / PW) void k_sw_tile(const HbmLattice *_
     __syncthreads();
     const uint32_t ends = 0x80000000u;
     const uint32_t r = R[i] & ~ends, up = i >= 2u ? D[i - 2u] : 0u, rup = i >= 2u ? R[i - 2u] & ~ends : 0u;
+    const uint32_t seam0 = D[kTileWords - 2u], seam1 = D[kTileWords - 1u];
     const uint32_t pm = part_mask<PW>(lo);
     sw_hook(lab, i, kTile, ~(r << 1) & pm, r, up, rup);
     __syncthreads();
@@ -508,7 +522,7 @@ __global__ __launch_bounds__(kTileSites / PW) void k_sw_tile(const HbmLattice *_
         const uint32_t w = 2u * y + (x >> 5);
         const uint32_t root = tile_root(lab, 33u * w + run_start(R[w] & ~ends, x & 31u));
         __hip_atomic_fetch_max(lab + root, kTag | pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        node_root[pos] = root;
+        node_root[pos] = (uint16_t)root;
     }
     {
         uint4 *z = reinterpret_cast<uint4 *>(scratch);
@@ -528,34 +542,37 @@ __global__ __launch_bounds__(kTileSites / PW) void k_sw_tile(const HbmLattice *_
     uint32_t f = 0, starts = ~(r << 1) & pm;
     uint8_t *map = reinterpret_cast<uint8_t *>(scratch);
     while (starts != 0u) {
-        uint32_t s[4], x[4], p[4], g[4];
+        uint32_t s[4], p[4], v[4];
 #pragma unroll
         for (uint32_t k = 0; k < 4u; ++k) {
             s[k] = starts ? (uint32_t)__builtin_ctz(starts) : 32u;
             starts &= starts - 1u;
-            x[k] = p[k] = 33u * i + (s[k] & 31u);
-            g[k] = lds_ld(lab + p[k]);  // g = the label of p, x the label before p
+            p[k] = 33u * i + (s[k] & 31u);
+            v[k] = lds_ld(lab + p[k]);
         }
-        for (bool more = true; more;) {
-            more = false;
-            uint32_t h[4];
+        // v is the label of p: less than p unless p is a root (labels point to
+        // smaller ids, and a root's is its own or a tag).  A label moves on to
+        // its parent's unless that is a root.
+        for (;;) {
+            if (__ballot(v[0] < p[0] || v[1] < p[1] || v[2] < p[2] || v[3] < p[3]) == 0ull) break;
+            uint32_t u[4];
 #pragma unroll
-            for (uint32_t k = 0; k < 4u; ++k) h[k] = lds_ld(lab + ((g[k] & kTag) ? p[k] : g[k]));
+            for (uint32_t k = 0; k < 4u; ++k) u[k] = lds_ld(lab + (v[k] < p[k] ? v[k] : p[k]));
 #pragma unroll
             for (uint32_t k = 0; k < 4u; ++k) {
-                if (g[k] == p[k] || (g[k] & kTag)) continue;
-                // p -> g -> h: p's label moves on to h unless g is a root
-                if (!(h[k] & kTag) && h[k] != g[k]) lds_st(lab + p[k], h[k]);
-                p[k] = g[k];
-                g[k] = h[k];
-                more = true;
+                const bool on = v[k] < p[k];
+                if (on && u[k] < v[k]) lds_st(lab + p[k], u[k]);
+                p[k] = on ? v[k] : p[k];
+                v[k] = u[k];
             }
         }
 #pragma unroll
         for (uint32_t k = 0; k < 4u; ++k) {
             if (s[k] >= 32u) continue;
-            if (g[k] & kTag) {
-                map[32u * i + s[k]] = (uint8_t)g[k];
+            // for the walks beside and behind this one
+            lds_st(lab + 33u * i + s[k], (v[k] & kTag) ? v[k] : p[k]);
+            if (v[k] & kTag) {
+                map[32u * i + s[k]] = (uint8_t)v[k];
             } else {
                 const uint32_t m = sw_site(p[k]);
                 f |= ((C[m >> 5] >> (m & 31u)) & 1u) << s[k];
@@ -571,7 +588,7 @@ __global__ __launch_bounds__(kTileSites / PW) void k_sw_tile(const HbmLattice *_
         const uint64_t b = __ballot((R[2u * lane + 1u] & ends) != 0u);
         if (lane == 0u) {
             st.seams[2u * tile] = b;
-            st.seams[2u * tile + 1u] = (uint64_t)D[kTileWords - 2u] | ((uint64_t)D[kTileWords - 1u] << 32);
+            st.seams[2u * tile + 1u] = (uint64_t)seam0 | ((uint64_t)seam1 << 32);
         }
     }
     __syncthreads();
