@@ -53,43 +53,18 @@ sys.path.insert(0, ROOT)
 
 METRIC = "spin-updates/ns (batched vs plain) at matched y_t error; p50/p99 job latency"
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per launch of k_resident<threads>, keyed by (replicas, sweeps per
-# launch, threads, min_team, max_slot_lds, threads_large, sub_chunks), from two rocprofv3
-# --pmc passes over `bench.py --only batched --sub-chunks 1` (FETCH_SIZE x 2.00
-# + WRITE_SIZE x 1.00 KiB per dispatch, the scale factors read off the same
-# counters on a 1 GiB read + 1 GiB write copy kernel, --copy-calibration).
-# Configurations without a counter run report null.  The passes ran with
-# every slot in one part (sub_chunks 1); the default splits slots into parts,
-# each of which reloads and writes back its lattices, and is not counted.
-# Every configuration the autotuner can keep has its passes (threads, min_team,
-# max_slot_lds); threads_large only concerns L >= 512 and leaves this manifest's
-# slots as they are.  A launch of two classes (max_slot_lds 65536) sums both.
-MEASURED_TRAFFIC = {
-    (4096, 100, 256, 16, 0, 0, 1): (3282.0 * 2.0 + 5048.0) * 1024.0,
-    (4096, 100, 256, 16, 0, 512, 1): (3282.0 * 2.0 + 5048.0) * 1024.0,
-    (4096, 100, 256, 32, 0, 0, 1): (3285.7 * 2.0 + 5047.8) * 1024.0,
-    (4096, 100, 256, 8, 0, 0, 1): (3284.3 * 2.0 + 5047.8) * 1024.0,
-    (4096, 100, 128, 16, 0, 0, 1): (3176.6 * 2.0 + 5066.3) * 1024.0,
-    (4096, 100, 512, 16, 0, 0, 1): (3267.4 * 2.0 + 5012.3) * 1024.0,
-    (4096, 100, 256, 16, 65536, 0, 1): (2.0 * 1746.6 * 2.0 + 2.0 * 2523.5) * 1024.0,
-}
+# HBM bytes per launch of k_wave, keyed by (replicas, sweeps per launch): every
+# lattice of this manifest (L <= 128) is held by one wave, whatever workgroup,
+# team and LDS sizes the run asks for.  From rocprofv3 --pmc passes over
+# `bench.py --only batched` (FETCH_SIZE x 2.00 + WRITE_SIZE x 1.00 KiB per
+# dispatch, the scale factors read off the same counters on a 1 GiB read + 1 GiB
+# write copy kernel, --copy-calibration).  Configurations without a counter run
+# report null.
+MEASURED_TRAFFIC = {(4096, 100): (4690.4 * 2.0 + 6159.1) * 1024.0}
 # The same kernel is bound by VALU issue, not HBM: rocprofv3 --pmc SQ_INSTS_VALU
-# and GRBM_GUI_ACTIVE over the same one-part launches give the wave-level VALU
-# instructions per launch and the busy cycles per XCD (8 XCDs, 1024 SIMDs that
-# issue one wave64 VALU instruction per 4 cycles); parts add only their
-# reloads.  The 128- and 512-thread shapes and the 64 KiB cap were counted on
-# a kernel that read each lattice's two sweep counters with two loads (about
-# 0.5 % more VALU instructions than this one).
-MEASURED_VALU = {
-    (4096, 100, 256, 16, 0, 0, 1): {"valu_wave_instr_per_launch": 4.6509e8, "gui_active_cycles_per_xcd": 2.4379e7 / 8},
-    (4096, 100, 256, 16, 0, 512, 1): {"valu_wave_instr_per_launch": 4.6509e8, "gui_active_cycles_per_xcd": 2.4379e7 / 8},
-    (4096, 100, 256, 32, 0, 0, 1): {"valu_wave_instr_per_launch": 4.6509e8, "gui_active_cycles_per_xcd": 2.4261e7 / 8},
-    (4096, 100, 256, 8, 0, 0, 1): {"valu_wave_instr_per_launch": 4.6509e8, "gui_active_cycles_per_xcd": 2.4248e7 / 8},
-    (4096, 100, 128, 16, 0, 0, 1): {"valu_wave_instr_per_launch": 4.9458e8, "gui_active_cycles_per_xcd": 3.4708e7 / 8},
-    (4096, 100, 512, 16, 0, 0, 1): {"valu_wave_instr_per_launch": 4.6728e8, "gui_active_cycles_per_xcd": 3.7474e7 / 8},
-    (4096, 100, 256, 16, 65536, 0, 1): {"valu_wave_instr_per_launch": 2.0 * 2.3104e8,
-                                        "gui_active_cycles_per_xcd": 2.4222e7 / 8},
-}
+# over the same launches gives the wave-level VALU instructions per launch (1024
+# SIMDs that issue one wave64 VALU instruction per 4 cycles).
+MEASURED_VALU = {(4096, 100): {"valu_wave_instr_per_launch": 2.5651e8}}
 
 
 KIND_STRIP = 4  # mcrg_ctx_kernel_time kind of the strip kernel
@@ -364,21 +339,18 @@ def cpu_baseline(jobs, sweeps, threads):
 
 
 def valu_roofline(cfg_key, sites, sps, avg_ms, clock_khz, cus):
-    """VALU issue roof of the resident kernel: wave64 VALU instructions per
+    """VALU issue roof of the batched kernel: wave64 VALU instructions per
     launch (rocprofv3 SQ_INSTS_VALU) x 64 lanes over the launch's event-timed
     duration, against cus x 4 SIMDs x 16 lanes x the engine clock."""
-    m = MEASURED_VALU.get(cfg_key) or MEASURED_VALU.get(cfg_key[:-1] + (1,))
+    m = MEASURED_VALU.get(cfg_key)
     if not m:
         return None
     peak = cus * 4 * 16 * clock_khz * 1e3 / 1e12  # T lane-instructions / s
     achieved = 64.0 * m["valu_wave_instr_per_launch"] / (avg_ms * 1e-3) / 1e12
-    exact = cfg_key in MEASURED_VALU
     return {"bound": "valu", "achieved": achieved, "peak": peak, "unit": "T lane-instr/s", "frac": achieved / peak,
             "lane_instr_per_update": 64.0 * m["valu_wave_instr_per_launch"] / (sites * sps),
-            "source": ("rocprofv3 --pmc SQ_INSTS_VALU on bench.py --only batched "
-                       + ("(this configuration)" if exact else "with every slot in one part (the parts of this "
-                          "configuration add only their reloads)"))
-                      + f"; duration {avg_ms:.4f} ms from HIP events on the kernel's stream in this run"}
+            "source": "rocprofv3 --pmc SQ_INSTS_VALU on bench.py --only batched "
+                      f"(this configuration); duration {avg_ms:.4f} ms from HIP events on the kernel's stream in this run"}
 
 
 def run_bisection(rounds):
@@ -512,8 +484,7 @@ def main():
         f"threads_large={tuned['threads_large']} sub_chunks={tuned['sub_chunks']}")
 
     avg_ms, n_launch = run_batched_timed(mcrg_amd, ctx, jobs, args.sweeps_per_step, tuned, 11)
-    cfg_key = (len(jobs), args.sweeps_per_step, tuned["threads"], tuned["min_team"], tuned["max_slot_lds"],
-               tuned["threads_large"], tuned["sub_chunks"])
+    cfg_key = (len(jobs), args.sweeps_per_step)
     bpl = bytes_per_update(True) * sites * args.sweeps_per_step
     achieved = bpl / (avg_ms * 1e-3) / 1e9
     log(f"bench: resident kernel {avg_ms:.3f} ms/launch over {n_launch} launches -> {achieved:.1f} GB/s algorithmic")
@@ -570,13 +541,12 @@ def main():
                    "sites": sites, "layout": "packed", "schedule": "resident", "device": dev["name"]},
         "roofline": dict(valu or {"bound": "valu", "achieved": None, "peak": None, "unit": "T lane-instr/s",
                                   "frac": None, "source": "no counter run for this configuration"},
-                         traffic=MEASURED_TRAFFIC.get(cfg_key), kernel=f"k_resident<{tuned['threads']}>",
+                         traffic=MEASURED_TRAFFIC.get(cfg_key), kernel="k_wave",
                          avg_ms=avg_ms,
                          hbm={"achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                               "frac": achieved / HBM_PEAK_GBS, "bytes_per_launch": bpl,
-                              "counted_bytes_one_part": MEASURED_TRAFFIC.get(cfg_key[:-1] + (1,)),
-                              "counted_basis": "rocprofv3 FETCH_SIZE x 2 + WRITE_SIZE on the same configuration "
-                                               "with every slot in one part (parts add their reloads)",
+                              "counted_bytes": MEASURED_TRAFFIC.get(cfg_key),
+                              "counted_basis": "rocprofv3 FETCH_SIZE x 2 + WRITE_SIZE on the same configuration",
                               "basis": "algorithmic bytes (3/8 B per site update + 5/24 B per site per measured "
                                        "sweep, bit-packed streaming model)"}),
         "plain_mixed": plain_mixed,

@@ -175,12 +175,14 @@ mcrg_status mcrg_chain_operators(mcrg_chain ch, int64_t out[4]);
 /* ------------------------------------------------------------------ batches */
 /* Many independent chains (uneven L and coupling) advanced together.  Jobs of
  * 8 <= L <= 512 with the Metropolis sampler run on the resident schedule:
- * bit-packed lattices held in LDS by a persistent grid (L <= 128: in the
- * registers of single waves), one launch per chunk of sweeps.  Jobs of L = 2, 4 and L >= 1024, and Swendsen-Wang jobs, run on the
- * HBM schedule (int8 in device memory): jobs of the same L, n_levels, n_therm,
- * n_meas, sweeps_per_bin and sampler share every launch, on
- * a second stream that overlaps the resident launches, and long runs replay
- * captured HIP graphs of 32 sweeps.  A job is the reference's whole
+ * bit-packed lattices held in the registers of single waves (L <= 128) or in
+ * the LDS of a persistent grid of workgroups (L = 256, 512), one launch of each
+ * per chunk of sweeps.  Jobs of L = 2, 4 and L >= 1024, and Swendsen-Wang jobs,
+ * keep int8 lattices in device memory: jobs of the same L, n_levels, n_therm,
+ * n_meas, sweeps_per_bin and sampler share every launch, on a second stream
+ * that overlaps the resident launches.  Swendsen-Wang jobs of L <= 128 run a
+ * chunk of sweeps in one launch, a workgroup each; the others launch each phase
+ * of a sweep, and long runs replay captured HIP graphs of 32 sweeps.  A job is the reference's whole
  * calc_critical_exponent chain (src/mcrg.cpp:22-98) for one (L, K, seed):
  * n_therm unmeasured sweeps (equilibrate, src/ising.cpp:14-84) then n_meas
  * measured sweeps.  Every job is bit-identical to the same chain run alone
@@ -199,7 +201,7 @@ typedef struct {
     int32_t sweeps_per_bin; /* measured sweeps per record bin (>= 1); the job
                                has ceil(n_meas / sweeps_per_bin) bins         */
     int32_t sampler;        /* MCRG_SAMPLER_* (0 = Metropolis); Swendsen-Wang
-                               jobs run on the HBM schedule at any L          */
+                               jobs keep int8 lattices at any L               */
 } mcrg_job_desc;
 
 typedef struct {
@@ -260,11 +262,11 @@ mcrg_status mcrg_batch_get_opts(mcrg_batch b, mcrg_batch_opts *out);
  * arrival order while their spins and records fit the device-memory budget and
  * their share of LDS (slot LDS / lattices per slot) fits the LDS budget,
  * advances every admitted job by
- * one time slice per launch of the LDS-resident schedule (jobs of different L
+ * one time slice per launch of the resident schedule (jobs of different L
  * and coupling share each launch; a slot of G lattices of side L runs
  * min(sweeps_per_launch, max(1, launch_quantum / t_sweep)) sweeps, with the
- * slot's measured-sweep time modelled as 8 us + 75 ns x (sites each of its
- * lanes sweeps), so every workgroup works about launch_quantum), and retires
+ * slot's measured-sweep time modelled as 4 us + 50 ns x (sites each of its
+ * lanes sweeps), or 1.5, 2.5 and 8 us for L <= 32, 64 and 128, so every workgroup works about launch_quantum), and retires
  * finished jobs
  * between launches: their records are copied to host memory and their device
  * memory is reused by the next admissions.  A job's results are bit-identical
@@ -404,7 +406,7 @@ mcrg_status mcrg_critical_point_step_bins(const int64_t *rec_large, int32_t n_bi
 /* Kernel-duration statistics measured with HIP events on the stream that
  * launched the kernel, enabled per context.  kind: 0 = half-sweep kernel,
  * 1 = level-0 measurement kernel, 2 = levels/accumulate kernel,
- * 3 = batched resident kernel, 4 = strip kernel (one launch per
+ * 3 = batched resident kernels, 4 = strip kernel (one launch per
  * mcrg_chain_sweep call on the strip schedule). */
 mcrg_status mcrg_ctx_set_timing(mcrg_ctx ctx, int32_t enable);
 mcrg_status mcrg_ctx_kernel_time(mcrg_ctx ctx, int32_t kind, int64_t *launches, double *total_ms);

@@ -359,7 +359,7 @@ def n_bins(n_meas, sweeps_per_bin):
 
 
 class Batch:
-    """Independent chains advanced together on the LDS-resident schedule
+    """Independent chains advanced together on the resident schedule
     (mcrg_batch).  `jobs` is a list of dicts with keys L, coupling, seed,
     n_therm, n_meas, n_levels, sweeps_per_bin."""
 
@@ -426,7 +426,7 @@ class Batch:
 
 class Server:
     """Continuous-batching job server (mcrg_server): jobs are admitted while the
-    device budget has room, advance one chunk per launch of the LDS-resident
+    device budget has room, advance one chunk per launch of the resident
     schedule and retire to host memory when done.  Drive it with step() from
     this thread, or start() a scheduler thread of its own."""
 

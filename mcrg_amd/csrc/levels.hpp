@@ -200,24 +200,12 @@ __device__ __forceinline__ void cb_ops_item(const uint32_t *own, const uint32_t 
 {
     const uint32_t s = own[w];
     const Nbr4 n = cb_neighbours(oth, L, W, w, c);
-    uint32_t dr, dl;  // same colour, row y+1: (x+1, y+1) and (x-1, y+1)
-    if (L >= 64u) {
-        const uint32_t wpr = L >> 6, sh = ilog2u(wpr);
-        const uint32_t y = w >> sh, q = w & (wpr - 1u);
-        const uint32_t p = (y + c) & 1u;
-        const uint32_t row = ((y + 1u) & (L - 1u)) << sh;
-        const uint32_t nx = own[row + q];
-        const uint32_t side = own[row + ((q + 2u * p - 1u) & (wpr - 1u))];
-        dr = p == 0u ? nx : (nx >> 1) | (side << 31);
-        dl = p == 0u ? (nx << 1) | (side >> 31) : nx;
-    } else {
-        const SegMasks m = seg_masks(L);
-        const uint32_t sn = own[(w + 1u) & (W - 1u)];
-        const uint32_t nx = (s >> m.r) | (sn << (32u - m.r));
-        const uint32_t m0 = c == 0u ? m.even : ~m.even;
-        dr = (nx & m0) | (rotr_seg(nx, m) & ~m0);
-        dl = (rotl_seg(nx, m) & m0) | (nx & ~m0);
-    }
+    const SegMasks m = seg_masks(L);
+    const uint32_t sn = own[(w + 1u) & (W - 1u)];
+    const uint32_t nx = (s >> m.r) | (sn << (32u - m.r));
+    const uint32_t m0 = c == 0u ? m.even : ~m.even;
+    // same colour, row y+1: (x+1, y+1) and (x-1, y+1)
+    const uint32_t dr = (nx & m0) | (rotr_seg(nx, m) & ~m0), dl = (rotl_seg(nx, m) & m0) | (nx & ~m0);
     if (c == 0u)
         dnn += (uint32_t)(popc(s ^ n.nu) + popc(s ^ n.nd) + popc(s ^ n.nl) + popc(s ^ n.nr));
     dnnn += (uint32_t)(popc(s ^ dr) + popc(s ^ dl));
@@ -225,24 +213,12 @@ __device__ __forceinline__ void cb_ops_item(const uint32_t *own, const uint32_t 
     ndown += (uint32_t)popc(s);
 }
 
-// Work items of cb_block_item: level-1 RM words.
-__device__ __forceinline__ uint32_t cb_block_items(uint32_t L) { return (L * L / 4u + 31u) >> 5; }
-
 // Level-1 RM word i from the CB level 0 (c0, c1 = colour 0 and 1 words); ties
 // take bits of coin word i.  The four spins of block (bx, by) sit at the same
 // bit, k = bx, of the colour-0 and colour-1 words of rows 2by and 2by+1.
 __device__ __forceinline__ uint32_t cb_block_item(const uint32_t *c0, const uint32_t *c1, uint32_t L,
                                                   uint32_t W, uint32_t i, uint32_t coin)
 {
-    if (L >= 64u) {
-        const uint32_t wpr = L >> 6, sh = ilog2u(wpr);
-        const uint32_t by = i >> sh, q = i & (wpr - 1u);
-        const uint32_t r0 = ((2u * by) << sh) + q, r1 = ((2u * by + 1u) << sh) + q;
-        const uint32_t b1 = c0[r0], b2 = c1[r0], b3 = c0[r1], b4 = c1[r1];
-        const uint32_t maj3 = (b1 & b2 & (b3 | b4)) | (b3 & b4 & (b1 | b2));
-        const uint32_t tie = ~(xor3(b1, b2, b3) ^ b4) & ~(b1 & b2 & b3 & b4) & (b1 | b2 | b3 | b4);
-        return maj3 | (tie & coin);
-    }
     // L in {8, 16, 32}: CB word w holds rows w*R .. w*R + R - 1 (R = 64/L, even),
     // i.e. R/2 blocked rows = 16 output bits; output word i takes words 2i, 2i+1.
     const SegMasks m = seg_masks(L);
