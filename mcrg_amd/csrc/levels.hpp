@@ -237,23 +237,24 @@ __device__ __forceinline__ uint32_t cb_block_item(const uint32_t *c0, const uint
     return out;
 }
 
-// Word column q of rows y .. y + ROWS - 1 (y and ROWS even) of a CB level 0 with
-// L >= 64 and the row below them: their part of the operator counts, and with
+// Word column q of rows y .. y + ROWS - 1 (y and ROWS even) of a CB level 0 of wpr
+// words a row, and of the row below them (row numbers are taken & mask): their part of the operator counts, and with
 // `blocks` the words of level 1, out[0], out[wpr], .., with their coins.  Sites are taken in
 // row order, E the even columns and O the odd ones (colour 0 and 1 in even rows,
 // 1 and 0 in odd ones), so that a row needs one shift, its words serve both
 // neighbouring rows, and plaquettes come from the horizontal bonds: 12 counts
 // and 11 other operations for 64 sites (a word at a time about 70).
 template <uint32_t ROWS>
-__device__ __forceinline__ void cb_rows(const uint32_t *c0, const uint32_t *c1, uint32_t L, uint32_t q, uint32_t y,
+__device__ __forceinline__ void cb_rows(const uint32_t *c0, const uint32_t *c1, uint32_t wpr, uint32_t mask,
+                                        uint32_t q, uint32_t y,
                                         bool blocks, const uint32_t *coin, uint32_t *out, uint32_t &dnn, uint32_t &dnnn,
                                         uint32_t &dp, uint32_t &ndown)
 {
-    const uint32_t wpr = L >> 6, qn = (q + 1u) & (wpr - 1u);
+    const uint32_t qn = (q + 1u) & (wpr - 1u);
     uint32_t E = c0[y * wpr + q], O = c1[y * wpr + q], X = (E >> 1) | (c0[y * wpr + qn] << 31), h = E ^ O, hx = O ^ X;
 #pragma unroll
     for (uint32_t r = 0; r < ROWS; ++r) {
-        const uint32_t *even = r & 1u ? c0 : c1, *odd = r & 1u ? c1 : c0, row = ((y + r + 1u) & (L - 1u)) * wpr;
+        const uint32_t *even = r & 1u ? c0 : c1, *odd = r & 1u ? c1 : c0, row = ((y + r + 1u) & mask) * wpr;
         const uint32_t E1 = even[row + q], O1 = odd[row + q], X1 = (E1 >> 1) | (even[row + qn] << 31);
         const uint32_t h1 = E1 ^ O1, hx1 = O1 ^ X1;
         dnn += (uint32_t)popc(h) + (uint32_t)popc(hx) + (uint32_t)popc(E ^ E1) + (uint32_t)popc(O ^ O1);

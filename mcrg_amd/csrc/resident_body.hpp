@@ -215,7 +215,7 @@ __device__ __forceinline__ void run_slot(const Slot sl, const int32_t *__restric
             uint32_t d0 = 0, d1 = 0, d2 = 0, d3 = 0;
             for (uint32_t k = lane; k < n; k += 64u) {
                 const uint32_t i = band * n + k, q = i % wpr, y = i / wpr * 2u;
-                cb_rows<2u>(c0, c1, L, q, y, nl > 0u, coins + i, lvl + i, d0, d1, d2, d3);
+                cb_rows<2u>(c0, c1, wpr, L - 1u, q, y, nl > 0u, coins + i, lvl + i, d0, d1, d2, d3);
             }
             uint32_t off = 0;
             for (uint32_t l = 1; l < ls && l < nl; ++l) {

@@ -382,10 +382,19 @@ __device__ void strip_measure(const StripArgs &a, const StripLds &m, const uint3
         strip_levels<64u, true>(a, m, src, threadIdx.x);
     } else {
         const uint32_t t0 = one_wave ? 64u : 0u;
-        for (uint32_t j = threadIdx.x - t0; j < 2u * R * wpr; j += NT - t0) {
-            const uint32_t c = j >> sc, jj = j & ((1u << sc) - 1u);
-            const uint32_t r = 1u + (jj >> sw), qq = jj & (wpr - 1u);
-            strip_ops0(src + c * m.cbs, src + (c ^ 1u) * m.cbs, wpr, r, qq, y0 + r - 1u, c, d0, d1, d2, d3);
+        if constexpr (NT >= 512) {
+            // two rows a thread; local row 1 is the strip's first row, an even
+            // one (measured L = 4096 12.1 -> 11.4 us a sweep, 8192 28.6 -> 25.8;
+            // smaller workgroups, which wait for wave 0's levels, took 1% longer)
+            for (uint32_t j = threadIdx.x - t0; j < (R >> 1) * wpr; j += NT - t0)
+                cb_rows<2u>(src + wpr, src + m.cbs + wpr, wpr, ~0u, j & (wpr - 1u), (j >> sw) << 1, false, nullptr,
+                            nullptr, d0, d1, d2, d3);
+        } else {
+            for (uint32_t j = threadIdx.x - t0; j < 2u * R * wpr; j += NT - t0) {
+                const uint32_t c = j >> sc, jj = j & ((1u << sc) - 1u);
+                const uint32_t r = 1u + (jj >> sw), qq = jj & (wpr - 1u);
+                strip_ops0(src + c * m.cbs, src + (c ^ 1u) * m.cbs, wpr, r, qq, y0 + r - 1u, c, d0, d1, d2, d3);
+            }
         }
         wave_add(m.pend, 4u, d0, d1, d2, d3);
     }
