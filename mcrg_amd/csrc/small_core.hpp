@@ -5,13 +5,16 @@
 // w = u mod W of both colours; the T / W groups of W lanes hold copies and do
 // the same updates.  Neighbour words come from DPP rotations within a group, so
 // a sweep touches neither LDS nor a barrier.  What the copies are for:
-//   * group j draws the Philox calls of sweep it0 + j, both colours, and every
-//     group fetches them when that sweep is due: one draw per T / W sweeps;
+//   * group j draws and prepares the random numbers of sweep it0 + j, both
+//     colours, and every group fetches them when that sweep is due: one draw per
+//     T / W sweeps;
 //   * samples are kept in LDS as words, and once T sweeps have passed lane u
 //     measures sample u by itself, whole levels as words in registers: no lane
 //     idles and nothing is reduced but the record's terms.
 // Bound by the latency of a wave's dependent instructions (a measured sweep of
-// one lattice 0.8 us at L = 8, 0.9 at 16, 1.25 at 32); teams of 4 or 16 lanes in
+// one lattice 0.56 us at L = 8, 0.72 at 16, 0.98 at 32, unmeasured 0.46, 0.51 and
+// 0.74; with the calls' words fetched as they are drawn 0.73, 0.89 and 1.11, and
+// 0.63, 0.67 and 0.84); teams of 4 or 16 lanes in
 // a workgroup's LDS took 8 to 10 us, and one launch per phase 32 us.
 #pragma once
 
@@ -223,6 +226,40 @@ __device__ __forceinline__ void small_accumulate(int64_t *rec, const int32_t (&S
     }
 }
 
+// A word's random numbers as metropolis_ahead prepares them, the outcomes of its
+// four ranks as bits (class 1 from bit 0, class 2 from bit 4): a lane prepares one
+// sweep of a team's B at a time, and five words a half sweep go to the lanes that
+// decide, which then have 65 instructions instead of 95 and eight words.
+struct SmallDraw {
+    uint32_t a1, o1, a2, o2, ranks;
+};
+
+__device__ __forceinline__ SmallDraw small_draw(const Accept &acc, uint32_t k0, uint32_t k1, uint32_t word, uint32_t t,
+                                                uint32_t colour)
+{
+    const MetropolisAhead<1u> h = metropolis_ahead<1u>(acc, k0, k1, word, t, colour);
+    uint32_t ranks = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) ranks |= (h.p1[k] & (1u << k)) | (h.p2[k] & (16u << k));
+    return SmallDraw{h.a1, h.o1, h.a2, h.o2, ranks};
+}
+
+__device__ __forceinline__ uint32_t small_decide(const SmallDraw &d, uint32_t s, const Nbr4 &nb, const Accept &acc,
+                                                 uint32_t k0, uint32_t k1, uint32_t word, uint32_t t, uint32_t colour)
+{
+    MetropolisAhead<1u> h;
+    h.a1 = d.a1;
+    h.o1 = d.o1;
+    h.a2 = d.a2;
+    h.o2 = d.o2;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        h.p1[k] = (uint32_t)((int32_t)(d.ranks << (31u - k)) >> 31);
+        h.p2[k] = (uint32_t)((int32_t)(d.ranks << (27u - k)) >> 31);
+    }
+    return metropolis_decide<1u>(h, s, nb.nu, nb.nd, nb.nl, nb.nr, acc, k0, k1, word, t, colour);
+}
+
 // ------------------------------------------------------------------ the run
 // Advances the wave's lattices by up to n sweeps.  c0, c1 are the lane's words;
 // nl blockings; `lds` small_lds_words(L, 64 / T, nl) words.
@@ -257,7 +294,7 @@ __device__ __forceinline__ void run_small(const SmallLattice &me, uint32_t n, ui
     }
     last = (uint32_t)__builtin_amdgcn_readfirstlane((int)last);
     begin = (uint32_t)__builtin_amdgcn_readfirstlane((int)begin);
-    u32x4 r0{0u, 0u, 0u, 0u}, f0 = r0, r1 = r0, f1 = r0;
+    SmallDraw d0{}, d1{};
     uint32_t block = 0;  // sweep of the sample block's first slot
     uint32_t k0 = me.k0, k1 = me.k1;
     for (uint32_t it = 0; it < last; ++it) {
@@ -266,26 +303,25 @@ __device__ __forceinline__ void run_small(const SmallLattice &me, uint32_t n, ui
         const uint32_t j = it & (B - 1u), t = me.t + it;
         if (j == 0u) {
             const uint32_t tj = t + u / W;
-            metropolis_rng(w, tj, 0u, k0, k1, r0, f0);
-            metropolis_rng(w, tj, 1u, k0, k1, r1, f1);
+            d0 = small_draw(me.acc, k0, k1, w, tj, 0u);
+            d1 = small_draw(me.acc, k0, k1, w, tj, 1u);
         }
         const int src = (int)((lane & ~(T - 1u)) + j * W + w);
-        auto fetch = [&](const u32x4 &x) {
-            if (B == 1u) return x;
-            return u32x4{(uint32_t)__shfl((int)x.v0, src, 64), (uint32_t)__shfl((int)x.v1, src, 64),
-                         (uint32_t)__shfl((int)x.v2, src, 64), (uint32_t)__shfl((int)x.v3, src, 64)};
+        auto fetch = [&](const SmallDraw &d) {
+            if (B == 1u) return d;
+            return SmallDraw{(uint32_t)__shfl((int)d.a1, src, 64), (uint32_t)__shfl((int)d.o1, src, 64),
+                             (uint32_t)__shfl((int)d.a2, src, 64), (uint32_t)__shfl((int)d.o2, src, 64),
+                             (uint32_t)__shfl((int)d.ranks, src, 64)};
         };
         const bool running = it < total;
         {
             const Nbr4 nb = cb_neighbours_small(c1, lane_prev<W>(c1), lane_next<W>(c1), L, 0u);
-            const uint32_t f = metropolis_word_drawn(c0, nb.nu, nb.nd, nb.nl, nb.nr, 0xFFFFFFFFu, me.acc, k0, k1, w,
-                                                     t, 0u, fetch(r0), fetch(f0));
+            const uint32_t f = small_decide(fetch(d0), c0, nb, me.acc, k0, k1, w, t, 0u);
             c0 ^= running ? f : 0u;
         }
         {
             const Nbr4 nb = cb_neighbours_small(c0, lane_prev<W>(c0), lane_next<W>(c0), L, 1u);
-            const uint32_t f = metropolis_word_drawn(c1, nb.nu, nb.nd, nb.nl, nb.nr, 0xFFFFFFFFu, me.acc, k0, k1, w,
-                                                     t, 1u, fetch(r1), fetch(f1));
+            const uint32_t f = small_decide(fetch(d1), c1, nb, me.acc, k0, k1, w, t, 1u);
             c1 ^= running ? f : 0u;
         }
         if (it < begin) continue;
