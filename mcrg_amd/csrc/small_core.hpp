@@ -6,15 +6,15 @@
 // the same updates.  Neighbour words come from DPP rotations within a group, so
 // a sweep touches neither LDS nor a barrier.  What the copies are for:
 //   * group j draws and prepares the random numbers of sweep it0 + j, both
-//     colours, and every group fetches them when that sweep is due: one draw per
+//     colours, and every group fetches them a sweep before they are due: one draw per
 //     T / W sweeps;
 //   * samples are kept in LDS as words, and once T sweeps have passed lane u
 //     measures sample u by itself, whole levels as words in registers: no lane
 //     idles and nothing is reduced but the record's terms.
 // Bound by the latency of a wave's dependent instructions (a measured sweep of
-// one lattice 0.56 us at L = 8, 0.72 at 16, 0.98 at 32, unmeasured 0.46, 0.51 and
-// 0.74; with the calls' words fetched as they are drawn 0.73, 0.89 and 1.11, and
-// 0.63, 0.67 and 0.84); teams of 4 or 16 lanes in
+// one lattice 0.52 us at L = 8, 0.64 at 16, 0.95 at 32, unmeasured 0.41, 0.47 and
+// 0.68; with the numbers fetched in the sweep that needs them 0.56, 0.72 and 0.98,
+// and with the calls' words as they are drawn 0.73, 0.89 and 1.11); teams of 4 or 16 lanes in
 // a workgroup's LDS took 8 to 10 us, and one launch per phase 32 us.
 #pragma once
 
@@ -294,15 +294,14 @@ __device__ __forceinline__ void run_small(const SmallLattice &me, uint32_t n, ui
     }
     last = (uint32_t)__builtin_amdgcn_readfirstlane((int)last);
     begin = (uint32_t)__builtin_amdgcn_readfirstlane((int)begin);
-    SmallDraw d0{}, d1{};
+    SmallDraw d0{}, d1{}, n0{}, n1{};
     uint32_t block = 0;  // sweep of the sample block's first slot
     uint32_t k0 = me.k0, k1 = me.k1;
-    for (uint32_t it = 0; it < last; ++it) {
-        // the keys anew in every sweep: their 18 round keys are not kept
-        asm volatile("" : "+v"(k0), "+v"(k1));
-        const uint32_t j = it & (B - 1u), t = me.t + it;
+    // sweep it's numbers to n0 and n1
+    auto next = [&](uint32_t it) {
+        const uint32_t j = it & (B - 1u);
         if (j == 0u) {
-            const uint32_t tj = t + u / W;
+            const uint32_t tj = me.t + it + u / W;
             d0 = small_draw(me.acc, k0, k1, w, tj, 0u);
             d1 = small_draw(me.acc, k0, k1, w, tj, 1u);
         }
@@ -313,15 +312,26 @@ __device__ __forceinline__ void run_small(const SmallLattice &me, uint32_t n, ui
                              (uint32_t)__shfl((int)d.a2, src, 64), (uint32_t)__shfl((int)d.o2, src, 64),
                              (uint32_t)__shfl((int)d.ranks, src, 64)};
         };
+        n0 = fetch(d0);
+        n1 = fetch(d1);
+    };
+    if (last > 0u) next(0u);
+    for (uint32_t it = 0; it < last; ++it) {
+        // the keys anew in every sweep: their 18 round keys are not kept
+        asm volatile("" : "+v"(k0), "+v"(k1));
+        const uint32_t t = me.t + it;
+        const SmallDraw e0 = n0, e1 = n1;
+        // the next sweep's while this one is decided
+        next(it + 1u);
         const bool running = it < total;
         {
             const Nbr4 nb = cb_neighbours_small(c1, lane_prev<W>(c1), lane_next<W>(c1), L, 0u);
-            const uint32_t f = small_decide(fetch(d0), c0, nb, me.acc, k0, k1, w, t, 0u);
+            const uint32_t f = small_decide(e0, c0, nb, me.acc, k0, k1, w, t, 0u);
             c0 ^= running ? f : 0u;
         }
         {
             const Nbr4 nb = cb_neighbours_small(c0, lane_prev<W>(c0), lane_next<W>(c0), L, 1u);
-            const uint32_t f = small_decide(fetch(d1), c1, nb, me.acc, k0, k1, w, t, 1u);
+            const uint32_t f = small_decide(e1, c1, nb, me.acc, k0, k1, w, t, 1u);
             c1 ^= running ? f : 0u;
         }
         if (it < begin) continue;
