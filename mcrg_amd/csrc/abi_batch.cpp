@@ -6,10 +6,8 @@
 // stream that overlaps the resident launches.
 #include <algorithm>
 #include <cstdlib>
-#include <cstring>
 #include <map>
 #include <memory>
-#include <mutex>
 #include <new>
 #include <string>
 #include <tuple>
@@ -17,6 +15,7 @@
 
 #include "engine.hpp"
 #include "hbm_group.hpp"
+#include "record_block.hpp"
 #include "runtime.hpp"
 
 using namespace mcrg;
@@ -39,19 +38,6 @@ bool resident_job(const JobSpec &s)
     }();
     return allowed && s.sampler == MCRG_SAMPLER_METROPOLIS && s.L >= kResidentMinL && s.L <= kResidentMaxL;
 }
-// Records read ahead.  One job's records cost a round trip to the device (26
-// us); a caller that reads one job after the other gets the following ones
-// along, more with every such read, in one copy (4096 jobs: 110 -> 12 ms with
-// the callers' own time).  What was read ahead is dropped once the batch runs on.
-struct RecordBlock {
-    static constexpr size_t kMaxBytes = size_t(1) << 20;
-    std::mutex mu;            // calls on one batch from several threads
-    std::vector<char> data;
-    std::vector<size_t> off;  // per job, into data
-    int first = 0, count = 0;
-    int next = -1, window = 1;  // the job behind the last one read, jobs then read at once
-    uint64_t runs = 0;          // mcrg_batch_run calls before the read
-};
 }  // namespace
 
 struct mcrg_batch_s {
@@ -63,7 +49,6 @@ struct mcrg_batch_s {
     uint32_t chunk = 250;
     std::vector<std::unique_ptr<HbmGroup>> groups;
     std::vector<JobRef> refs;  // job index -> where it runs
-    uint64_t runs = 0;         // mcrg_batch_run calls
     RecordBlock ahead;
 
     ~mcrg_batch_s()
@@ -241,10 +226,7 @@ mcrg_status mcrg_batch_run(mcrg_batch b, int32_t max_sweeps, int32_t *remaining)
     MCRG_REQUIRE(max_sweeps >= 0, "max_sweeps must be >= 0");
     MCRG_HIP(hipSetDevice(b->ctx->device));
     uint32_t left = (uint32_t)max_sweeps;
-    {
-        std::lock_guard<std::mutex> lk(b->ahead.mu);
-        ++b->runs;
-    }
+    RecordBlock::Running running(b->ahead);
     KernelTimer *tm = b->ctx->timer.enabled ? &b->ctx->timer : nullptr;
     while (left > 0 && b->max_remaining() > 0) {
         // HBM groups first: their launches queue on the second stream while the
@@ -289,54 +271,36 @@ mcrg_status mcrg_batch_get_records(mcrg_batch b, int32_t job, int64_t *host, int
     MCRG_HIP(hipSetDevice(b->ctx->device));
     const int64_t want = records_of(b, job);
     MCRG_REQUIRE(n == want, "n must be n_bins * mcrg_record_size(n_levels)");
-    RecordBlock &rb = b->ahead;
-    std::lock_guard<std::mutex> lk(rb.mu);
-    const bool fresh = rb.runs == b->runs;
-    if (fresh && job >= rb.first && job < rb.first + rb.count) {
-        std::memcpy(host, rb.data.data() + rb.off[(size_t)(job - rb.first)], (size_t)n * 8u);
-        rb.next = job + 1;
-        return MCRG_OK;
-    }
-    rb.window = fresh && job == rb.next ? std::min(8 * rb.window, 4096) : 1;
-    rb.count = 0;
-    rb.runs = b->runs;
-    rb.next = job + 1;
-    // the following jobs of the same place, as many as the window and the buffer hold
     const JobRef r = b->refs[(size_t)job];
-    int count = 1;
-    size_t bytes = (size_t)n * 8u;
-    while (count < rb.window && job + count < (int)b->refs.size()) {
-        const JobRef &x = b->refs[(size_t)(job + count)];
-        if (x.group != r.group || x.index != r.index + count) break;
-        const size_t more = x.group < 0 ? ResidentEngine::job_bytes(b->engine.spec(x.index))
+    const size_t bytes = (size_t)n * 8u;
+    // the following jobs of the same place come along
+    auto more = [&](int k) -> size_t {
+        if (job + k >= (int)b->refs.size()) return 0;
+        const JobRef &x = b->refs[(size_t)(job + k)];
+        if (x.group != r.group || x.index != r.index + k) return 0;
+        return x.group < 0 ? ResidentEngine::job_bytes(b->engine.spec(x.index))
                            : b->groups[(size_t)x.group]->record_pitch();
-        if (bytes + more > RecordBlock::kMaxBytes) break;
-        bytes += more;
-        ++count;
-    }
-    if (r.group < 0) {
-        size_t range = 0;
-        if (count > 1) range = b->engine.record_range(r.index, count, rb.off);
-        if (range == 0) {
-            MCRG_HIP(b->engine.read_records(r.index, host, n));
-            return MCRG_OK;
+    };
+    auto one = [&]() {
+        return r.group < 0 ? b->engine.read_records(r.index, host, n)
+                           : b->groups[(size_t)r.group]->read_records(r.index, host, n, b->hbm_stream);
+    };
+    auto block = [&](int count, std::vector<size_t> &off, std::vector<char> &data) {
+        if (r.group < 0) {
+            const size_t range = b->engine.record_range(r.index, count, off);
+            if (range == 0) {
+                off.clear();
+                return hipSuccess;
+            }
+            data.resize(range);
+            return b->engine.read_range(r.index, range, data.data());
         }
-        rb.data.resize(range);
-        MCRG_HIP(b->engine.read_range(r.index, range, rb.data.data()));
-    } else {
         HbmGroup &g = *b->groups[(size_t)r.group];
-        if (count == 1) {
-            MCRG_HIP(g.read_records(r.index, host, n, b->hbm_stream));
-            return MCRG_OK;
-        }
-        rb.off.resize((size_t)count);
-        for (int k = 0; k < count; ++k) rb.off[(size_t)k] = (size_t)k * g.record_pitch();
-        rb.data.resize(rb.off.back() + (size_t)n * 8u);
-        MCRG_HIP(g.read_records_block(r.index, count, rb.data.data(), b->hbm_stream));
-    }
-    rb.first = job;
-    rb.count = count;
-    std::memcpy(host, rb.data.data() + rb.off[0], (size_t)n * 8u);
+        for (int k = 0; k < count; ++k) off.push_back((size_t)k * g.record_pitch());
+        data.resize(off.back() + bytes);
+        return g.read_records_block(r.index, count, data.data(), b->hbm_stream);
+    };
+    MCRG_HIP(b->ahead.read<hipError_t>(job, reinterpret_cast<char *>(host), bytes, more, one, block));
     return MCRG_OK;
 }
 
