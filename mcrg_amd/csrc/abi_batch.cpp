@@ -27,16 +27,17 @@ struct JobRef {
 };
 
 // Metropolis jobs of kResidentMinL <= L <= kResidentMaxL run on the resident
-// engine, the rest in int8 HBM-schedule groups.  MCRG_BATCH_RESIDENT=0 in the
-// environment sends every job to the HBM schedule (same results), to compare
-// the two schedules.
+// engine, the rest in int8 HBM-schedule groups.
 bool resident_job(const JobSpec &s)
 {
-    static const bool allowed = [] {
-        const char *v = std::getenv("MCRG_BATCH_RESIDENT");
-        return !(v && std::atoi(v) == 0);
-    }();
-    return allowed && s.sampler == MCRG_SAMPLER_METROPOLIS && s.L >= kResidentMinL && s.L <= kResidentMaxL;
+    return s.sampler == MCRG_SAMPLER_METROPOLIS && s.L >= kResidentMinL && s.L <= kResidentMaxL;
+}
+// MCRG_BATCH_RESIDENT=0 in the environment sends every job of the batches that
+// are then made to the HBM schedule (same results), to compare the two.
+bool resident_allowed()
+{
+    const char *v = std::getenv("MCRG_BATCH_RESIDENT");
+    return !(v && std::atoi(v) == 0);
 }
 }  // namespace
 
@@ -116,6 +117,7 @@ mcrg_status mcrg_batch_create(mcrg_ctx ctx, const mcrg_job_desc *jobs, int32_t n
     std::vector<JobSpec> specs((size_t)n_jobs);
     size_t bytes = 0;
     int n_resident = 0, n_large = 0;
+    const bool allowed = resident_allowed();
     for (int32_t i = 0; i < n_jobs; ++i) {
         const mcrg_job_desc &d = jobs[i];
         MCRG_REQUIRE(d.n_therm >= 0 && d.n_meas >= 0, "sweep counts must be >= 0");
@@ -128,13 +130,14 @@ mcrg_status mcrg_batch_create(mcrg_ctx ctx, const mcrg_job_desc *jobs, int32_t n
         s.n_levels = d.n_levels;
         s.sweeps_per_bin = d.sweeps_per_bin;
         s.sampler = d.sampler;
-        const std::string why = resident_job(s) ? ResidentEngine::check(s) : HbmGroup::check(s);
+        const bool resident = allowed && resident_job(s);
+        const std::string why = resident ? ResidentEngine::check(s) : HbmGroup::check(s);
         if (!why.empty()) {
             set_error("job " + std::to_string(i) + ": " + why);
             return MCRG_ERR_INVALID_ARG;
         }
         specs[(size_t)i] = s;
-        if (resident_job(s)) {
+        if (resident) {
             bytes += ResidentEngine::job_bytes(s);
             ++n_resident;
             if (s.L >= eo.large_min_L) ++n_large;
@@ -178,7 +181,7 @@ mcrg_status mcrg_batch_create(mcrg_ctx ctx, const mcrg_job_desc *jobs, int32_t n
     std::vector<std::vector<int>> members;
     for (int32_t i = 0; i < n_jobs; ++i) {
         const JobSpec &s = specs[(size_t)i];
-        if (resident_job(s)) {
+        if (allowed && resident_job(s)) {
             const int id = b->engine.add(s);
             if (id < 0) {
                 set_error("batch arena exhausted");
