@@ -330,8 +330,9 @@ mcrg_status mcrg_chain_sweep(mcrg_chain ch, int32_t n_sweeps, int32_t measure)
     MCRG_REQUIRE((uint64_t)ch->t + (uint64_t)n_sweeps <= 0xFFFFFFFFull, "sweep counter overflow");
     MCRG_HIP(hipSetDevice(ch->ctx->device));
     KernelTimer *tm = ch->ctx->timer.enabled ? &ch->ctx->timer : nullptr;
-    if (!chain_on_chip(d.L, d.sampler == MCRG_SAMPLER_METROPOLIS) &&
-        n_sweeps > launched_singly(d.L, measure != 0) && ch->strip.usable(ch->host, measure != 0))
+    const bool strips = strip_forced() || (!chain_on_chip(d.L, d.sampler == MCRG_SAMPLER_METROPOLIS) &&
+                                           n_sweeps > launched_singly(d.L, measure != 0));
+    if (strips && ch->strip.usable(ch->host, measure != 0))
         MCRG_HIP(ch->strip.run(ch->d_desc, ch->host, ch->t, ch->n_measured, (uint32_t)n_sweeps, measure != 0,
                                ch->stream, tm));
     else

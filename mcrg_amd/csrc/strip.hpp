@@ -215,7 +215,10 @@ uint32_t *static_scratch(int device);
 // Metropolis sampler, 64 <= L <= 8192 (L = 16384 for unmeasured sweeps, whose
 // strips alone fill the LDS), and every workgroup of the launch resident at
 // once.  Owns the launch workspace.  MCRG_STRIP=0 in the environment keeps
-// every chain on the per-half-sweep HBM schedule (same results).
+// every chain off the strips, MCRG_STRIP=1 puts every sweep call on them whose
+// shape they take, however short (strip_forced; same results), to compare the
+// schedules.
+bool strip_forced();
 class StripRunner {
   public:
     StripRunner() = default;

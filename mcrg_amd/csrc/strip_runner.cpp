@@ -54,6 +54,12 @@ static bool strip_enabled()
     return !(v && std::strcmp(v, "0") == 0);
 }
 
+bool strip_forced()
+{
+    const char *v = std::getenv("MCRG_STRIP");
+    return v && std::strcmp(v, "1") == 0;
+}
+
 bool StripRunner::plan(const HbmLattice &h, bool measure, StripShape &sh, int &threads, size_t max_words)
 {
     if (h.sampler != MCRG_SAMPLER_METROPOLIS || !strip_enabled()) return false;

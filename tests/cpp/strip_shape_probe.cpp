@@ -1,6 +1,7 @@
 // Prints the strip schedule's launch shape (mcrg::strip_shape) for each line
-// "L nl n_wg n_tail measure halo_ok split_ok" read on stdin, one line of
-// "name=value" fields per shape, for tests/test_strip_shape_cpu.py.
+// "L nl n_wg n_tail measure halo_ok split_ok [sides]" read on stdin, one line of
+// "name=value" fields per shape, for tests/test_strip_shape_cpu.py and
+// tests/test_strip_sides_cpu.py.
 #include <cstdio>
 
 #include "../../mcrg_amd/csrc/strip.hpp"
@@ -11,9 +12,15 @@ int main()
                 "kStripCntWords=%u kRedWords=%u kStaticScratchWords=%zu kStripFlagStride=%u\n",
                 mcrg::kStripRing, mcrg::kStripSnapSlots, mcrg::kStripFirstSlots, mcrg::kStripFirstSlotsSplit,
                 mcrg::kStripCntWords, mcrg::kRedWords, mcrg::kStaticScratchWords, mcrg::kStripFlagStride);
-    unsigned L, nl, n_wg, n_tail, measure, halo_ok, split_ok;
-    while (std::scanf("%u %u %u %u %u %u %u", &L, &nl, &n_wg, &n_tail, &measure, &halo_ok, &split_ok) == 7) {
-        const mcrg::StripShape s = mcrg::strip_shape(L, nl, n_wg, n_tail, measure != 0, halo_ok != 0, split_ok != 0);
+    char line[256];
+    unsigned L, nl, n_wg, n_tail, measure, halo_ok, split_ok, sides;
+    while (std::fgets(line, sizeof(line), stdin)) {
+        sides = 1;
+        if (std::sscanf(line, "%u %u %u %u %u %u %u %u", &L, &nl, &n_wg, &n_tail, &measure, &halo_ok, &split_ok,
+                        &sides) < 7)
+            break;
+        const mcrg::StripShape s =
+            mcrg::strip_shape(L, nl, n_wg, n_tail, measure != 0, halo_ok != 0, split_ok != 0, sides);
         std::printf("shape L=%u nl=%u n_wg=%u R=%u wpr=%u lam=%u n_tail=%u measure=%u threads=%u overlap=%u halo=%u "
                     "split=%u n_meas=%u snap_words=%u first_slots=%u o_err=%u o_consumed=%u o_xhalo=%u "
                     "o_xfirst=%u o_ring=%u o_snapc=%u o_snap=%u ws_words=%u cnt_words=%u first_words=%u "
