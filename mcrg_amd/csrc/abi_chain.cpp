@@ -102,16 +102,21 @@ struct mcrg_chain_s {
     int line = -1;
 };
 
-// Fails when a strip launch since the last check gave up on a wait.
-static mcrg_status check_strip(mcrg_chain ch)
+static mcrg_status strip_status(bool bad)
 {
-    bool bad = false;
-    MCRG_HIP(ch->strip.failed(ch->stream, bad));
     if (bad) {
         set_error("strip launch: a workgroup's wait for its neighbours exceeded the limit; the chain state is lost");
         return MCRG_ERR_DEVICE;
     }
     return MCRG_OK;
+}
+
+// Fails when a strip launch since the last check gave up on a wait.
+static mcrg_status check_strip(mcrg_chain ch)
+{
+    bool bad = false;
+    MCRG_HIP(ch->strip.failed(ch->stream, bad));
+    return strip_status(bad);
 }
 
 extern "C" {
@@ -446,17 +451,23 @@ mcrg_status mcrg_chain_operators(mcrg_chain ch, int64_t out[4])
     MCRG_REQUIRE(ch != nullptr && out != nullptr, "null argument");
     MCRG_HIP(hipSetDevice(ch->ctx->device));
     hipStream_t s = ch->stream;
-    unsigned long long cnt[4];
+    unsigned long long cnt[kOperatorWords];
+    // the strips' error word comes with the counts: no copy and wait of its own
+    const uint32_t *error = ch->strip.error_word();
+    static_assert(kOperatorWords <= ResultLines::kWords, "a chain's line");
     if (ch->line >= 0) {
         unsigned long long *line = ch->lines->base + ch->line * ResultLines::kWords;
-        MCRG_HIP(launch_int8_operators(ch->d_desc, ch->desc.L, line, s));
+        MCRG_HIP(launch_int8_operators(ch->d_desc, ch->desc.L, error, line, s));
         MCRG_HIP(hipStreamSynchronize(s));
         std::memcpy(cnt, line, sizeof(cnt));
     } else {
-        MCRG_HIP(launch_int8_operators(ch->d_desc, ch->desc.L, ch->host.sums + kSumOut, s));
+        MCRG_HIP(launch_int8_operators(ch->d_desc, ch->desc.L, error, ch->host.sums + kSumOut, s));
         MCRG_HIP(hipMemcpyAsync(cnt, ch->host.sums + kSumOut, sizeof(cnt), hipMemcpyDeviceToHost, s));
         MCRG_HIP(hipStreamSynchronize(s));
     }
+    if (error) ch->strip.reported();
+    const mcrg_status st = strip_status(cnt[4] != 0u);
+    if (st != MCRG_OK) return st;
     const int64_t n0 = (int64_t)ch->desc.L * ch->desc.L;
     out[0] = 2 * n0 - 2 * (int64_t)cnt[0];
     out[1] = 2 * n0 - 2 * (int64_t)cnt[1];

@@ -276,6 +276,7 @@ static uint32_t operators_rows(uint32_t L)
 // Bound by the launch and the host's wait for it below L = 4096, and by memory
 // above (L = 16384 reads 268 MB).
 __global__ __launch_bounds__(1024) void k_int8_operators(const HbmLattice *__restrict__ lats, uint32_t rows,
+                                                         const uint32_t *__restrict__ error,
                                                          unsigned long long *__restrict__ out)
 {
     __shared__ uint32_t sum[4], last;
@@ -355,9 +356,10 @@ __global__ __launch_bounds__(1024) void k_int8_operators(const HbmLattice *__res
         add();
         if (threadIdx.x == 0u) lat.sums[kSumTicket] = 0ull;
     }
-    if (threadIdx.x < 4u)
-        __hip_atomic_store(out + threadIdx.x, (unsigned long long)sum[threadIdx.x], __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x < kOperatorWords)
+        __hip_atomic_store(out + threadIdx.x,
+                           (unsigned long long)(threadIdx.x < 4u ? sum[threadIdx.x] : error ? *error : 0u),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------- levels >= 1
@@ -502,12 +504,13 @@ hipError_t launch_int8_half_sweep(const HbmLattice *d, int n_lats, int L, uint32
     return hipGetLastError();
 }
 
-hipError_t launch_int8_operators(const HbmLattice *d, int L, unsigned long long *out, hipStream_t s)
+hipError_t launch_int8_operators(const HbmLattice *d, int L, const uint32_t *error, unsigned long long *out,
+                                 hipStream_t s)
 {
     const uint32_t rows = operators_rows((uint32_t)L), n = (uint32_t)L;
     const uint32_t n_items = n >= 16u ? n / rows * (n / 16u) : n * n;
     const uint32_t threads = n_items >= 1024u ? 1024u : 256u;  // 256: one workgroup
-    hipLaunchKernelGGL(k_int8_operators, dim3(cdiv(n_items, threads)), dim3(threads), 0, s, d, rows, out);
+    hipLaunchKernelGGL(k_int8_operators, dim3(cdiv(n_items, threads)), dim3(threads), 0, s, d, rows, error, out);
     return hipGetLastError();
 }
 

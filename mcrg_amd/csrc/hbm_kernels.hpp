@@ -20,7 +20,8 @@ constexpr uint32_t kWgLevelMaxL = kGridLevelMinL / 2;
 // every grid-measured level l >= 1 at 4 + 3 (l - 1).
 constexpr uint32_t kSumWords = 4u + 3u * kMaxLevels;
 // behind them: k_int8_operators' count of finished workgroups and its results
-constexpr uint32_t kSumTicket = kSumWords, kSumOut = kSumWords + 1u, kSumAlloc = kSumWords + 5u;
+constexpr uint32_t kOperatorWords = 5u;
+constexpr uint32_t kSumTicket = kSumWords, kSumOut = kSumWords + 1u, kSumAlloc = kSumOut + kOperatorWords;
 
 // Rows per thread strip of the int8 half-sweep (L >= 64).  Up to L = 8192 the
 // lattice (<= 64 MiB) stays in the 256 MB last-level cache, so each row's three
@@ -142,9 +143,11 @@ inline bool chain_on_chip(int L, bool metropolis)
 }
 hipError_t launch_int8_half_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
                                   uint32_t colour, hipStream_t s);
-// Level-0 disagreement counts of one lattice (as k_int8_measure0's) into out[0..3]:
+// Level-0 disagreement counts of one lattice (as k_int8_measure0's) into out[0..3]
+// and the word at `error` (0 without one) into out[4]: kOperatorWords words of
 // device memory or mapped host memory.
-hipError_t launch_int8_operators(const HbmLattice *d, int L, unsigned long long *out, hipStream_t s);
+hipError_t launch_int8_operators(const HbmLattice *d, int L, const uint32_t *error, unsigned long long *out,
+                                 hipStream_t s);
 hipError_t launch_int8_measure0(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
                                 hipStream_t s);
 // Levels 1..nl (grid launches for the large ones, then one workgroup per

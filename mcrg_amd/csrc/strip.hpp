@@ -35,8 +35,11 @@ namespace mcrg {
 constexpr uint32_t kStripRing = 8;         // per-sample slots between strips and tails
 constexpr uint32_t kStripFlagStride = 32;  // words between polled words (128 B lines)
 constexpr uint32_t kStripCntWords = 64;    // per-slot operator counts, 4 per level
-// A wait gives up (and sets the error word) after 2 s of the 100 MHz clock.
-constexpr uint64_t kStripWaitTicks = 200000000ull;
+// A wait gives up (and sets the error word) after the ticks of the 100 MHz clock
+// that stand behind the error word: 2 s, or MCRG_STRIP_WAIT_TICKS of the
+// environment, with which tests of the error path make waits give up.
+constexpr uint32_t kStripWaitTicks = 200000000u;
+constexpr uint32_t kStripLimitWord = 1u;  // from the error word on
 constexpr uint32_t kStripMaxWg = 256;
 // Slots per strip of a sample's first blocked rows with halo rows: they are
 // read a sweep after they are sent, while the sender may already send the
@@ -71,7 +74,7 @@ struct StripShape {
     uint32_t split, n_meas, snap_words, first_slots;
     // device workspace, offsets in 32-bit words (even where 64-bit words
     // start), all of it cleared per launch:
-    //   o_err       error word
+    //   o_err       error word, then the ticks after which a wait gives up
     //   o_consumed  per slot: samples the tails have finished with it
     //   o_xhalo     (data, seq) words: [colour][strip][first, last row][wpr],
     //               with halo [sweep parity][strip][first two, last two rows][wpr]
@@ -182,6 +185,7 @@ struct StripArgs {
     uint32_t n_sweeps;
     uint32_t strip_sleep;   // polls of a waiting strip thread are 64 x this many clocks apart
     uint32_t tail_sleep;    // the same for tail threads
+    uint32_t wait_ticks;    // a wait gives up after this many
 };
 
 // Clears the workspace, then runs n_sweeps sweeps (all measured when
@@ -236,6 +240,11 @@ class StripRunner {
     // After the stream has drained: true when a launch since the last call
     // gave up on a wait (its error word is set, then cleared here).
     hipError_t failed(hipStream_t s, bool &out);
+    // The error word that failed() would read (device memory), or null; for a
+    // kernel that reports it beside its own results.  reported() then takes
+    // failed()'s place.
+    const uint32_t *error_word() const { return launched_ ? last_ws_ : nullptr; }
+    void reported() { launched_ = false; }
 
   private:
     // The launch shape; max_words > 0 drops the measuring workgroups when

@@ -1,6 +1,6 @@
 // Strip schedule kernels (see strip.hpp for the structure).
 //
-//   k_strip_reset   clears a launch's workspace
+//   k_strip_reset   clears a launch's workspace, but for the limit of its waits
 //   k_strip         cooperative launch: workgroups 0 .. n_wg-1 each own a strip
 //                   of R rows held bit-packed in LDS and run every sweep of the
 //                   launch on it (checkerboard Metropolis replacing the Wolff
@@ -43,7 +43,7 @@ __device__ __forceinline__ uint64_t ll_peek(const uint64_t *p)
 
 // Polls *p until its sequence is `seq` and returns the word.  Gives up (the
 // returned word's sequence is then not `seq`) once the launch's error word is
-// set, by this thread after kStripWaitTicks of the 100 MHz clock or by any
+// set, by this thread after the limit (strip.hpp) or by any
 // other, so that every workgroup reaches the end of the kernel.  Not inlined:
 // the slow path stays out of the sweep's registers.
 __device__ __noinline__ uint64_t ll_wait(const uint64_t *p, uint32_t seq, uint32_t *err, uint32_t sleep)
@@ -54,7 +54,7 @@ __device__ __noinline__ uint64_t ll_wait(const uint64_t *p, uint32_t seq, uint32
         if ((uint32_t)(v >> 32) == seq) return v;
         if ((k & 7u) == 0u) {
             if (ld_relaxed(err) != 0u) return 0;
-            if ((uint64_t)wall_clock64() - t0 > kStripWaitTicks) {
+            if ((uint64_t)wall_clock64() - t0 > ld_relaxed(err + kStripLimitWord)) {
                 __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return 0;
             }
@@ -84,7 +84,7 @@ __device__ __noinline__ bool flag_wait(const uint32_t *flag, uint32_t want, uint
     while (ld_relaxed(flag) < want) {
         if (ld_relaxed(err) != 0u) return false;
         __builtin_amdgcn_s_sleep(1);
-        if ((uint64_t)wall_clock64() - t0 > kStripWaitTicks) {
+        if ((uint64_t)wall_clock64() - t0 > ld_relaxed(err + kStripLimitWord)) {
             __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return false;
         }
@@ -150,9 +150,10 @@ __device__ __forceinline__ void store64b(int8_t *p, uint32_t e, uint32_t o)
     }
 }
 
-__global__ void k_strip_reset(uint32_t *ws, uint32_t n)
+__global__ void k_strip_reset(uint32_t *ws, uint32_t n, uint32_t limit_at, uint32_t limit)
 {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) ws[i] = 0u;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        ws[i] = i == limit_at ? limit : 0u;
 }
 
 // Level-0 operator counts of one checkerboard word: colour c, local row r
@@ -1105,7 +1106,8 @@ static hipError_t launch_nt(const StripArgs &a, hipStream_t s)
 hipError_t launch_strip(const StripArgs &a, int threads, hipStream_t s)
 {
     const uint32_t blocks = std::min<uint32_t>(1024u, (a.sh.ws_words + 255u) / 256u);
-    hipLaunchKernelGGL(k_strip_reset, dim3(blocks), dim3(256), 0, s, a.ws, a.sh.ws_words);
+    hipLaunchKernelGGL(k_strip_reset, dim3(blocks), dim3(256), 0, s, a.ws, a.sh.ws_words,
+                       a.sh.o_err + kStripLimitWord, a.wait_ticks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     switch (threads) {

@@ -151,8 +151,11 @@ hipError_t StripRunner::run(const HbmLattice *d, const HbmLattice &h, uint32_t t
     a.n_sweeps = n;
     a.strip_sleep = 1;
     a.tail_sleep = 8;
+    a.wait_ticks = kStripWaitTicks;
     if (const char *v = std::getenv("MCRG_STRIP_SLEEP")) a.strip_sleep = (uint32_t)std::max(1, std::atoi(v));
     if (const char *v = std::getenv("MCRG_TAIL_SLEEP")) a.tail_sleep = (uint32_t)std::max(1, std::atoi(v));
+    if (const char *v = std::getenv("MCRG_STRIP_WAIT_TICKS"))
+        a.wait_ticks = (uint32_t)std::min<long>(std::max(0L, std::atol(v)), kStripWaitTicks);
     const int ev = tm ? tm->begin(kKindStrip, s) : -1;
     if ((e = launch_strip(a, threads, s)) != hipSuccess) return e;
     if (tm) tm->end(ev, s);
