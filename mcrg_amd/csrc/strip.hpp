@@ -186,6 +186,7 @@ struct StripArgs {
     uint32_t strip_sleep;   // polls of a waiting strip thread are 64 x this many clocks apart
     uint32_t tail_sleep;    // the same for tail threads
     uint32_t wait_ticks;    // a wait gives up after this many
+    uint32_t keep_err;      // nonzero: the error word stands for earlier launches too
 };
 
 // Clears the workspace, then runs n_sweeps sweeps (all measured when
@@ -238,7 +239,7 @@ class StripRunner {
     hipError_t run(const HbmLattice *d, const HbmLattice &h, uint32_t t0, uint32_t q0, uint32_t n, bool measure,
                    hipStream_t s, KernelTimer *tm, uint32_t *fixed_ws = nullptr, size_t fixed_words = 0);
     // After the stream has drained: true when a launch since the last call
-    // gave up on a wait (its error word is set, then cleared here).
+    // gave up on a wait.
     hipError_t failed(hipStream_t s, bool &out);
     // The error word that failed() would read (device memory), or null; for a
     // kernel that reports it beside its own results.  reported() then takes

@@ -1,6 +1,7 @@
 // Strip schedule kernels (see strip.hpp for the structure).
 //
-//   k_strip_reset   clears a launch's workspace, but for the limit of its waits
+//   k_strip_reset   clears a launch's workspace, but for the limit of its waits and
+//                   an error of the chain's earlier launches that was not reported
 //   k_strip         cooperative launch: workgroups 0 .. n_wg-1 each own a strip
 //                   of R rows held bit-packed in LDS and run every sweep of the
 //                   launch on it (checkerboard Metropolis replacing the Wolff
@@ -150,10 +151,10 @@ __device__ __forceinline__ void store64b(int8_t *p, uint32_t e, uint32_t o)
     }
 }
 
-__global__ void k_strip_reset(uint32_t *ws, uint32_t n, uint32_t limit_at, uint32_t limit)
+__global__ void k_strip_reset(uint32_t *ws, uint32_t n, uint32_t err_at, uint32_t keep_err, uint32_t limit)
 {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        ws[i] = i == limit_at ? limit : 0u;
+        if (i != err_at || !keep_err) ws[i] = i == err_at + kStripLimitWord ? limit : 0u;
 }
 
 // Level-0 operator counts of one checkerboard word: colour c, local row r
@@ -1106,8 +1107,8 @@ static hipError_t launch_nt(const StripArgs &a, hipStream_t s)
 hipError_t launch_strip(const StripArgs &a, int threads, hipStream_t s)
 {
     const uint32_t blocks = std::min<uint32_t>(1024u, (a.sh.ws_words + 255u) / 256u);
-    hipLaunchKernelGGL(k_strip_reset, dim3(blocks), dim3(256), 0, s, a.ws, a.sh.ws_words,
-                       a.sh.o_err + kStripLimitWord, a.wait_ticks);
+    hipLaunchKernelGGL(k_strip_reset, dim3(blocks), dim3(256), 0, s, a.ws, a.sh.ws_words, a.sh.o_err,
+                       a.keep_err, a.wait_ticks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     switch (threads) {

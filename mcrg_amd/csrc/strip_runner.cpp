@@ -133,11 +133,15 @@ hipError_t StripRunner::run(const HbmLattice *d, const HbmLattice &h, uint32_t t
         if (a.sh.ws_words > fixed_words) return hipErrorInvalidValue;
         a.ws = fixed_ws;
     } else if (a.sh.ws_words > ws_words_) {
-        // the stream may still run a launch that uses the old workspace
+        // the stream may still run a launch that uses the old workspace, and
+        // its error word goes with it
         if (ws_) {
-            if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+            bool bad = false;
+            if ((e = hipStreamSynchronize(s)) != hipSuccess || (e = failed(s, bad)) != hipSuccess) return e;
+            if (bad) return hipErrorLaunchFailure;
             (void)hipFree(ws_);
             ws_ = nullptr;
+            ws_words_ = 0;
         }
         void *p = nullptr;
         if ((e = hipMalloc(&p, (size_t)a.sh.ws_words * 4u)) != hipSuccess) return e;
@@ -152,6 +156,8 @@ hipError_t StripRunner::run(const HbmLattice *d, const HbmLattice &h, uint32_t t
     a.strip_sleep = 1;
     a.tail_sleep = 8;
     a.wait_ticks = kStripWaitTicks;
+    // not in an array that other chains use too
+    a.keep_err = launched_ && !fixed_ws && last_ws_ == a.ws ? 1u : 0u;
     if (const char *v = std::getenv("MCRG_STRIP_SLEEP")) a.strip_sleep = (uint32_t)std::max(1, std::atoi(v));
     if (const char *v = std::getenv("MCRG_TAIL_SLEEP")) a.tail_sleep = (uint32_t)std::max(1, std::atoi(v));
     if (const char *v = std::getenv("MCRG_STRIP_WAIT_TICKS"))
@@ -181,7 +187,7 @@ hipError_t StripRunner::failed(hipStream_t s, bool &out)
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
     launched_ = false;
     out = err != 0u;
-    return hipSuccess;  // the next launch clears the word
+    return hipSuccess;  // reported: the next launch clears the word
 }
 
 }  // namespace mcrg

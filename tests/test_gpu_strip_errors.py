@@ -45,3 +45,21 @@ def test_lost_state_is_reported(amd, ctx, orc, monkeypatch, reader, lines):
     finally:
         for c in others:
             c.close()
+
+
+@pytest.mark.parametrize("then", ["same", "larger"])
+def test_a_later_launch_does_not_hide_it(amd, ctx, monkeypatch, then):
+    """An error that nobody has asked about yet outlives the next launch, in the
+    same workspace or in a larger one."""
+    print("strip error, then", then, flush=True)
+    with amd.Chain(ctx, 1024, 0.44, seed=3, n_levels=3, sweeps_per_bin=1000) as ch:
+        monkeypatch.setenv("MCRG_STRIP_WAIT_TICKS", "0")
+        if then == "larger":
+            monkeypatch.setenv("MCRG_STRIP_WG", "8")
+        ch.sweep(400, measure=True)
+        monkeypatch.delenv("MCRG_STRIP_WAIT_TICKS")
+        monkeypatch.delenv("MCRG_STRIP_WG", raising=False)
+        with pytest.raises(amd.MCRGError) as e:
+            ch.sweep(50, measure=True)
+            ch.sync()
+        assert e.value.status == amd.ERR_DEVICE
