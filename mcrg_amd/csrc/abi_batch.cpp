@@ -204,7 +204,7 @@ mcrg_status mcrg_batch_create(mcrg_ctx ctx, const mcrg_job_desc *jobs, int32_t n
         std::vector<JobSpec> ms;
         for (int i : m) ms.push_back(specs[(size_t)i]);
         b->groups.emplace_back(new HbmGroup());
-        if ((e = b->groups.back()->init(ms, b->hbm_stream, ctx->arenas.get())) != hipSuccess) return fail(e, "batch HBM group");
+        if ((e = b->groups.back()->init(ms, b->hbm_stream)) != hipSuccess) return fail(e, "batch HBM group");
     }
     if ((e = b->engine.flush_pending()) != hipSuccess) return fail(e, "batch init");
     if (opts && opts->autotune && n_resident > 0) b->engine.enable_autotune();

@@ -173,7 +173,7 @@ mcrg_status mcrg_ctx_create(int32_t device, mcrg_ctx *out)
     (void)static_scratch_setup(device);
     try {
         c->lines = std::make_shared<ResultLines>();
-        c->arenas = std::make_shared<ArenaPool>();
+        c->arenas = std::make_shared<ArenaPool>(device);
     } catch (const std::bad_alloc &) {  // results are copied, arenas freed
     }
     *out = c;
@@ -250,7 +250,7 @@ mcrg_status mcrg_chain_create(mcrg_ctx ctx, const mcrg_chain_desc *desc, mcrg_ch
     const HbmBlock blk = hbm_block(d.L, d.n_levels, d.max_bins, d.sampler);
     const size_t o_desc = blk.bytes;
     const size_t total = align256(o_desc + sizeof(HbmLattice));
-    hipError_t e = device_malloc(&ch->d_block, total, ctx->arenas.get());
+    hipError_t e = device_malloc(&ch->d_block, total);
     if (e != hipSuccess) {
         delete ch;
         set_error(std::string("hipMalloc: ") + hipGetErrorString(e));

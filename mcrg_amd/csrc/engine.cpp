@@ -21,7 +21,7 @@ hipError_t Arena::init(size_t bytes, std::shared_ptr<ArenaPool> pool, bool keep)
     keep_ = keep && pool_ != nullptr;
     void *p = keep_ ? pool_->take(cap_) : nullptr;
     if (!p) {
-        hipError_t e = device_malloc(&p, cap_, pool_.get());
+        hipError_t e = device_malloc(&p, cap_);
         if (e != hipSuccess) {
             cap_ = 0;
             return e;
@@ -155,13 +155,13 @@ hipError_t ResidentEngine::init(int device, size_t arena_bytes, int capacity, co
     capacity_ = capacity;
     hipError_t e;
     if ((e = arena_.init(arena_bytes, std::move(pool), keep)) != hipSuccess) return e;
-    if ((e = hipMalloc(&d_lats_, sizeof(PackedLattice) * (size_t)capacity)) != hipSuccess) return e;
-    if ((e = hipMalloc(&d_queue_, 64u * kMaxClasses)) != hipSuccess) return e;
-    if ((e = hipMalloc(&d_err_, sizeof(uint32_t))) != hipSuccess) return e;
+    if ((e = device_malloc(&d_lats_, sizeof(PackedLattice) * (size_t)capacity)) != hipSuccess) return e;
+    if ((e = device_malloc(&d_queue_, 64u * kMaxClasses)) != hipSuccess) return e;
+    if ((e = device_malloc(&d_err_, sizeof(uint32_t))) != hipSuccess) return e;
     if ((e = hipMemset(d_err_, 0, sizeof(uint32_t))) != hipSuccess) return e;
     if ((e = hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, device)) != hipSuccess) return e;
-    if ((e = hipMalloc(&d_init_idx_, sizeof(int32_t) * (size_t)capacity)) != hipSuccess) return e;
-    if ((e = hipMalloc(&d_stage_, sizeof(PackedLattice) * (size_t)capacity)) != hipSuccess) return e;
+    if ((e = device_malloc(&d_init_idx_, sizeof(int32_t) * (size_t)capacity)) != hipSuccess) return e;
+    if ((e = device_malloc(&d_stage_, sizeof(PackedLattice) * (size_t)capacity)) != hipSuccess) return e;
     for (hipStream_t &a : aux_)
         if ((e = hipStreamCreateWithFlags(&a, hipStreamNonBlocking)) != hipSuccess) return e;
     if ((e = hipEventCreateWithFlags(&ev_fork_, hipEventDisableTiming)) != hipSuccess) return e;
@@ -517,16 +517,8 @@ hipError_t ResidentEngine::upload_slots()
     // still read: only then does the host wait for the stream.
     if (slots_.size() > slot_cap_ || slot_lats_.size() > slot_lat_cap_ || slots_.size() > done_cap_)
         if ((e = hipStreamSynchronize(stream_)) != hipSuccess) return e;
-    if (slots_.size() > slot_cap_) {
-        if (d_slots_) (void)hipFree(d_slots_);
-        slot_cap_ = std::max<size_t>(slots_.size(), 2 * slot_cap_);
-        if ((e = hipMalloc(&d_slots_, sizeof(Slot) * slot_cap_)) != hipSuccess) return e;
-    }
-    if (slot_lats_.size() > slot_lat_cap_) {
-        if (d_slot_lats_) (void)hipFree(d_slot_lats_);
-        slot_lat_cap_ = std::max<size_t>(slot_lats_.size(), 2 * slot_lat_cap_);
-        if ((e = hipMalloc(&d_slot_lats_, sizeof(int32_t) * slot_lat_cap_)) != hipSuccess) return e;
-    }
+    if ((e = device_regrow(d_slots_, slot_cap_, slots_.size())) != hipSuccess) return e;
+    if ((e = device_regrow(d_slot_lats_, slot_lat_cap_, slot_lats_.size())) != hipSuccess) return e;
     if (!slots_.empty()) {
         // copies on the stream, after the launches that read the old tables,
         // from pinned staging used in turn
@@ -543,11 +535,7 @@ hipError_t ResidentEngine::upload_slots()
             return e;
         if ((e = slot_stage_.used(stream_)) != hipSuccess) return e;
     }
-    if (slots_.size() > done_cap_) {
-        if (d_done_) (void)hipFree(d_done_);
-        done_cap_ = std::max<size_t>(slots_.size(), 2 * done_cap_);
-        if ((e = hipMalloc(&d_done_, sizeof(uint32_t) * done_cap_)) != hipSuccess) return e;
-    }
+    if ((e = device_regrow(d_done_, done_cap_, slots_.size())) != hipSuccess) return e;
     for (LaunchClass &lc : classes_) {
         if (lc.small) continue;  // one workgroup per slot, no parts
         const int resident = resident_max_active_groups(lc.threads, lc.lds);

@@ -177,7 +177,7 @@ std::string HbmGroup::check(const JobSpec &j)
     return std::string();
 }
 
-hipError_t HbmGroup::init(const std::vector<JobSpec> &members, hipStream_t s, ArenaPool *pool)
+hipError_t HbmGroup::init(const std::vector<JobSpec> &members, hipStream_t s)
 {
     members_ = members;
     const JobSpec &j = members_[0];
@@ -190,7 +190,7 @@ hipError_t HbmGroup::init(const std::vector<JobSpec> &members, hipStream_t s, Ar
     const size_t desc_off = blk_.bytes * n;
     hipError_t e;
     void *p = nullptr;
-    if ((e = device_malloc(&p, desc_off + sizeof(HbmLattice) * n, pool)) != hipSuccess) return e;
+    if ((e = device_malloc(&p, desc_off + sizeof(HbmLattice) * n)) != hipSuccess) return e;
     d_block_ = static_cast<char *>(p);
     d_desc_ = reinterpret_cast<HbmLattice *>(d_block_ + desc_off);
     host_.resize(n);

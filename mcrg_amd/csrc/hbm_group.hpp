@@ -59,7 +59,7 @@ class HbmGroup {
     // Same-shaped jobs (L, n_levels, n_therm, n_meas, sweeps_per_bin, sampler equal).
     static bool same_shape(const JobSpec &a, const JobSpec &b);
     static std::string check(const JobSpec &j);
-    hipError_t init(const std::vector<JobSpec> &members, hipStream_t s, ArenaPool *pool);
+    hipError_t init(const std::vector<JobSpec> &members, hipStream_t s);
     // Advances every member by min(n, remaining) sweeps (asynchronous).
     hipError_t advance(uint32_t n, hipStream_t s, KernelTimer *tm);
     uint32_t remaining() const { return therm_left_ + meas_left_; }

@@ -9,6 +9,8 @@
 #include <string>
 #include <vector>
 
+#include "arena_pool.hpp"
+
 #include "../../include/mcrg_abi.h"
 #include "hbm_kernels.hpp"
 
@@ -106,61 +108,6 @@ struct ResultLines {
         if (k >= 0) used &= ~(1ull << k);
     }
 };
-
-// The job arena of the last server that was destroyed, for the next one of the
-// same size: device memory that is freed has to be cleared by the driver (about
-// 100 ms for 4 GiB) before it can be allocated again, and once all of the
-// device's memory has been through a process's hands every new arena waits for
-// that.  At most one arena of at most kMaxBytes; it is freed when another
-// allocation of the library finds no memory, and with the context and the last
-// of its servers.
-struct ArenaPool {
-    static constexpr size_t kMaxBytes = size_t(4) << 30;
-    void *take(size_t bytes)
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        if (!base_ || bytes_ != bytes) return nullptr;
-        void *p = base_;
-        base_ = nullptr;
-        return p;
-    }
-    // False when the caller has to free it.
-    bool give(void *base, size_t bytes)
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        if (base_ || bytes > kMaxBytes) return false;
-        base_ = base;
-        bytes_ = bytes;
-        return true;
-    }
-    bool drop()
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        if (!base_) return false;
-        (void)hipFree(base_);
-        base_ = nullptr;
-        return true;
-    }
-    ArenaPool() = default;
-    ~ArenaPool() { (void)drop(); }
-    ArenaPool(const ArenaPool &) = delete;
-    ArenaPool &operator=(const ArenaPool &) = delete;
-
-  private:
-    std::mutex mu_;
-    void *base_ = nullptr;
-    size_t bytes_ = 0;
-};
-
-inline hipError_t device_malloc(void **p, size_t bytes, ArenaPool *pool)
-{
-    hipError_t e = hipMalloc(p, bytes);
-    if (e == hipErrorOutOfMemory && pool && pool->drop()) {
-        (void)hipGetLastError();
-        e = hipMalloc(p, bytes);
-    }
-    return e;
-}
 
 }  // namespace mcrg
 

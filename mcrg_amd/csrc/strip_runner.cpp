@@ -143,9 +143,7 @@ hipError_t StripRunner::run(const HbmLattice *d, const HbmLattice &h, uint32_t t
             ws_ = nullptr;
             ws_words_ = 0;
         }
-        void *p = nullptr;
-        if ((e = hipMalloc(&p, (size_t)a.sh.ws_words * 4u)) != hipSuccess) return e;
-        ws_ = static_cast<uint32_t *>(p);
+        if ((e = device_malloc(&ws_, (size_t)a.sh.ws_words * 4u)) != hipSuccess) return e;
         ws_words_ = a.sh.ws_words;
     }
     if (!fixed_ws) a.ws = ws_;
