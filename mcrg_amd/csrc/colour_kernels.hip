@@ -1,6 +1,7 @@
 // int8 chains of L = 64 and 128 in one workgroup, its waves split by colour:
 // Metropolis sweeps (replacing src/ising.cpp:87-149) and the measurement of
 // every level (src/lattice.cpp:102-120, src/mcrg.cpp:72-98, :314-348).
+#include "lds_opt_in.hpp"
 #include "wave_core.hpp"
 
 namespace mcrg {
@@ -172,20 +173,24 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
     }
 }
 
+template <uint32_t L>
+static hipError_t launch_colour(const HbmLattice *d, int n_lats, int n_levels, uint32_t n, bool measure, hipStream_t s)
+{
+    const uint32_t lds_bytes = 4u * colour_lds_words<L>((uint32_t)n_levels);  // L = 128: up to 72,992 bytes
+    static LdsOptIn lds;
+    const hipError_t le = lds.need(reinterpret_cast<const void *>(&k_colour_chain<L>), lds_bytes);
+    if (le != hipSuccess) return le;
+    hipLaunchKernelGGL(k_colour_chain<L>, dim3((uint32_t)n_lats), dim3(ColourGeom<L>::threads), lds_bytes, s, d, n,
+                       measure ? 1u : 0u);
+    return hipGetLastError();
+}
+
 hipError_t launch_colour_chain(const HbmLattice *d, int n_lats, int L, int n_levels, uint32_t n, bool measure,
                                hipStream_t s)
 {
-    const dim3 grid((uint32_t)n_lats);
-    const uint32_t m = measure ? 1u : 0u;
-    if (L == 64)
-        hipLaunchKernelGGL(k_colour_chain<64u>, grid, dim3(ColourGeom<64u>::threads),
-                           4u * colour_lds_words<64u>((uint32_t)n_levels), s, d, n, m);
-    else if (L == 128)
-        hipLaunchKernelGGL(k_colour_chain<128u>, grid, dim3(ColourGeom<128u>::threads),
-                           4u * colour_lds_words<128u>((uint32_t)n_levels), s, d, n, m);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
+    if (L == 64) return launch_colour<64u>(d, n_lats, n_levels, n, measure, s);
+    if (L == 128) return launch_colour<128u>(d, n_lats, n_levels, n, measure, s);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace mcrg

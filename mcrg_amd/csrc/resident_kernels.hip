@@ -11,8 +11,8 @@
 //                   Metropolis; src/lattice.cpp:102-120, src/mcrg.cpp:72-98 and
 //                   :314-348 fused)
 //   k_reset_queue   zeroes a launch's work counter and per-slot progress words
-#include <mutex>
 
+#include "lds_opt_in.hpp"
 #include "resident_body.hpp"
 
 namespace mcrg {
@@ -145,20 +145,9 @@ static hipError_t launch_nt(const Slot *slots, uint32_t n_slots, uint32_t n_sub,
                             PackedLattice *lats, uint32_t *queue, uint32_t *done, uint32_t *err,
                             uint32_t lds_bytes, uint32_t grid, hipStream_t s)
 {
-    // Above 64 KiB of dynamic LDS the kernel has to be opted in.  Batches and
-    // servers may launch from different threads: the level only ever rises,
-    // under a lock, so a launch never finds it lowered by another.
-    static std::mutex mu;
-    static uint32_t opted_in = 65536u;
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        if (lds_bytes > opted_in) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_resident<NT>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-            if (e != hipSuccess) return e;
-            opted_in = lds_bytes;
-        }
-    }
+    static LdsOptIn lds;
+    const hipError_t le = lds.need(reinterpret_cast<const void *>(&k_resident<NT>), lds_bytes);
+    if (le != hipSuccess) return le;
     const uint32_t n_done = n_sub > 1u ? n_slots : 0u;
     hipLaunchKernelGGL(k_reset_queue, dim3(n_done / 256u + 1u), dim3(256), 0, s, queue, done, n_done);
     hipLaunchKernelGGL(k_resident<NT>, dim3(grid), dim3(NT), lds_bytes, s, slots, n_slots, n_sub, slot_lats,

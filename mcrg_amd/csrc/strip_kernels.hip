@@ -18,8 +18,8 @@
 // bit-identical to the HBM schedule's and the oracle's.
 #include <algorithm>
 #include <cstdlib>
-#include <mutex>
 
+#include "lds_opt_in.hpp"
 #include "levels.hpp"
 #include "strip.hpp"
 
@@ -1074,17 +1074,9 @@ template <int NT>
 static hipError_t launch_nt(const StripArgs &a, hipStream_t s)
 {
     const uint32_t lds_bytes = a.sh.lds_words * 4u;
-    static std::mutex mu;
-    static uint32_t opted_in = 65536u;
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        if (lds_bytes > opted_in) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_strip<NT>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-            if (e != hipSuccess) return e;
-            opted_in = lds_bytes;
-        }
-    }
+    static LdsOptIn lds;
+    const hipError_t le = lds.need(reinterpret_cast<const void *>(&k_strip<NT>), lds_bytes);
+    if (le != hipSuccess) return le;
     StripArgs arg = a;
     const dim3 grid(a.sh.n_wg + a.sh.n_meas + a.sh.n_tail);
     // MCRG_STRIP_NONCOOP=1: an ordinary launch, for profilers that fail on

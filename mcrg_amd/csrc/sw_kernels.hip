@@ -10,8 +10,8 @@
 //   k_sw_measure0
 //             level-0 operators and the blocking into level 1, from bits
 #include <algorithm>
-#include <mutex>
 
+#include "lds_opt_in.hpp"
 #include "sw_core.hpp"
 
 namespace mcrg {
@@ -326,17 +326,9 @@ template <uint32_t PW>
 static hipError_t launch_sw_wg_pw(const HbmLattice *d, int n_lats, uint32_t lds_bytes, uint32_t n, bool measure,
                                   uint32_t n_work, uint32_t threads, hipStream_t s)
 {
-    static std::mutex mu;
-    static uint32_t opted_in = 65536u;
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        if (lds_bytes > opted_in) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_sw_wg<PW>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-            if (e != hipSuccess) return e;
-            opted_in = lds_bytes;
-        }
-    }
+    static LdsOptIn lds;
+    const hipError_t le = lds.need(reinterpret_cast<const void *>(&k_sw_wg<PW>), lds_bytes);
+    if (le != hipSuccess) return le;
     hipLaunchKernelGGL(k_sw_wg<PW>, dim3((uint32_t)n_lats), dim3(threads), lds_bytes, s, d, n, measure ? 1u : 0u,
                        n_work);
     return hipGetLastError();

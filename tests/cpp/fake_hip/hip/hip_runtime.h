@@ -1,5 +1,6 @@
-// A stand-in for the HIP runtime's memory calls: devices of a few bytes each, in
-// host memory, for tests of the code that allocates (no GPU).
+// A stand-in for the HIP runtime's memory and attribute calls: devices of a few
+// bytes each, in host memory, for tests of the code that allocates and launches
+// (no GPU).
 #pragma once
 #include <cstddef>
 #include <cstdlib>
@@ -13,6 +14,8 @@ struct FakeHip {
     int device = 0, frees = 0;
     hipError_t last = hipSuccess;
     std::map<void *, std::pair<int, size_t>> live;
+    int set_calls = 0, set_max = 1 << 30;
+    std::map<std::pair<int, const void *>, int> lds;  // (device, kernel) -> dynamic LDS it may take
 };
 inline FakeHip g_hip;
 
@@ -44,4 +47,13 @@ inline hipError_t hipGetLastError()
     const hipError_t e = g_hip.last;
     g_hip.last = hipSuccess;
     return e;
+}
+
+enum hipFuncAttribute { hipFuncAttributeMaxDynamicSharedMemorySize = 8 };
+inline hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute, int value)
+{
+    ++g_hip.set_calls;
+    if (value > g_hip.set_max) return hipErrorInvalidValue;
+    g_hip.lds[{g_hip.device, f}] = value;
+    return hipSuccess;
 }
