@@ -125,6 +125,22 @@ size_t sw_scratch_bytes(int L);
 // their counters in one launch, a thread for each `part` sites (sw_wg_part).
 constexpr int kSwWgMaxL = 128;
 int sw_wg_part(int n_lats, int L, int n_cus);
+// The LDS that a workgroup asks for which needs `need` bytes: no more of them on
+// one compute unit than an even share, or some units would take six and others
+// two (1024 lattices of L = 64).  So that share + 1 of them do not fit, and not
+// more than that: what is left of a unit's LDS is for the kernels beside.  420
+// sweeps of 256 lattices of L = 64 and 2200 of 1024 resident ones of L = 128, 4.8
+// and 11.0 ms by themselves, took 18.4 ms together when each asked for the whole
+// share, and take 12.2; with 1024 of L = 256 (5.5 ms) 10.0 -> 8.7.  Where the
+// others' waves fill a unit (600 of L = 512 beside 16) it gives nothing: 12.6, 12.8.
+constexpr uint32_t kCuLdsBytes = 163840u, kLdsUnit = 1280u;  // a unit's LDS, and its allocation unit
+inline uint32_t sw_wg_lds_bytes(uint32_t need, int n_lats, int n_cus)
+{
+    const uint32_t share = (uint32_t)((n_lats + n_cus - 1) / n_cus);
+    if (share > 8u) return need;
+    const uint32_t pad = (kCuLdsBytes / (share + 1u) / kLdsUnit + 1u) * kLdsUnit;
+    return need > pad ? need : pad;
+}
 hipError_t launch_sw_wg(const HbmLattice *d, int n_lats, int L, int n_levels, int part, uint32_t n, bool measure,
                         int n_cus, hipStream_t s);
 // Metropolis chains of 8 <= L <= 32: n sweeps (all measured or none) of n_lats

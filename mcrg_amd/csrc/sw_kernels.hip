@@ -358,12 +358,8 @@ hipError_t launch_sw_wg(const HbmLattice *d, int n_lats, int L, int n_levels, in
     // workgroups of 4 + 1 waves a unit holds three, since each puts two waves on
     // one of the four SIMDs (1024 x L = 64 measured: 32 us a sweep, 24 without).
     const uint32_t threads = n_work + (measure && n_levels > 0 && n_lats <= n_cus ? 64u : 0u);
-    uint32_t lds_bytes = 4u * sw_wg_layout((uint32_t)L, (uint32_t)n_levels, n_work).total;
-    // No more workgroups on one compute unit than an even share: LDS is asked
-    // for that keeps the others out, or some units would take six and others
-    // two (1024 lattices of L = 64).
-    const uint32_t share = (uint32_t)((n_lats + n_cus - 1) / n_cus);
-    if (share <= 8u) lds_bytes = std::max(lds_bytes, kMaxLdsBytes / share / 2048u * 2048u);
+    const uint32_t lds_bytes =
+        sw_wg_lds_bytes(4u * sw_wg_layout((uint32_t)L, (uint32_t)n_levels, n_work).total, n_lats, n_cus);
     switch (part) {
     case 4: return launch_sw_wg_pw<4>(d, n_lats, lds_bytes, n, measure, n_work, threads, s);
     case 8: return launch_sw_wg_pw<8>(d, n_lats, lds_bytes, n, measure, n_work, threads, s);
