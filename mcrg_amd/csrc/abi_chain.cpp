@@ -100,6 +100,7 @@ struct mcrg_chain_s {
     StripRunner strip;             // cooperative strip launches (large Metropolis chains)
     std::shared_ptr<ResultLines> lines;  // the context's, of which this chain has `line`, or -1
     int line = -1;
+    bool colour_ran = false;       // a k_colour_chain since the last check of its error word
 };
 
 static mcrg_status strip_status(bool bad)
@@ -111,12 +112,29 @@ static mcrg_status strip_status(bool bad)
     return MCRG_OK;
 }
 
-// Fails when a strip launch since the last check gave up on a wait.
-static mcrg_status check_strip(mcrg_chain ch)
+// Fails when a launch since the last check gave up on a wait (the stream has
+// drained).
+static mcrg_status check_waits(mcrg_chain ch)
 {
     bool bad = false;
     MCRG_HIP(ch->strip.failed(ch->stream, bad));
-    return strip_status(bad);
+    const mcrg_status st = strip_status(bad);
+    if (st != MCRG_OK || !ch->colour_ran) return st;
+    uint32_t word = 0;
+    if (ch->line >= 0) {
+        word = __atomic_load_n(ch->host.error, __ATOMIC_RELAXED);
+        if (word) __atomic_store_n(ch->host.error, 0u, __ATOMIC_RELAXED);
+    } else {
+        MCRG_HIP(hipMemcpyAsync(&word, ch->host.error, sizeof(word), hipMemcpyDeviceToHost, ch->stream));
+        MCRG_HIP(hipMemsetAsync(ch->host.error, 0, sizeof(word), ch->stream));
+        MCRG_HIP(hipStreamSynchronize(ch->stream));
+    }
+    ch->colour_ran = false;
+    if (word) {
+        set_error("one-workgroup launch: a wave's wait for the others exceeded the limit; the chain state is lost");
+        return MCRG_ERR_DEVICE;
+    }
+    return MCRG_OK;
 }
 
 extern "C" {
@@ -259,11 +277,14 @@ mcrg_status mcrg_chain_create(mcrg_ctx ctx, const mcrg_chain_desc *desc, mcrg_ch
     char *base = static_cast<char *>(ch->d_block);
     ch->host = hbm_descriptor(base, blk, d.L, d.n_levels, d.sweeps_per_bin, d.seed, d.coupling, d.sampler);
     ch->d_desc = reinterpret_cast<HbmLattice *>(base + o_desc);
+    ch->lines = ctx->lines;
+    if (ch->lines && (ch->line = ch->lines->take()) >= 0) ch->host.error = ch->lines->error(ch->line);
 
     auto fail = [&](hipError_t err, const char *what) {
         set_error(std::string(what) + ": " + hipGetErrorString(err));
         if (ch->stream) (void)hipStreamDestroy(ch->stream);
         (void)hipFree(ch->d_block);
+        if (ch->lines) ch->lines->give(ch->line);
         delete ch;
         return MCRG_ERR_DEVICE;
     };
@@ -275,8 +296,6 @@ mcrg_status mcrg_chain_create(mcrg_ctx ctx, const mcrg_chain_desc *desc, mcrg_ch
         return fail(e, "hipMemcpyAsync");
     if ((e = launch_int8_init(ch->d_desc, 1, d.L, ch->stream)) != hipSuccess) return fail(e, "k_int8_init");
     if ((e = hipStreamSynchronize(ch->stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
-    ch->lines = ctx->lines;
-    if (ch->lines) ch->line = ch->lines->take();
     *out = ch;
     return MCRG_OK;
 }
@@ -343,6 +362,7 @@ mcrg_status mcrg_chain_sweep(mcrg_chain ch, int32_t n_sweeps, int32_t measure)
     else
         MCRG_HIP(ch->runner.run(ch->d_desc, 1, d.L, d.n_levels, d.sampler, (uint32_t)n_sweeps, measure != 0,
                                 ch->stream, tm));
+    ch->colour_ran = ch->colour_ran || colour_chain(d.L, d.sampler == MCRG_SAMPLER_METROPOLIS);
     ch->t += (uint32_t)n_sweeps;
     if (measure) ch->n_measured += (uint32_t)n_sweeps;
     return MCRG_OK;
@@ -385,7 +405,7 @@ mcrg_status mcrg_chain_sync(mcrg_chain ch)
     MCRG_REQUIRE(ch != nullptr, "chain is null");
     MCRG_HIP(hipSetDevice(ch->ctx->device));
     MCRG_HIP(hipStreamSynchronize(ch->stream));
-    return check_strip(ch);
+    return check_waits(ch);
 }
 
 mcrg_status mcrg_chain_get_spins(mcrg_chain ch, int8_t *host, int64_t n)
@@ -395,7 +415,7 @@ mcrg_status mcrg_chain_get_spins(mcrg_chain ch, int8_t *host, int64_t n)
     MCRG_HIP(hipSetDevice(ch->ctx->device));
     MCRG_HIP(hipMemcpyAsync(host, ch->host.spins, (size_t)n, hipMemcpyDeviceToHost, ch->stream));
     MCRG_HIP(hipStreamSynchronize(ch->stream));
-    return check_strip(ch);
+    return check_waits(ch);
 }
 
 mcrg_status mcrg_chain_set_spins(mcrg_chain ch, const int8_t *host, int64_t n)
@@ -418,7 +438,7 @@ mcrg_status mcrg_chain_get_records(mcrg_chain ch, int64_t *host, int64_t n)
     MCRG_HIP(hipSetDevice(ch->ctx->device));
     MCRG_HIP(hipMemcpyAsync(host, ch->host.records, (size_t)n * 8, hipMemcpyDeviceToHost, ch->stream));
     MCRG_HIP(hipStreamSynchronize(ch->stream));
-    return check_strip(ch);
+    return check_waits(ch);
 }
 
 mcrg_status mcrg_chain_get_state(mcrg_chain ch, uint32_t *sweep, uint32_t *n_measured)
@@ -454,7 +474,7 @@ mcrg_status mcrg_chain_operators(mcrg_chain ch, int64_t out[4])
     unsigned long long cnt[kOperatorWords];
     // the strips' error word comes with the counts: no copy and wait of its own
     const uint32_t *error = ch->strip.error_word();
-    static_assert(kOperatorWords <= ResultLines::kWords, "a chain's line");
+    static_assert(kOperatorWords < ResultLines::kWords, "a chain's line, its error word behind the counts");
     if (ch->line >= 0) {
         unsigned long long *line = ch->lines->base + ch->line * ResultLines::kWords;
         MCRG_HIP(launch_int8_operators(ch->d_desc, ch->desc.L, error, line, s));
@@ -466,7 +486,8 @@ mcrg_status mcrg_chain_operators(mcrg_chain ch, int64_t out[4])
         MCRG_HIP(hipStreamSynchronize(s));
     }
     if (error) ch->strip.reported();
-    const mcrg_status st = strip_status(cnt[4] != 0u);
+    mcrg_status st = strip_status(cnt[4] != 0u);
+    if (st == MCRG_OK) st = check_waits(ch);
     if (st != MCRG_OK) return st;
     const int64_t n0 = (int64_t)ch->desc.L * ch->desc.L;
     out[0] = 2 * n0 - 2 * (int64_t)cnt[0];

@@ -1,6 +1,9 @@
 // int8 chains of L = 64 and 128 in one workgroup, its waves split by colour:
 // Metropolis sweeps (replacing src/ising.cpp:87-149) and the measurement of
 // every level (src/lattice.cpp:102-120, src/mcrg.cpp:72-98, :314-348).
+#include <algorithm>
+#include <cstdlib>
+
 #include "lds_opt_in.hpp"
 #include "wave_core.hpp"
 
@@ -21,7 +24,11 @@ namespace mcrg {
 // waves of a workgroup are resident.  Why no word is overwritten too early: a
 // word of sweep t is stored after its neighbours' and its own of half a sweep
 // and a sweep before have been read, whose lanes had by then read everything up
-// to sweep t - 1, and colour 0 waits for the sample of sweep t - kRing.
+// to sweep t - 1, and colour 0 waits for the sample of sweep t - kRing.  Polls
+// are counted all the same: a wave that gives up ends with the step it is in, the
+// others, who wait for its words, do so as well, and the error word says that the
+// state is lost (leaving the step at once took L = 128 6 % more time: its branch
+// stands between the words and their decisions).
 //
 // Bound by the latency of a half sweep (L = 64: 740 cycles) and, at L = 128, by
 // VALU issue (8 wave-words a sweep on each SIMD).  us a sweep, unmeasured and
@@ -44,7 +51,7 @@ template <uint32_t L>
 static uint32_t colour_lds_words(uint32_t nl)
 {
     using G = ColourGeom<L>;
-    return kRing * 4u * G::W + G::M + G::M * 64u * G::entry + 2u * G::M * record_size(nl);
+    return kRing * 4u * G::W + G::M + 2u + G::M * 64u * G::entry + 2u * G::M * record_size(nl);
 }
 
 __device__ __forceinline__ uint64_t word_ld(const uint64_t *p)
@@ -55,14 +62,14 @@ __device__ __forceinline__ uint64_t word_ld(const uint64_t *p)
 // One lattice: n sweeps, all measured or none, and its counters.
 template <uint32_t L>
 __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const HbmLattice *__restrict__ lats, uint32_t n,
-                                                                         uint32_t measure)
+                                                                         uint32_t measure, uint32_t spins)
 {
     using G = ColourGeom<L>;
     constexpr uint32_t W = G::W, NW = G::NW, M = G::M, half = L / 2u, sites = L * half, WPR = L / 64u;
     static_assert(kRing % M == 0u, "the sample that a buffer holds");
     extern __shared__ __align__(16) uint32_t lds[];
     uint64_t *ring = reinterpret_cast<uint64_t *>(lds);  // word | sweeps done << 32
-    uint32_t *read = lds + kRing * 4u * W, *samples = read + M;
+    uint32_t *read = lds + kRing * 4u * W, *lost = read + M, *samples = lost + 2;  // lost: 1 once a wave gave up
     const HbmLattice &lat = lats[blockIdx.x];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uni<true>(tid >> 6);
     const uint32_t nl = (uint32_t)lat.n_levels, rs = record_size(nl), t0 = lat.state[0], q0 = lat.state[1];
@@ -73,7 +80,7 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
     };
     for (uint32_t k = tid; k < kRing * 2u * W; k += G::threads)
         if (k >= 2u * W) ring[k] = 0u;
-    if (tid < M) read[tid] = 0u;
+    if (tid <= M) read[tid] = 0u;
     for (uint32_t m0 = 64u * wave; m0 < 2u * sites; m0 += G::threads) {
         const uint32_t c = m0 >= sites ? 1u : 0u, mc = m0 - c * sites + lane;
         const uint64_t b = __ballot(lat.spins[at(mc, c)] < 0);
@@ -86,7 +93,8 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
         const uint32_t set = wave / NW, word = 64u * (wave - set * NW) + lane, y = word / WPR, q = word % WPR;
         const uint32_t up = ((y - 1u) & (L - 1u)) * WPR + q, dn = ((y + 1u) & (L - 1u)) * WPR + q;
         const Accept acc = lat.acc;
-        for (uint32_t step = set; step < 2u * n; step += G::SETS) {
+        uint32_t end = 2u * n;
+        for (uint32_t step = set; step < end; step += G::SETS) {
             const uint32_t it = step >> 1, c = step & 1u, t = t0 + it, have = it + c, p = (y + c) & 1u;
             const MetropolisAhead<2u> h = metropolis_ahead<2u>(acc, k0, k1, word, t, c);
             const uint64_t *mine = ring + (it % kRing) * 2u * W + c * W;
@@ -95,6 +103,7 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
             // colour 0 writes over the sample of kRing sweeps ago
             const uint32_t want = c == 0u && measure && it >= kRing ? it - kRing + 1u : 0u;
             uint64_t own, o, side, nu, nd;
+            uint32_t left = spins;
             for (;;) {
                 own = word_ld(mine + word);
                 o = word_ld(oth + word);
@@ -106,6 +115,11 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
                                      ((uint32_t)(side >> 32) ^ have) | ((uint32_t)(nu >> 32) ^ have) |
                                      ((uint32_t)(nd >> 32) ^ have);
                 if (__ballot(off != 0u || done < want) == 0ull) break;
+                if (left-- == 0u) {  // the last step, from whatever is there
+                    lds_st(lost, 1u);
+                    end = 0u;
+                    break;
+                }
             }
             const uint32_t w = (uint32_t)own ^
                                metropolis_decide(h, (uint32_t)own, (uint32_t)nu, (uint32_t)nd,
@@ -119,7 +133,7 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
         uint32_t *mine = samples + j * 64u * G::entry;
         int64_t *rec = reinterpret_cast<int64_t *>(samples + M * 64u * G::entry) + j * rs;
         for (uint32_t k = lane; k < rs; k += 64u) rec[k] = 0;
-        uint32_t rec_bin = 0xFFFFFFFFu, slot = 0;
+        uint32_t rec_bin = 0xFFFFFFFFu, slot = 0, end = n;
         auto flush = [&]() {
             small_sync();
             // the measuring waves share bins
@@ -131,11 +145,11 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
             for (uint32_t k = lane; k < rs; k += 64u) rec[k] = 0;
             small_sync();
         };
-        for (uint32_t it = j; it < n; it += M) {
+        for (uint32_t it = j; it < end; it += M) {
             constexpr uint32_t WPL = WaveGeom<L>::WPL;
             const uint64_t *buf = ring + ((it + 1u) % kRing) * 2u * W + WPL * lane;
             uint32_t c0[WPL], c1[WPL];
-            for (;;) {
+            for (uint32_t left = spins;; --left) {
                 uint32_t off = 0;
 #pragma unroll
                 for (uint32_t k = 0; k < WPL; ++k) {
@@ -145,6 +159,11 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
                     off |= ((uint32_t)(a >> 32) ^ (it + 1u)) | ((uint32_t)(b >> 32) ^ (it + 1u));
                 }
                 if (__ballot(off != 0u) == 0ull) break;
+                if (left == 0u) {
+                    lds_st(lost, 1u);
+                    end = 0u;
+                    break;
+                }
                 __builtin_amdgcn_s_sleep(1);
             }
             if (lane == 0u) lds_st(read + j, it + 1u);
@@ -162,6 +181,10 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
         if (rec_bin != 0xFFFFFFFFu) flush();
     }
     __syncthreads();
+    if (lds_ld(lost) != 0u) {
+        if (tid == 0u) __hip_atomic_store(lat.error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
+    }
     const uint64_t *end = ring + (n % kRing) * 2u * W;
     for (uint32_t mc = tid; mc < 2u * sites; mc += G::threads) {
         const uint32_t c = mc >= sites ? 1u : 0u;
@@ -180,8 +203,10 @@ static hipError_t launch_colour(const HbmLattice *d, int n_lats, int n_levels, u
     static LdsOptIn lds;
     const hipError_t le = lds.need(reinterpret_cast<const void *>(&k_colour_chain<L>), lds_bytes);
     if (le != hipSuccess) return le;
+    uint32_t spins = kColourSpins;
+    if (const char *v = std::getenv("MCRG_COLOUR_SPINS")) spins = (uint32_t)std::min<long>(std::max(0L, std::atol(v)), kColourSpins);
     hipLaunchKernelGGL(k_colour_chain<L>, dim3((uint32_t)n_lats), dim3(ColourGeom<L>::threads), lds_bytes, s, d, n,
-                       measure ? 1u : 0u);
+                       measure ? 1u : 0u, spins);
     return hipGetLastError();
 }
 

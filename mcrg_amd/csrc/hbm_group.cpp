@@ -48,6 +48,7 @@ HbmLattice hbm_descriptor(char *base, const HbmBlock &b, int L, int n_levels, in
     h.sampler = sampler;
     h.sw = sw_tiled(L, sampler) ? reinterpret_cast<uint32_t *>(base + b.sw) : nullptr;
     h.bond_thr = bond_threshold(coupling);
+    h.error = reinterpret_cast<uint32_t *>(h.sums + kSumError);
     return h;
 }
 
@@ -197,6 +198,7 @@ hipError_t HbmGroup::init(const std::vector<JobSpec> &members, hipStream_t s)
     for (size_t k = 0; k < n; ++k)
         host_[k] = hbm_descriptor(d_block_ + k * blk_.bytes, blk_, j.L, j.n_levels, j.sweeps_per_bin,
                                   members_[k].seed, members_[k].coupling, j.sampler);
+    for (HbmLattice &h : host_) h.error = host_[0].error;
     if ((e = hipMemsetAsync(d_block_, 0, desc_off, s)) != hipSuccess) return e;
     if ((e = hipMemcpyAsync(d_desc_, host_.data(), sizeof(HbmLattice) * n, hipMemcpyHostToDevice, s)) !=
         hipSuccess)
@@ -230,7 +232,22 @@ hipError_t HbmGroup::read_records(int member, int64_t *host, int64_t n, hipStrea
     if ((e = hipMemcpyAsync(host, host_[(size_t)member].records, (size_t)n * 8u, hipMemcpyDeviceToHost, s)) !=
         hipSuccess)
         return e;
-    return hipStreamSynchronize(s);
+    return finish(s);
+}
+
+// The stream's end; fails once when a launch gave up on a wait.
+hipError_t HbmGroup::finish(hipStream_t s)
+{
+    hipError_t e;
+    uint32_t bad = 0;
+    const bool waits = colour_chain(spec().L, spec().sampler == MCRG_SAMPLER_METROPOLIS);
+    if (waits && (e = hipMemcpyAsync(&bad, host_[0].error, sizeof(bad), hipMemcpyDeviceToHost, s)) != hipSuccess)
+        return e;
+    if ((e = hipStreamSynchronize(s)) != hipSuccess || bad == 0u) return e;
+    bad = 0u;
+    if ((e = hipMemcpyAsync(host_[0].error, &bad, sizeof(bad), hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+    return hipErrorLaunchFailure;
 }
 
 size_t HbmGroup::record_pitch() const
@@ -249,7 +266,7 @@ hipError_t HbmGroup::read_records_block(int member, int count, char *host, hipSt
     else
         e = hipMemcpy2DAsync(host, width, rec, blk_.bytes, width, (size_t)count, hipMemcpyDeviceToHost, s);
     if (e != hipSuccess) return e;
-    return hipStreamSynchronize(s);
+    return finish(s);
 }
 
 hipError_t HbmGroup::read_spins(int member, int8_t *host, hipStream_t s)
@@ -257,7 +274,7 @@ hipError_t HbmGroup::read_spins(int member, int8_t *host, hipStream_t s)
     hipError_t e;
     const size_t n = (size_t)spec().L * (size_t)spec().L;
     if ((e = hipMemcpyAsync(host, host_[(size_t)member].spins, n, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
-    return hipStreamSynchronize(s);
+    return finish(s);
 }
 
 }  // namespace mcrg

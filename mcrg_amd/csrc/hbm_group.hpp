@@ -80,6 +80,7 @@ class HbmGroup {
     hipError_t read_spins(int member, int8_t *host, hipStream_t s);
 
   private:
+    hipError_t finish(hipStream_t s);
     std::vector<JobSpec> members_;
     HbmBlock blk_;
     char *d_block_ = nullptr;

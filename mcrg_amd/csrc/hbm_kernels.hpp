@@ -21,7 +21,9 @@ constexpr uint32_t kWgLevelMaxL = kGridLevelMinL / 2;
 constexpr uint32_t kSumWords = 4u + 3u * kMaxLevels;
 // behind them: k_int8_operators' count of finished workgroups and its results
 constexpr uint32_t kOperatorWords = 5u;
-constexpr uint32_t kSumTicket = kSumWords, kSumOut = kSumWords + 1u, kSumAlloc = kSumOut + kOperatorWords;
+constexpr uint32_t kSumTicket = kSumWords, kSumOut = kSumWords + 1u;
+// and the error word of launches whose waits gave up, where it has no other place
+constexpr uint32_t kSumError = kSumOut + kOperatorWords, kSumAlloc = kSumError + 1u;
 
 // Rows per thread strip of the int8 half-sweep (L >= 64).  Up to L = 8192 the
 // lattice (<= 64 MiB) stays in the 256 MB last-level cache, so each row's three
@@ -108,6 +110,7 @@ struct HbmLattice {
     uint32_t *sw;               // tile scratch (Swendsen-Wang lattices beyond kSwWgMaxL)
     uint32_t bond_thr;          // floor((1 - exp(-2J)) 2^32): bond probability of an aligned pair
     uint32_t pad;
+    uint32_t *error;            // set to 1 by a k_colour_chain that gave up (device or mapped host memory)
 };
 
 // Launchers (host).  `d` points to n_lats device descriptors that all share side L.
@@ -148,7 +151,12 @@ hipError_t launch_sw_wg(const HbmLattice *d, int n_lats, int L, int n_levels, in
 constexpr int kSmallChainMinL = 8, kSmallChainMaxL = 32;
 hipError_t launch_small_chain(const HbmLattice *d, int n_lats, int L, int n_levels, uint32_t n, bool measure,
                               hipStream_t s);
-// The same for 64 <= L <= kColourMaxL, a workgroup each.
+// The same for 64 <= L <= kColourMaxL, a workgroup each, whose waves wait for
+// each other's words: a wait that polls more than kColourSpins times (a second at
+// least; MCRG_COLOUR_SPINS in the environment, with which tests of the error
+// path make waits give up) sets the lattice's error word, and its spins and
+// counters stay as they were.
+constexpr uint32_t kColourSpins = 1u << 24;
 constexpr int kColourMaxL = 128;
 hipError_t launch_colour_chain(const HbmLattice *d, int n_lats, int L, int n_levels, uint32_t n, bool measure,
                                hipStream_t s);
@@ -156,6 +164,11 @@ hipError_t launch_colour_chain(const HbmLattice *d, int n_lats, int L, int n_lev
 inline bool chain_on_chip(int L, bool metropolis)
 {
     return metropolis && L >= kSmallChainMinL && L <= kColourMaxL;
+}
+// Whether that is a k_colour_chain, whose launches may give up.
+inline bool colour_chain(int L, bool metropolis)
+{
+    return chain_on_chip(L, metropolis) && L > kSmallChainMaxL;
 }
 hipError_t launch_int8_half_sweep(const HbmLattice *d, int n_lats, int L, uint32_t t_off,
                                   uint32_t colour, hipStream_t s);

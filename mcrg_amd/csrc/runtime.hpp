@@ -100,8 +100,11 @@ struct ResultLines {
         if (!base || ~used == 0ull) return -1;
         const int k = __builtin_ctzll(~used);
         used |= 1ull << k;
+        *error(k) = 0u;
         return k;
     }
+    // The error word of line k, its last one.
+    uint32_t *error(int k) const { return reinterpret_cast<uint32_t *>(base + k * kWords + kWords - 1); }
     void give(int k)
     {
         std::lock_guard<std::mutex> lock(mu);
