@@ -205,25 +205,25 @@ typedef struct {
 } mcrg_job_desc;
 
 typedef struct {
-    int32_t threads;           /* workgroup size 64/128/256/512; 0 = 256       */
+    int32_t threads;           /* workgroup size 64/128/256/512 of lattices of
+                                  L = 256 (and 512: threads_large); 0 = 256     */
     int32_t sweeps_per_launch; /* sweeps per kernel launch; 0 = 250           */
-    int32_t max_group;         /* upper bound on lattices per workgroup; 0 = 256 */
-    int32_t max_slot_lds;      /* LDS bytes a workgroup of small lattices may take
-                                  (lattices per workgroup halve until it fits);
-                                  0 = 32 KiB per 256 threads                    */
-    int32_t min_team;          /* lanes per lattice at least (1..threads, power
-                                  of two); 0 = 16.  The team and workgroup sizes
-                                  are those of L >= 256; smaller lattices take
-                                  64 / (lattices of the wave) lanes             */
-    int32_t max_team;          /* lanes per lattice at most (power of two,
-                                  >= min_team); 0 = threads                     */
+    int32_t max_group;         /* upper bound on lattices per wave (L <= 32);
+                                  0 = 256                                       */
+    /* The next three are checked and reported by mcrg_batch_get_opts, and have
+     * no effect on the launches: a lattice of L >= 256 takes a workgroup, one of
+     * L = 64 or 128 a wave, smaller ones share a wave. */
+    int32_t max_slot_lds;      /* >= 0                                          */
+    int32_t min_team;          /* 1..threads, a power of two; 0 = 16            */
+    int32_t max_team;          /* a power of two, min_team..threads; 0          */
     int32_t threads_large;     /* workgroup size for lattices of L = 512
                                   (64/128/256/512/1024); 0 = 1024 when there
                                   are at most as many of them as compute
                                   units, else 512                               */
     int32_t autotune;          /* nonzero: the first launches each try one
-                                  candidate configuration (timed with events)
-                                  and the fastest is kept if it beats the
+                                  candidate configuration (workgroup sizes of
+                                  lattices of L >= 256; timed with events) and
+                                  the fastest is kept if it beats the
                                   configuration given here by more than 4 %;
                                   results are the same under every
                                   configuration                                 */
@@ -260,7 +260,9 @@ mcrg_status mcrg_batch_get_opts(mcrg_batch b, mcrg_batch_opts *out);
 /* Continuous batching of MCRG jobs (mcrg_job_desc) on one device.  Jobs are
  * submitted at any time from any thread; a scheduler admits queued jobs in
  * arrival order while their spins and records fit the device-memory budget and
- * their share of LDS (slot LDS / lattices per slot) fits the LDS budget,
+ * their LDS weights fit the LDS budget (a weight is what spins, blocked levels,
+ * counts and records of a lattice of this shape take, about 0.7 KB at L = 8 and
+ * 58 KB at L = 512; kernels take somewhat more or less),
  * advances every admitted job by
  * one time slice per launch of the resident schedule (jobs of different L
  * and coupling share each launch; a slot of G lattices of side L runs
@@ -277,7 +279,7 @@ typedef struct mcrg_server_s *mcrg_server;
 
 typedef struct {
     int64_t hbm_budget_bytes;  /* device memory for resident jobs; 0 = 4 GiB          */
-    int64_t lds_budget_bytes;  /* summed LDS share of resident jobs; 0 = two full
+    int64_t lds_budget_bytes;  /* summed LDS weights of resident jobs; 0 = two full
                                   waves of workgroups (2 x CUs x LDS per CU)          */
     int64_t launch_quantum;    /* microseconds of work per workgroup and launch;
                                   0 = 4000                                            */
@@ -404,7 +406,9 @@ mcrg_status mcrg_critical_point_step_bins(const int64_t *rec_large, int32_t n_bi
 
 /* ------------------------------------------------------------------ timing */
 /* Kernel-duration statistics measured with HIP events on the stream that
- * launched the kernel, enabled per context.  kind: 0 = half-sweep kernel,
+ * launched the kernel, enabled per context.  kind: 0 = half-sweep kernel, or a
+ * kernel that runs many sweeps and their measurements (Metropolis L = 8 .. 128,
+ * Swendsen-Wang L <= 128), or the three of a larger Swendsen-Wang sweep,
  * 1 = level-0 measurement kernel, 2 = levels/accumulate kernel,
  * 3 = batched resident kernels, 4 = strip kernel (one launch per
  * mcrg_chain_sweep call on the strip schedule). */

@@ -202,46 +202,29 @@ size_t ResidentEngine::job_bytes(const JobSpec &j)
     return spins + rec;
 }
 
-uint32_t ResidentEngine::lds_bytes(int L, int G, int nl, int NT) const
-{
-    const uint32_t T = (uint32_t)NT / (uint32_t)G;
-    return slot_words((uint32_t)L, (uint32_t)G, (uint32_t)nl, T) * 4u;
-}
-
 void ResidentEngine::enable_autotune()
 {
+    // Workgroups of other sizes, where they change a launch: smaller lattices are
+    // waves whatever the sizes.
+    bool mid = false, large = false;
+    for (const Job &j : jobs_) {
+        const bool big = j.live && j.spec.L > kWaveMaxL;
+        large = large || (big && j.spec.L >= opt_.large_min_L);
+        mid = mid || (big && j.spec.L < opt_.large_min_L);
+    }
+    auto shape = [&](const TuneCandidate &c) {
+        return std::make_pair(mid ? c.threads : 0, !large ? 0 : c.threads_large > 0 ? c.threads_large : c.threads);
+    };
     // the first entry repeats the configuration in use to absorb first-launch costs
-    const EngineOptions o = opt_;
-    tune_ = {{o.threads, o.min_team, o.threads_large, o.max_slot_lds, 0.0},
-             {o.threads, o.min_team, o.threads_large, o.max_slot_lds, 0.0},
-             {128, 16, 0, 0, 0.0},
-             {256, 16, 0, 0, 0.0},
-             {512, 16, 0, 0, 0.0},
-             {256, 32, 0, 0, 0.0},
-             {256, 8, 0, 0, 0.0},
-             {256, 16, 512, 0, 0.0},
-             {256, 16, 0, 65536, 0.0}};
+    const TuneCandidate now{opt_.threads, opt_.threads_large, 0.0};
+    tune_ = {now, now};
+    for (const TuneCandidate &c : {TuneCandidate{128, 0, 0.0}, TuneCandidate{256, 0, 0.0}, TuneCandidate{512, 0, 0.0},
+                                   TuneCandidate{256, 512, 0.0}}) {
+        bool new_shape = true;
+        for (const TuneCandidate &t : tune_) new_shape = new_shape && shape(t) != shape(c);
+        if (new_shape) tune_.push_back(c);
+    }
     tune_next_ = 0;
-}
-
-int ResidentEngine::group_size(int L, int nl, int NT) const
-{
-    const int W = (int)cb_words((uint32_t)L);
-    int G = W >= NT ? 1 : NT / W;
-    if (opt_.max_team > 0) G = std::max(G, NT / opt_.max_team);
-    int cap = 1;
-    while (cap * 2 <= opt_.max_group) cap *= 2;  // positions are a power of two
-    G = std::min(G, cap);
-    // a team of at least min_team lanes shares each lattice's measurement, but
-    // no more than max(4, W) lanes: a lattice of W words per colour keeps the
-    // rest of a larger team idle in its sweeps (L = 8: 121 -> 300 updates/ns
-    // with 4 lanes instead of 16; L = 16: 372 -> 574)
-    const int team_min = std::min(std::max(1, opt_.min_team), std::max(4, W));
-    G = std::min(G, std::max(1, NT / team_min));
-    // keep a slot's LDS modest so that several workgroups share a CU
-    const uint32_t soft = opt_.max_slot_lds ? opt_.max_slot_lds : 32768u * (uint32_t)NT / 256u;
-    while (G > 1 && lds_bytes(L, G, nl, NT) > soft) G /= 2;
-    return std::max(G, 1);
 }
 
 int ResidentEngine::small_group(int L, int n, bool alone) const
@@ -258,10 +241,16 @@ int ResidentEngine::small_group(int L, int n, bool alone) const
     return G;
 }
 
-uint32_t ResidentEngine::lds_share(int L, int nl, int NT) const
+uint32_t ResidentEngine::lds_share(int L, int nl, int NT)
 {
-    const int G = group_size(L, nl, NT);
-    return (lds_bytes(L, G, nl, NT) + (uint32_t)G - 1u) / (uint32_t)G;
+    // lattices of a workgroup: a word of a colour a thread, at least 16 lanes each
+    // (the words' number where that is less, but 4), and 32 KiB per 256 threads
+    const int W = (int)cb_words((uint32_t)L);
+    int G = std::min(W >= NT ? 1 : NT / W, 256);
+    G = std::max(1, std::min(G, NT / std::min(16, std::max(4, W))));
+    auto bytes = [&]() { return 4u * slot_words((uint32_t)L, (uint32_t)G, (uint32_t)nl, (uint32_t)(NT / G)); };
+    while (G > 1 && bytes() > 32768u * (uint32_t)NT / 256u) G /= 2;
+    return (bytes() + (uint32_t)G - 1u) / (uint32_t)G;
 }
 
 uint64_t ResidentEngine::slot_time_ns(int L, int G, uint32_t n_sweeps) const
@@ -639,9 +628,7 @@ hipError_t ResidentEngine::tick(uint32_t n, uint32_t &advanced, KernelTimer *tm)
     if (timing) {
         const TuneCandidate &c = tune_[tune_next_];
         opt_.threads = c.threads;
-        opt_.min_team = std::min(c.min_team, c.threads);
         opt_.threads_large = c.threads_large;
-        opt_.max_slot_lds = c.max_slot_lds;
         slots_dirty_ = true;
         if (!tune_a_ && (e = hipEventCreate(&tune_a_)) != hipSuccess) return e;
         if (!tune_b_ && (e = hipEventCreate(&tune_b_)) != hipSuccess) return e;
@@ -698,14 +685,15 @@ hipError_t ResidentEngine::tick(uint32_t n, uint32_t &advanced, KernelTimer *tm)
             // timing noise (up to 3 % between launches of the batched
             // workload), so near-equal candidates do not flip the choice from
             // run to run
-            size_t best = 2;
-            for (size_t i = 3; i < tune_.size(); ++i)
+            size_t best = 1;
+            for (size_t i = 2; i < tune_.size(); ++i)
                 if (tune_[i].rate > tune_[best].rate) best = i;
             if (tune_[best].rate <= kTuneMargin * tune_[1].rate) best = 1;
             opt_.threads = tune_[best].threads;
-            opt_.min_team = std::min(tune_[best].min_team, tune_[best].threads);
             opt_.threads_large = tune_[best].threads_large;
-            opt_.max_slot_lds = tune_[best].max_slot_lds;
+            // options that were accepted with the workgroup size stay acceptable
+            opt_.min_team = std::min(opt_.min_team, opt_.threads);
+            opt_.max_team = std::min(opt_.max_team, opt_.threads);
             slots_dirty_ = true;
         }
     }

@@ -70,14 +70,12 @@ struct EngineOptions {
     int threads = 256;           // workgroup size of the resident kernel
     int sweeps_per_launch = 250;  // chunk length (the most sweeps any lattice runs per launch)
     int max_group = 256;          // upper bound on lattices per slot
-    int min_team = 16;            // lanes per lattice at least (measurement parallelism)
-    int max_team = 0;             // lanes per lattice at most (0 = threads): smaller teams
-                                  // loop over more words and measure lattices side by side
+    // accepted, checked and reported, without an effect on the launches: a lattice
+    // has a workgroup (L = 256, 512) or a share of a wave
+    int min_team = 16, max_team = 0;
+    uint32_t max_slot_lds = 0;
     int threads_large = 0;        // workgroup size for lattices of L >= large_min_L (0 = threads)
     int large_min_L = 512;
-    // LDS a slot of small lattices may take (G halves until it fits);
-    // 0 = 32 KiB per 256 threads, which leaves room for five workgroups per CU.
-    uint32_t max_slot_lds = 0;
     // Time slicing: when nonzero, a slot runs min(chunk, max(1, quantum_ns /
     // t_sweep)) sweeps per launch, with the measured-sweep time of a slot
     // modelled as t_sweep = kSweepFixedNs + kSweepPerSiteNs * (G L^2 / threads)
@@ -172,9 +170,9 @@ class ResidentEngine {
     hipStream_t stream() const { return stream_; }
     // Name of the HIP call behind the last error returned by this engine.
     const char *failed_call() const { return failed_; }
-    // Autotuning: the next launches each run one candidate configuration
-    // (workgroup size, team bounds, slot LDS cap) and are timed with events;
-    // then the fastest is kept.  Results do not depend on the configuration,
+    // Autotuning: the next launches each run one candidate configuration (workgroup
+    // sizes of the lattices of L = 256 and 512; without such lattices only the one
+    // in use) and are timed with events; then the fastest is kept.  Results do not depend on the configuration,
     // so the jobs advance exactly as they would otherwise.
     void enable_autotune();
     bool tuning() const { return tune_next_ < tune_.size(); }
@@ -187,17 +185,14 @@ class ResidentEngine {
             slots_dirty_ = true;
         }
     }
-    // Lattices per slot of side L on NT-thread workgroups.
-    int group_size(int L, int nl, int NT) const;
     // Workgroup size of the slots of side L.
     int threads_for(int L) const
     {
         return opt_.threads_large > 0 && L >= opt_.large_min_L ? opt_.threads_large : opt_.threads;
     }
-    uint32_t lds_bytes(int L, int G, int nl, int NT) const;
-    // LDS bytes one lattice of this shape takes in its slot (slot LDS / G), on
-    // NT-thread workgroups or on the ones the engine uses now.
-    uint32_t lds_share(int L, int nl, int NT) const;
+    // What a lattice of this shape counts in a server's LDS budget, on NT-thread
+    // workgroups or on the ones the engine uses now (slot_words).
+    static uint32_t lds_share(int L, int nl, int NT);
     uint32_t lds_share(int L, int nl) const { return lds_share(L, nl, threads_for(L)); }
 
   private:
@@ -210,8 +205,7 @@ class ResidentEngine {
         uint32_t t = 0, n_measured = 0, therm_left = 0, meas_left = 0;
     };
     struct TuneCandidate {
-        int threads, min_team, threads_large;
-        uint32_t max_slot_lds;
+        int threads, threads_large;
         double rate;
     };
     std::vector<TuneCandidate> tune_;

@@ -47,10 +47,13 @@ __host__ __device__ inline uint32_t level_words(uint32_t L, uint32_t l)
     return w ? w : 1u;
 }
 
-// LDS words that admission counts for G lattices of one slot, T = threads per
-// lattice: spins, blocked levels and their tie coins, counts, operator values
-// and records.  What a launch takes is big_layout() (up to 1.6 k words more: 64
-// samples wait there), small_lds_words() or wave_lds_words().
+// LDS words that a server's admission counts for G lattices of a workgroup, T =
+// threads per lattice: spins, blocked levels and their tie coins, counts,
+// operator values and records.  A weight by which the budget limits the resident
+// jobs (and refuses some), not what a launch takes: big_layout() (1.1 k to 3.3 k
+// words more for a lattice, since 64 samples wait there), wave_lds_words() (half
+// a thousand words more for L = 64, a hundred to two hundred less for L = 128 with
+// two levels or more) or small_lds_words().
 __host__ __device__ inline uint32_t slot_words(uint32_t L, uint32_t G, uint32_t nl, uint32_t T)
 {
     uint32_t lvl = 0;
