@@ -375,6 +375,7 @@ class Batch:
         check(_lib.mcrg_batch_create(ctx.handle, arr, len(jobs), ctypes.byref(opts), ctypes.byref(h)))
         self.handle = h
         self.jobs = [dict(j) for j in jobs]
+        self._record_size = {n: record_size(n) for n in {j.get("n_levels", 0) for j in jobs}}
 
     def run(self, max_sweeps):
         rem = ctypes.c_int32()
@@ -391,7 +392,7 @@ class Batch:
     def records(self, j):
         job = self.jobs[j]
         a = np.zeros((n_bins(job.get("n_meas", 0), job.get("sweeps_per_bin", 1)),
-                      22 * job.get("n_levels", 0) + 16), dtype=np.int64)  # record_size(n_levels)
+                      self._record_size[job.get("n_levels", 0)]), dtype=np.int64)
         check(_lib.mcrg_batch_get_records(self.handle, j, a.ctypes.data, a.size))
         return a
 
