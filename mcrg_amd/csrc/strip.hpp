@@ -39,7 +39,7 @@ constexpr uint32_t kStripCntWords = 64;    // per-slot operator counts, 4 per le
 // that stand behind the error word: 2 s, or MCRG_STRIP_WAIT_TICKS of the
 // environment, with which tests of the error path make waits give up.
 constexpr uint32_t kStripWaitTicks = 200000000u;
-constexpr uint32_t kStripLimitWord = 1u;  // from the error word on
+constexpr uint32_t kStripLimitWord = 1u;  // from the error word on; both are read as one 64-bit word
 constexpr uint32_t kStripMaxWg = 256;
 // Slots per strip of a sample's first blocked rows with halo rows: they are
 // read a sweep after they are sent, while the sender may already send the

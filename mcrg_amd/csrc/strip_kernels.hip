@@ -54,8 +54,9 @@ __device__ __noinline__ uint64_t ll_wait(const uint64_t *p, uint32_t seq, uint32
         const uint64_t v = ll_peek(p);
         if ((uint32_t)(v >> 32) == seq) return v;
         if ((k & 7u) == 0u) {
-            if (ld_relaxed(err) != 0u) return 0;
-            if ((uint64_t)wall_clock64() - t0 > ld_relaxed(err + kStripLimitWord)) {
+            const uint64_t el = ll_peek(reinterpret_cast<const uint64_t *>(err));  // error, limit
+            if ((uint32_t)el != 0u) return 0;
+            if ((uint64_t)wall_clock64() - t0 > el >> 32) {
                 __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return 0;
             }
@@ -83,9 +84,10 @@ __device__ __noinline__ bool flag_wait(const uint32_t *flag, uint32_t want, uint
 {
     const uint64_t t0 = (uint64_t)wall_clock64();
     while (ld_relaxed(flag) < want) {
-        if (ld_relaxed(err) != 0u) return false;
+        const uint64_t el = ll_peek(reinterpret_cast<const uint64_t *>(err));  // error, limit
+        if ((uint32_t)el != 0u) return false;
         __builtin_amdgcn_s_sleep(1);
-        if ((uint64_t)wall_clock64() - t0 > ld_relaxed(err + kStripLimitWord)) {
+        if ((uint64_t)wall_clock64() - t0 > el >> 32) {
             __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return false;
         }
