@@ -28,12 +28,14 @@ namespace mcrg {
 // are counted all the same: a wave that gives up ends with the step it is in, the
 // others, who wait for its words, do so as well, and the error word says that the
 // state is lost (leaving the step at once took L = 128 6 % more time: its branch
-// stands between the words and their decisions).
+// stands between the words and their decisions).  The count costs a poll 6 % of a
+// half sweep at L = 64; one comparison of everything that is waited for, instead
+// of one a word and their masks joined, gives that back and more.
 //
-// Bound by the latency of a half sweep (L = 64: 740 cycles) and, at L = 128, by
+// Bound by the latency of a half sweep (L = 64: 720 cycles) and, at L = 128, by
 // VALU issue (8 wave-words a sweep on each SIMD).  us a sweep, unmeasured and
-// measured, against strips on many compute units: L = 64 2.41 -> 0.62 and 3.01 ->
-// 0.72; L = 128 2.40 -> 1.05 and 2.64 -> 1.12.  One lattice: two sets take 0.70
+// measured, against strips on many compute units: L = 64 2.41 -> 0.60 and 3.01 ->
+// 0.70; L = 128 2.40 -> 1.04 and 2.64 -> 1.14.  One lattice: two sets take 0.70
 // and 0.78 at L = 64, three sets 1.02 and 1.34 at L = 128 (four measuring waves;
 // two 1.91); with the random numbers drawn when the words are there L = 64 takes
 // 1.09, with one refinement call ahead instead of two 0.85.  Groups of lattices:
@@ -105,16 +107,18 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
             uint64_t own, o, side, nu, nd;
             uint32_t left = spins;
             for (;;) {
+                const uint32_t done = want ? lds_ld(read + (it % M)) : 0u;
                 own = word_ld(mine + word);
                 o = word_ld(oth + word);
                 side = WPR == 1u ? o : word_ld(oth + beside);
                 nu = word_ld(oth + up);
                 nd = word_ld(oth + dn);
-                const uint32_t done = want ? lds_ld(read + (it % M)) : 0u;
-                const uint32_t off = ((uint32_t)(own >> 32) ^ it) | ((uint32_t)(o >> 32) ^ have) |
-                                     ((uint32_t)(side >> 32) ^ have) | ((uint32_t)(nu >> 32) ^ have) |
-                                     ((uint32_t)(nd >> 32) ^ have);
-                if (__ballot(off != 0u || done < want) == 0ull) break;
+                uint32_t off = ((uint32_t)(own >> 32) ^ it) | ((uint32_t)(o >> 32) ^ have) |
+                               ((uint32_t)(side >> 32) ^ have) | ((uint32_t)(nu >> 32) ^ have) |
+                               ((uint32_t)(nd >> 32) ^ have);
+                off |= done < want ? 1u : 0u;
+                asm("" : "+v"(off));  // one comparison, not one a word and their masks joined
+                if (__builtin_amdgcn_ballot_w64(off != 0u) == 0ull) break;
                 if (left-- == 0u) {  // the last step, from whatever is there
                     lds_st(lost, 1u);
                     end = 0u;
@@ -158,7 +162,7 @@ __global__ __launch_bounds__(ColourGeom<L>::threads) void k_colour_chain(const H
                     c1[k] = (uint32_t)b;
                     off |= ((uint32_t)(a >> 32) ^ (it + 1u)) | ((uint32_t)(b >> 32) ^ (it + 1u));
                 }
-                if (__ballot(off != 0u) == 0ull) break;
+                if (__builtin_amdgcn_ballot_w64(off != 0u) == 0ull) break;
                 if (left == 0u) {
                     lds_st(lost, 1u);
                     end = 0u;
