@@ -60,11 +60,11 @@ HBM_PEAK_GBS = 8000.0
 # dispatch, the scale factors read off the same counters on a 1 GiB read + 1 GiB
 # write copy kernel, --copy-calibration).  Configurations without a counter run
 # report null.
-MEASURED_TRAFFIC = {(4096, 100): (4690.4 * 2.0 + 6159.1) * 1024.0}
+MEASURED_TRAFFIC = {(4096, 100): (4735.8 * 2.0 + 6105.3) * 1024.0}
 # The same kernel is bound by VALU issue, not HBM: rocprofv3 --pmc SQ_INSTS_VALU
 # over the same launches gives the wave-level VALU instructions per launch (1024
 # SIMDs that issue one wave64 VALU instruction per 4 cycles).
-MEASURED_VALU = {(4096, 100): {"valu_wave_instr_per_launch": 2.5651e8}}
+MEASURED_VALU = {(4096, 100): {"valu_wave_instr_per_launch": 2.5566e8}}
 
 
 KIND_STRIP = 4  # mcrg_ctx_kernel_time kind of the strip kernel

@@ -247,7 +247,9 @@ mcrg_status mcrg_batch_destroy(mcrg_batch b);
  * job still has to run after them. */
 mcrg_status mcrg_batch_run(mcrg_batch b, int32_t max_sweeps, int32_t *remaining);
 mcrg_status mcrg_batch_sync(mcrg_batch b);
-/* Records of job j: n = ceil(n_meas / sweeps_per_bin) * mcrg_record_size(n_levels). */
+/* Records of job j: n = ceil(n_meas / sweeps_per_bin) * mcrg_record_size(n_levels).
+ * While another thread is in mcrg_batch_run they are those of the launches
+ * enqueued so far. */
 mcrg_status mcrg_batch_get_records(mcrg_batch b, int32_t job, int64_t *host, int64_t n);
 /* Spins of job j as +-1 int8, row-major, n = L*L. */
 mcrg_status mcrg_batch_get_spins(mcrg_batch b, int32_t job, int8_t *host, int64_t n);

@@ -70,7 +70,7 @@ struct StripShape {
     // seq) words) and workgroup n_wg + (k mod split) n_wg + w measures sample k
     // of strip w, so a strip's sweeps no longer wait for its measurements.  A
     // measuring workgroup takes about 13,400 cycles a sample at L = 2048, a
-    // strip 7,800 a sweep: two of them, each on every other sample, keep up.
+    // strip 7,200 a sweep: two of them, each on every other sample, keep up.
     uint32_t split, n_meas, snap_words, first_slots;
     // device workspace, offsets in 32-bit words (even where 64-bit words
     // start), all of it cleared per launch:

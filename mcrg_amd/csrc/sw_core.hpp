@@ -91,9 +91,11 @@ __device__ __forceinline__ uint32_t run_later(uint32_t g, uint32_t r)
 // Joins the trees of a and b, walking up both at once and halving the paths
 // (every second label on the way moves to its parent's parent, so that the
 // chains that simultaneous links leave behind shrink under the walks); of two
-// roots the larger is linked below the smaller.  A label only decreases and
-// always names a site of the same cluster, so a stale read lengthens a path but
-// never leaves the cluster; the atomics decide.
+// roots the larger is linked below the smaller.  A label is smaller than its own
+// id (but a root's) and always names a site of the same cluster, so a stale read
+// lengthens a path but never leaves the cluster.  A halving store that comes late
+// may raise a label that another thread's fetch_min has just lowered; that thread
+// then unites the old label's tree itself, since fetch_min gave it that label.
 __device__ __forceinline__ void lds_unite(uint32_t *lab, uint32_t a, uint32_t b)
 {
     for (;;) {
